@@ -36,9 +36,11 @@
 //                          S0(c+1) = e^{A_L(c)} S0(c) + local(c) gives every chunk's
 //                          start state, the reverse chain dS1 of every chunk and dS0
 //                          of the sequence's start
-//   ssd_bwd_chunk_kernel  (chunk, C group): everything else, for the group's heads
+//   ssd_bwd_group_kernel  (chunk, C group): everything else, for the group's heads
 //                          in turn, the next head's inputs loading into registers
-//                          during the current head's products
+//                          during the current head's products; where B and C are
+//                          grouped alike and there is no z gate
+//   ssd_bwd_chunk_kernel  the same without those two conditions
 // dC (and dB when B's groups are C's) sum over the workgroup's heads in registers;
 // x shared by several heads (HX < H), or B shared wider than a C group, accumulate
 // with fp32 atomics; everything else is stored.
@@ -387,7 +389,552 @@ __global__ __launch_bounds__(256) void ssd_bwd_scan_kernel(Params p, int PN) {
 }
 
 // ---------------------------------------------------------------------------
-// chunk kernel
+// chunk kernel where B and C are grouped alike (G == GC) and there is no z gate:
+// one workgroup of eight waves per (chunk, group), the group's heads in turn.
+//
+// Everything that depends on B and C alone is formed once per workgroup and held in
+// registers: C B^T (its tiles of the wave), B as an MFMA operand, and B and C at the
+// positions of the wave's gradient tiles.  Per head there remain five products,
+//   Q = g x^T, g S0, x dS1, dS1 B^T and g^T (M dt'),
+// where the general kernel below issues nine, because
+//   - sum_h W_h B = (sum_h W_h) B and sum_h W_h^T C = (sum_h W_h)^T C: W is summed over
+//     the heads in fp32 registers and its products are formed once per group;
+//   - g_t . (S0 C_t) = C_t . (S0^T g_t) and x_s . (dS1 B_s) = B_s . (dS1^T x_s): the
+//     decay gradient's state terms are dot products of rows that dC and dB need
+//     anyway, so C S0^T is not formed and no x or g is read back;
+//   - sum_t W_ts (C_t.B_s) = dt'_s sum_t M_ts Q_ts: one column sum serves both.
+// Tiles: wave w holds token block w & 3 and half w >> 2 of the other dimension (key
+// blocks of Q, p blocks of dx, n blocks of dC and dB).  Q and dx are formed transposed,
+// so M goes to LDS and dx to memory as four consecutive elements per lane.
+// LDS rows are 36 or 72 dwords in the interleaved feature order (mfma.hpp): row and
+// transposing fragment reads are conflict-free.  At headdim 64 two sets of a head's
+// tiles alternate: the next head is staged while this head's dx is formed (two
+// barriers per head); at 128 one set fits, and the next head's loads are issued late,
+// after the products whose tiles leave no registers for them.
+// What bounds it: latency at two waves per SIMD, then memory (1.8 GB read and 0.45 GB
+// written at 2 x 16384 tokens, H = 64, P = 64, N = 128, G = 8: 0.44 ms at the rate of a
+// copy; S0 and dS1, 16 KB each per head and chunk, are 1.07 GB of it).  Measured there:
+// 0.76 ms where ssd_bwd_chunk_kernel (four waves per CU, nine products, scalar LDS
+// reads) takes 1.96; forward + backward 3.14 -> 1.95 ms.  At 8 x 4096 tokens, H = 32,
+// P = N = 128 with 1, 4 or 8 heads per group 3.13 -> 2.27, 2.76 -> 2.00, 2.70 -> 1.97 ms;
+// at 2 x 8192, H = 64, P = 64 with one head per group 2.17 -> 1.47 ms.
+// ---------------------------------------------------------------------------
+constexpr int GTHR = 512;
+
+constexpr int row_ld(int w) { return w == 64 ? w + 8 : w + 16; }
+
+template <int P, int N>
+struct GLay {
+  static constexpr int LDP = row_ld(P), LDN = row_ld(N), LDM = row_ld(L);
+  static constexpr int NSET = P == 64 ? 2 : 1;
+  static constexpr int OFF_X = 0;                           // x    [L][LDP]
+  static constexpr int OFF_G = OFF_X + L * LDP * 2;         // g    [L][LDP]
+  static constexpr int OFF_S = OFF_G + L * LDP * 2;         // S0   [P][LDN]
+  static constexpr int OFF_DS = OFF_S + P * LDN * 2;        // dS1  [P][LDN]
+  static constexpr int OFF_SC = OFF_DS + P * LDN * 2;       // scalars of the head
+  // dt', A, e^A, e^{A_L - A}, d dt'/d dt [L] each; D [P]; dD partials [8][P]; <dS1,S0> [8]
+  static constexpr int F_D = 5 * L, F_DD = F_D + P, F_HD = F_DD + 8 * P;
+  static constexpr int SET = OFF_SC + (F_HD + 8) * 4;
+  static constexpr int OFF_M = NSET * SET;                  // M dt' (the heads' W at the end)
+  // sums: rows of dt' M Q [2][L], columns of M Q [4][L], C.(S0 g) [2][L], B.(dS1 x) [2][L]
+  static constexpr int OFF_R = OFF_M + L * LDM * 2;
+  static constexpr int BYTES = OFF_R + 10 * L * 4;
+  static_assert(BYTES <= 160 * 1024 && P >= L, "LDS budget");
+};
+
+template <int CTRL>
+__device__ __forceinline__ float dppf(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                                               0xF, 0xF, false));
+}
+// The sums of x[0..3] over the 16 lanes of a DPP row by a transposing reduction: lane
+// l16 receives the sum of x[l16 & 3].
+__device__ __forceinline__ float row16_sum4(const f32x4& x, int l16) {
+  const bool b = l16 & 1, c = l16 & 2;
+  const float y0 = (b ? x[1] : x[0]) + dppf<0xB1>(b ? x[0] : x[1]);
+  const float y1 = (b ? x[3] : x[2]) + dppf<0xB1>(b ? x[2] : x[3]);
+  float z = (c ? y1 : y0) + dppf<0x4E>(c ? y0 : y1);
+  z += dppf<0x124>(z);
+  z += dppf<0x128>(z);
+  return z;
+}
+// a + b with their halves of 32 lanes exchanged: lanes 0-31 receive a over the lane
+// pairs (l, l + 32), lanes 32-63 b; with b = a the sum over the pair in every lane
+__device__ __forceinline__ float pair_sum32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a),
+                                                  __builtin_bit_cast(unsigned, b), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+// the same over (l, l + 16): even rows of 16 lanes receive a's sums, odd rows b's
+__device__ __forceinline__ float pair_sum16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a),
+                                                  __builtin_bit_cast(unsigned, b), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ __forceinline__ float wave_sum_v(float x) {
+  x = row16_sum(x);
+  x = pair_sum16(x, x);
+  return pair_sum32(x, x);
+}
+
+// row and transposed fragments of interleaved bf16 rows (mfma.hpp)
+__device__ __forceinline__ bf16x8 fr(const bf16* b, int ld, int r0, int k0, int lane) {
+  return __builtin_bit_cast(bf16x8, frag_i(reinterpret_cast<const f16*>(b), ld, r0, k0, lane));
+}
+// position of the 4-feature chunk m of 16-feature block `blk`, icol(16 blk + 4 m): written
+// so that a compile-time block of an even first block stays an immediate offset
+__device__ __forceinline__ int icol4(int blk, int m) { return ((blk >> 1) << 5) + ((blk & 1) << 2) + 8 * m; }
+// transposed fragment (frag_t_i) of rows t0.., 16-column block c0 + c (c0 even)
+__device__ __forceinline__ bf16x8 fr_t(const bf16* b, int ld, int t0, int c0, int c, int lane) {
+  const bf16* a = b + (4 * (lane >> 4) + ((lane & 15) >> 2)) * ld + icol4(c0, lane & 3) +
+                  t0 * ld + icol4(c, 0);
+  typedef __attribute__((address_space(3))) s16x4* lds4;
+  const bf16x4 x = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(a)));
+  const bf16x4 y = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(a + 16 * ld)));
+  return bf16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+}
+__device__ __forceinline__ void st8(bf16* row, int f0, const bf16x8& y) {
+  store8_i(reinterpret_cast<f16*>(row), f0, __builtin_bit_cast(f16x8, y));
+}
+
+// Raw buffer resource over rows 0 .. nrows-1 (w elements of `es` bytes, ts elements
+// apart): rows past the end read zeros and write nothing.  The host keeps 64 rows of
+// any stride inside 32-bit offsets.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, int nrows, int64_t ts,
+                                                           int w, int es) {
+  const uint32_t bytes = nrows > 0 ? (uint32_t)(((int64_t)(nrows - 1) * ts + w) * es) : 0u;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ bf16x8 ld_row(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+
+// One head's inputs for the chunk, in flight while the heads before it are computed.
+template <int P, int N>
+struct GroupIn {
+  static constexpr int VX = L * P / 8 / GTHR, VS = P * N / 8 / GTHR;
+  bf16x8 x[VX], dy[VX], s0[VS], ds[VS];
+  uint32_t dt;   // of token `lane` (wave 0), as stored: converted where it is used
+  float d;       // D of feature tid (tid < P)
+};
+
+template <int P, int N>
+__global__ __launch_bounds__(GTHR, 2) void ssd_bwd_group_kernel(Params p) {
+  using K = GLay<P, N>;
+  using In = GroupIn<P, N>;
+  constexpr int LDP = K::LDP, LDN = K::LDN, LDM = K::LDM;
+  constexpr int VX = In::VX, VS = In::VS, VB = L * N / 8 / GTHR;
+  constexpr int PW = P / 32, NW = N / 32;   // p and n blocks per wave
+  constexpr int RX = GTHR / (P / 8), RS = GTHR / (N / 8);   // rows per staging pass
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q4 = lane >> 4, l16 = lane & 15;
+  const int tb = wave & 3, half = wave >> 2;
+  bf16* sM = reinterpret_cast<bf16*>(smem + K::OFF_M);
+  float* sR = reinterpret_cast<float*>(smem + K::OFF_R);
+  const auto set_bf = [&](int b, int off) { return reinterpret_cast<bf16*>(smem + b * K::SET + off); };
+  const auto set_sc = [&](int b) { return reinterpret_cast<float*>(smem + b * K::SET + K::OFF_SC); };
+  const auto at4 = [&](const float* f, int t) { return *reinterpret_cast<const f32x4*>(f + t); };
+
+  const int H = p.H, GC = p.GC, HC = H / GC, HXS = H / p.HX;
+  const int r = blockIdx.x / GC, gc = blockIdx.x % GC;
+  const Row ro = load_row(p.seg, r);
+  const int tok0 = ro.bos, nval = ro.eos - ro.bos;
+  const int h_first = gc * HC;
+
+  // B and C rows of the chunk into two sets of registers
+  const auto fetch_bc = [&](int tid, bf16x8* bv, bf16x8* cv) {
+    const auto rb = rows_rsrc(p.B + (int64_t)tok0 * p.b_ts + (int64_t)gc * p.b_gs, nval, p.b_ts, N, 2);
+    const auto rc = rows_rsrc(p.C + (int64_t)tok0 * p.c_ts + (int64_t)gc * p.c_gs, nval, p.c_ts, N, 2);
+#pragma unroll
+    for (int i = 0; i < VB; ++i) {
+      const int t = i * RS + tid / (N / 8), c = (tid % (N / 8)) * 8;
+      bv[i] = ld_row(rb, (uint32_t)(((int64_t)t * p.b_ts + c) * 2));
+      cv[i] = ld_row(rc, (uint32_t)(((int64_t)t * p.c_ts + c) * 2));
+    }
+  };
+  const auto fetch = [&](int tid, int h, In& q) {
+    const int lane = tid & 63;
+    const auto rx = rows_rsrc(p.x + (int64_t)tok0 * p.x_ts + (int64_t)(h / HXS) * p.x_hs, nval, p.x_ts, P, 2);
+    const auto ry = rows_rsrc(p.dy + (int64_t)tok0 * p.dy_ts + (int64_t)h * p.dy_hs, nval, p.dy_ts, P, 2);
+#pragma unroll
+    for (int i = 0; i < VX; ++i) {
+      const int t = i * RX + tid / (P / 8), c = (tid % (P / 8)) * 8;
+      q.x[i] = ld_row(rx, (uint32_t)(((int64_t)t * p.x_ts + c) * 2));
+      q.dy[i] = ld_row(ry, (uint32_t)(((int64_t)t * p.dy_ts + c) * 2));
+    }
+    const bf16* s0 = p.S0 + ((int64_t)r * H + h) * P * N;
+    const bf16* ds = p.dS1 + ((int64_t)r * H + h) * P * N;
+#pragma unroll
+    for (int i = 0; i < VS; ++i) {
+      q.s0[i] = *reinterpret_cast<const bf16x8*>(s0 + (i * GTHR + tid) * 8);
+      q.ds[i] = *reinterpret_cast<const bf16x8*>(ds + (i * GTHR + tid) * 8);
+    }
+    q.dt = (wave == 0 && lane < nval)
+               ? ld_bits(p.dt, (int64_t)(tok0 + lane) * p.dt_ts + (int64_t)h * p.dt_hs, p.dt_dt) : 0u;
+    q.d = (p.D && tid < P) ? p.D[(int64_t)h * P + tid] : 0.f;
+  };
+  In in;
+  // in flight after head h's inputs: the next head, or after the last one B and C again
+  // (in the registers of S0 and dS1) for the products at the end
+  const auto fetch_next = [&](int tid, int h) {
+    if (h < h_first + HC) fetch(tid, h, in);
+    else fetch_bc(tid, in.s0, in.ds);
+  };
+
+  // ---- B and C through the S0 / dS1 tiles of set 0 into registers ------------------
+  const auto stage_bc = [&](const bf16x8* bv, const bf16x8* cv, bf16* sb, bf16* sc) {
+#pragma unroll
+    for (int i = 0; i < VB; ++i) {
+      const int t = i * RS + tid / (N / 8), c = (tid % (N / 8)) * 8;
+      st8(sb + t * LDN, c, bv[i]);
+      st8(sc + t * LDN, c, cv[i]);
+    }
+  };
+  bf16x8 bfr[N / 32];        // B rows of token block tb (an operand of dS1 B^T)
+  f32x4 cbt[2], wsum[2];     // (C B^T)^T and sum_h W_h^T, key block 2 half + j, query block tb
+  bf16x4 creg[NW], breg[NW];  // C and B at rows 16 tb + 4 q4 + v, columns 16 (half NW + j) + l16
+  f32x4 dC[NW], dB[NW];
+  {
+    bf16* sb = set_bf(0, K::OFF_S);
+    bf16* sc = set_bf(0, K::OFF_DS);
+    bf16x8 bv[VB], cv[VB];
+    fetch_bc(tid, bv, cv);
+    fetch(tid, h_first, in);
+    stage_bc(bv, cv, sb, sc);
+    // the tiles above the diagonal that M's products read (key block 1 of query block
+    // 0, 3 of 2) stay zero
+    if ((wave == 0 || wave == 2) && lane < 32) {
+      const int t = 16 * wave + (lane >> 1), c = 16 * wave + 16 + 8 * (lane & 1);
+      st8(sM + t * LDM, c, bf16x8{});
+    }
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < N / 32; ++k) bfr[k] = fr(sb, LDN, 16 * tb, 32 * k, lane);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      cbt[j] = wsum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < N / 32; ++k)
+        cbt[j] = mfma16(fr(sb, LDN, 16 * (2 * half + j), 32 * k, lane), fr(sc, LDN, 16 * tb, 32 * k, lane), cbt[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      dC[j] = dB[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int e = (16 * tb + 4 * q4 + v) * LDN + icol(16 * (half * NW + j) + l16);
+        creg[j][v] = sc[e];
+        breg[j][v] = sb[e];
+      }
+    }
+    lds_barrier();   // set 0 is free again
+  }
+
+  // ---- one head's registers into set b: tiles, token scalars, D, the partial sums of
+  // dD = sum_t g_t x_t and <dS1, S0> of each wave --------------------------------------
+  const auto stage = [&](int tid, int b, int h) {
+    const int lane = tid & 63, l16 = lane & 15;
+    bf16 *sX = set_bf(b, K::OFF_X), *sG = set_bf(b, K::OFF_G);
+    bf16 *sS = set_bf(b, K::OFF_S), *sDS = set_bf(b, K::OFF_DS);
+    float* sf = set_sc(b);
+    float dd[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < VX; ++i) {
+      const int t = i * RX + tid / (P / 8), c = (tid % (P / 8)) * 8;
+      st8(sX + t * LDP, c, in.x[i]);
+      st8(sG + t * LDP, c, in.dy[i]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) dd[j] += (float)in.dy[i][j] * (float)in.x[i][j];
+    }
+    float hd = 0.f;
+#pragma unroll
+    for (int i = 0; i < VS; ++i) {
+      const int e = (i * GTHR + tid) * 8;
+      st8(sS + (e / N) * LDN, e % N, in.s0[i]);
+      st8(sDS + (e / N) * LDN, e % N, in.ds[i]);
+#pragma unroll
+      for (int j = 0; j < 8; j += 2)
+        hd = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{in.s0[i][j], in.s0[i][j + 1]},
+                                             bf16x2{in.ds[i][j], in.ds[i][j + 1]}, hd, false);
+    }
+    if (p.dD) {
+      // over the wave's lanes of the same eight features: halving the values at each
+      // exchange; lane l ends with feature 4 (l >> 5) + 2 (l >> 4 & 1) (+ (l >> 3 & 1))
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dd[j] = pair_sum32(dd[j], dd[j + 4]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) dd[j] = pair_sum16(dd[j], dd[j + 2]);
+      float* o = sf + K::F_DD + wave * P + 4 * (lane >> 5) + 2 * ((lane >> 4) & 1);
+      if constexpr (P == 64) {
+        const bool up = lane & 8;
+        o[(lane & 7) * 8 + ((lane >> 3) & 1)] = (up ? dd[1] : dd[0]) + dppf<0x128>(up ? dd[0] : dd[1]);
+      } else {
+        o[l16 * 8] = dd[0];
+        o[l16 * 8 + 1] = dd[1];
+      }
+    }
+    hd = wave_sum_v(hd);
+    if (lane == 0) sf[K::F_HD + wave] = hd;
+    if (tid < P) sf[K::F_D + tid] = in.d;
+    if (wave == 0) {
+      const Tok tk = token_scalars_raw(p, h, bits_f32(in.dt, p.dt_dt), nval, lane);
+      const float aend = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tk.acs), 63));
+      sf[lane] = tk.dtv;
+      sf[L + lane] = tk.acs;
+      sf[2 * L + lane] = fast_exp(tk.acs);
+      sf[3 * L + lane] = fast_exp(aend - tk.acs);
+      sf[4 * L + lane] = tk.fac;
+    }
+  };
+
+  stage(tid, 0, h_first);
+  if constexpr (K::NSET == 2) fetch_next(tid, h_first + 1);
+  lds_barrier();
+
+#pragma unroll 1
+  for (int ih = 0; ih < HC; ++ih) {
+    // opaque per head: the lane's LDS offsets are formed again instead of being hoisted
+    // out of the loop into registers that the tiles need
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, q4 = lane >> 4, l16 = lane & 15;
+    const int h = h_first + ih, b = K::NSET == 2 ? (ih & 1) : 0;
+    const bf16 *sX = set_bf(b, K::OFF_X), *sG = set_bf(b, K::OFF_G);
+    const bf16 *sS = set_bf(b, K::OFF_S), *sDS = set_bf(b, K::OFF_DS);
+    const float* sf = set_sc(b);
+    if (p.dD && tid < P) {
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) s += sf[K::F_DD + w * P + tid];
+      unsafeAtomicAdd(p.dD + (int64_t)h * P + tid, s);
+    }
+    // ---- Q^T (key rows, query columns), M dt' to LDS, W summed over the heads --------
+    {
+      float rowr = 0.f;   // sum over the wave's keys of dt'_s M_ts Q_ts, t = 16 tb + l16
+      const float acs_t = sf[L + 16 * tb + l16];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int sb = 2 * half + j;
+        if (sb > tb) continue;
+        f32x4 qq = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < P / 32; ++k)
+          qq = mfma16(fr(sX, LDP, 16 * sb, 32 * k, lane), fr(sG, LDP, 16 * tb, 32 * k, lane), qq);
+        const f32x4 acs_s = at4(sf + L, 16 * sb + 4 * q4), dt_s = at4(sf, 16 * sb + 4 * q4);
+        f32x4 u;
+        bf16x4 md;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          float dec = fast_exp(acs_t - acs_s[v]);
+          if (sb == tb && 4 * q4 + v > l16) dec = 0.f;
+          const float e = dec * dt_s[v];
+          u[v] = cbt[j][v] * qq[v] * dec;
+          rowr += u[v] * dt_s[v];
+          wsum[j][v] += qq[v] * e;
+          md[v] = (bf16)(cbt[j][v] * e);
+        }
+        *reinterpret_cast<bf16x4*>(sM + (16 * tb + l16) * LDM + icol4(sb, q4)) = md;
+        const float cs = row16_sum4(u, l16);
+        if (l16 < 4) sR[(2 + tb) * L + 16 * sb + 4 * q4 + l16] = cs;
+      }
+      rowr = pair_sum16(rowr, rowr);
+      rowr = pair_sum32(rowr, rowr);
+      if (lane < 16) sR[half * L + 16 * tb + lane] = rowr;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- dC += e^{A_t} g S0 and C_t . (S0^T g_t) ---------------------------------------
+    {
+      f32x4 acc[NW];
+#pragma unroll
+      for (int j = 0; j < NW; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < P / 32; ++k) {
+        const bf16x8 a = fr(sG, LDP, 16 * tb, 32 * k, lane);
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+          acc[j] = mfma16(a, fr_t(sS, LDN, 32 * k, half * NW, j, lane), acc[j]);
+      }
+      const f32x4 ea = at4(sf + 2 * L, 16 * tb + 4 * q4);
+      f32x4 ds = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NW; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          ds[v] += (float)creg[j][v] * acc[j][v];
+          dC[j][v] += ea[v] * acc[j][v];
+        }
+      const float s = row16_sum4(ds, l16);
+      if (l16 < 4) sR[(6 + half) * L + 16 * tb + 4 * q4 + l16] = s;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- dB += e dt' x dS1 and B_s . (dS1^T x_s) ---------------------------------------
+    {
+      f32x4 acc[NW];
+#pragma unroll
+      for (int j = 0; j < NW; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < P / 32; ++k) {
+        const bf16x8 a = fr(sX, LDP, 16 * tb, 32 * k, lane);
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+          acc[j] = mfma16(a, fr_t(sDS, LDN, 32 * k, half * NW, j, lane), acc[j]);
+      }
+      const f32x4 e = at4(sf + 3 * L, 16 * tb + 4 * q4), dt = at4(sf, 16 * tb + 4 * q4);
+      f32x4 ds = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NW; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          ds[v] += (float)breg[j][v] * acc[j][v];
+          dB[j][v] += e[v] * dt[v] * acc[j][v];
+        }
+      const float s = row16_sum4(ds, l16);
+      if (l16 < 4) sR[(8 + half) * L + 16 * tb + 4 * q4 + l16] = s;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- (dS1 B^T): p rows, key columns --------------------------------------------------
+    f32x4 dh[PW];
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      dh[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < N / 32; ++k)
+        dh[i] = mfma16(fr(sDS, LDN, 16 * (half * PW + i), 32 * k, lane), bfr[k], dh[i]);
+    }
+    lds_barrier();   // M and the sums are whole
+
+    if constexpr (K::NSET == 2) {
+      if (ih + 1 < HC) {
+        stage(tid, b ^ 1, h + 1);
+        fetch_next(tid, h + 2);
+      }
+    } else {
+      fetch_next(tid, h + 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- dx^T = g^T (M dt') + e dt' (dS1 B^T) + D g ---------------------------------------
+    {
+      f32x4 acc[PW];
+#pragma unroll
+      for (int i = 0; i < PW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        if (k == 0 && tb >= 2) continue;   // M's tiles above the diagonal
+        const bf16x8 m = fr_t(sM, LDM, 32 * k, tb, 0, lane);
+#pragma unroll
+        for (int i = 0; i < PW; ++i)
+          acc[i] = mfma16(fr_t(sG, LDP, 32 * k, half * PW, i, lane), m, acc[i]);
+      }
+      const int s = 16 * tb + l16, hx = h / HXS;
+      const float f = sf[3 * L + s] * sf[s];
+      const int es = p.gbf16 ? 2 : 4;
+      const auto rx = rows_rsrc(static_cast<char*>(p.dx) + ((int64_t)tok0 * p.HX + hx) * P * es, nval,
+                                (int64_t)p.HX * P, P, es);
+#pragma unroll
+      for (int i = 0; i < PW; ++i) {
+        const int c = 16 * (half * PW + i) + 4 * q4;
+        const bf16x4 g = *reinterpret_cast<const bf16x4*>(sG + s * LDP + icol4(half * PW, q4) + icol4(i, 0));
+        const f32x4 dv = at4(sf + K::F_D, c);
+        f32x4 d;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) d[v] = acc[i][v] + f * dh[i][v] + dv[v] * (float)g[v];
+        const uint32_t off = (uint32_t)((s * p.HX * P + c) * es);
+        if (p.gbf16) {
+          const bf16x4 o = {(bf16)d[0], (bf16)d[1], (bf16)d[2], (bf16)d[3]};
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, o), rx, off, 0, 0);
+        } else if (!p.x_shared) {
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, d), rx, off, 0, 0);
+        } else if (s < nval) {
+          float* o = static_cast<float*>(p.dx) + ((int64_t)(tok0 + s) * p.HX + hx) * P + c;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) unsafeAtomicAdd(o + v, d[v]);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- scalar chain on one wave: dA_t, da (reverse cumsum), d dt, dA_h, d dt_bias -------
+    if (wave == (ih & 7)) {
+      const int t = lane, tt = t >> 4;
+      float cmq = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        if (w >= tt) cmq += sR[(2 + w) * L + t];   // query blocks before the key's hold nothing
+      const float dt_t = sf[t];
+      const float dds = sf[3 * L + t] * (sR[8 * L + t] + sR[9 * L + t]);
+      const float das = sf[2 * L + t] * (sR[6 * L + t] + sR[7 * L + t]);
+      float dacs = sR[t] + sR[L + t] - dt_t * cmq + das - dt_t * dds;
+      // <dS1, S1> = e^{A_L} <dS1, S0> + sum_s dt'_s e_s x_s . (dS1 B_s), on the last token
+      const float tail = wave_sum_v(dt_t * dds);
+      float hd = 0.f;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) hd += sf[K::F_HD + w];
+      if (t == L - 1) dacs += sf[2 * L + L - 1] * hd + tail;
+      const float incl = scan64(dacs, lane);
+      const float total = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, incl), 63));
+      const float da = total - incl + dacs;   // sum_{u >= t} dA_u
+      const float ddt = (cmq + dds + p.A[h] * da) * sf[4 * L + t];
+      if (t < nval) p.ddt[(int64_t)(tok0 + t) * H + h] = ddt;
+      const float sa = wave_sum_v(dt_t * da), sbias = wave_sum_v(ddt);
+      if (lane == 0) {
+        unsafeAtomicAdd(p.dA + h, sa);
+        if (p.dbias) unsafeAtomicAdd(p.dbias + h, sbias);
+      }
+    }
+    lds_barrier();   // this head's tiles, M and sums are free; the next head is staged
+    if (K::NSET == 1 && ih + 1 < HC) {
+      stage(tid, 0, h + 1);
+      lds_barrier();
+    }
+  }
+
+  // ---- dC += (sum_h W) B, dB += (sum_h W)^T C --------------------------------------------
+  {
+    bf16* sb = set_bf(0, K::OFF_S);
+    bf16* sc = set_bf(0, K::OFF_DS);
+    stage_bc(in.s0, in.ds, sb, sc);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int kb = 2 * half + j;
+      if (kb > tb) continue;
+      *reinterpret_cast<bf16x4*>(sM + (16 * tb + l16) * LDM + icol4(kb, q4)) =
+          bf16x4{(bf16)wsum[j][0], (bf16)wsum[j][1], (bf16)wsum[j][2], (bf16)wsum[j][3]};
+    }
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (k == 0 || tb >= 2) {
+        const bf16x8 w = fr(sM, LDM, 16 * tb, 32 * k, lane);
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+          dC[j] = mfma16(w, fr_t(sb, LDN, 32 * k, half * NW, j, lane), dC[j]);
+      }
+      if (k == 1 || tb < 2) {
+        const bf16x8 w = fr_t(sM, LDM, 32 * k, tb, 0, lane);
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+          dB[j] = mfma16(w, fr_t(sc, LDN, 32 * k, half * NW, j, lane), dB[j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int t = 16 * tb + 4 * q4 + v;
+    if (t >= nval) continue;
+    const int64_t row = ((int64_t)(tok0 + t) * GC + gc) * N + 16 * half * NW + l16;
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      st_grad(p.dC, row + 16 * j, dC[j][v], p.gbf16);
+      st_grad(p.dB, row + 16 * j, dB[j][v], p.gbf16);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// chunk kernel for a z gate, or B and C grouped differently
 // ---------------------------------------------------------------------------
 template <int P, int N>
 struct Lay {
@@ -862,7 +1409,17 @@ void launch(const Params& p, hipStream_t s) {
                      dim3(NTHR), lsm, s, p);
   hipLaunchKernelGGL(ssd_bwd_scan_kernel, dim3(p.nseq * p.H, (P * N + 1023) / 1024), dim3(256), 0,
                      s, p, P * N);
-  hipLaunchKernelGGL((ssd_bwd_chunk_kernel<P, N>), dim3(p.nrows * p.GC), dim3(NTHR), smem, s, p);
+  // the group kernel shares C B^T and W's products over the heads (B and C grouped
+  // alike) and forms no y' (which only z needs); it is the faster one at every size
+  // measured (its comment), from one head per group on
+  if (p.G == p.GC && !p.z) {
+    constexpr int gsm = GLay<P, N>::BYTES;
+    (void)hipFuncSetAttribute((const void*)ssd_bwd_group_kernel<P, N>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, gsm);
+    hipLaunchKernelGGL((ssd_bwd_group_kernel<P, N>), dim3(p.nrows * p.GC), dim3(GTHR), gsm, s, p);
+  } else {
+    hipLaunchKernelGGL((ssd_bwd_chunk_kernel<P, N>), dim3(p.nrows * p.GC), dim3(NTHR), smem, s, p);
+  }
 }
 
 }  // namespace ssdb

@@ -157,6 +157,26 @@ def test_backward_headdim_128(dev, N):
         _check(g[k], g_ref[k], f"hdim128 N={N} d{k}", scale=sA if k == "A" else None)
 
 
+@pytest.mark.parametrize("P,N,H,G,l", [(64, 128, 5, 1, 130), (64, 64, 6, 2, 65), (64, 128, 3, 3, 64),
+                                       (128, 128, 3, 1, 200), (128, 64, 4, 4, 1)])
+def test_backward_groups_without_z(dev, P, N, H, G, l):
+    """B and C grouped alike, no z (the kernel that shares C B^T and W's products over a
+    group's heads): one, odd and even heads per group, whole, ragged and one-token
+    chunks, restarts, D per (head, headdim) and initial and final states."""
+    inp, wy, wf = _inputs(1, l, H, G, P, N, 970 + l, False, True)
+    kw = dict(dt_softplus=True, return_final_states=True)
+    kw_dev = dict(kw)
+    if l > 100:
+        kw["seq_idx"] = (torch.arange(l) >= 70).to(torch.int32)[None]
+        kw_dev["seq_idx"] = kw["seq_idx"].to(dev)
+    g = _grads(inp, wy, wf, kw_dev, dev, None)
+    torch.cuda.synchronize()
+    g_ref = _grads(inp, wy, wf, kw, None, torch.float64)
+    sA = _dA_scale(inp, wy, wf, kw)
+    for k in g_ref:
+        _check(g[k], g_ref[k], f"groups P={P} N={N} d{k}", scale=sA if k == "A" else None)
+
+
 def test_backward_headdim_128_with_z_raises(dev):
     inp, _, _ = _inputs(1, 64, 2, 1, 128, 64, 1, True, False)
     x = inp["x"].to(dev).requires_grad_(True)
