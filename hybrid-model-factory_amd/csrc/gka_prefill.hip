@@ -925,22 +925,30 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
       f16x8 dh[4], dl[4];
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) h8_hilo(Dd[2 * ks], Dd[2 * ks + 1], dh[ks], dl[ks], one);
-      // -Z~^T[j][t] = -m_tj (k~_j . d_t), hi/lo B operands over all four key tiles (the
-      // keys past this wave's tokens get m = 0; one uniform instruction stream)
+      // -Z~^T[j][t] = -m_tj (k~_j . d_t), hi/lo B operands, in pairs of key tiles: the
+      // second pair is past every token of waves 0 and 1, which skip it here and in
+      // K~^T below (a uniform branch; 64 of 96 products and 40 of 64 KB of LDS reads per
+      // step for those waves).  32768 tokens, H = 32, 30 iterations: 3.30 -> 3.12 ms.
+      // Skipping single tiles, or exchanging the waves' tokens in every second
+      // workgroup to even out the SIMDs, measured no better.
       f16x8 zh[2], zl[2];
       {
         f32x4 Z[4];
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) Z[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          f16x8 a[4];
+        for (int j2 = 0; j2 < 4; j2 += 2) {
+          if (j2 > wave) break;
 #pragma unroll
-          for (int jt = 0; jt < 4; ++jt) a[jt] = frag_i(sK, LDP, 16 * jt, 32 * ks, lane);
+          for (int ks = 0; ks < 4; ++ks) {
+            f16x8 a[2];
 #pragma unroll
-          for (int jt = 0; jt < 4; ++jt) Z[jt] = mfma16h(a[jt], dh[ks], Z[jt]);
+            for (int jt = 0; jt < 2; ++jt) a[jt] = frag_i(sK, LDP, 16 * (j2 + jt), 32 * ks, lane);
 #pragma unroll
-          for (int jt = 0; jt < 4; ++jt) Z[jt] = mfma16h(a[jt], dl[ks], Z[jt]);
+            for (int jt = 0; jt < 2; ++jt) Z[j2 + jt] = mfma16h(a[jt], dh[ks], Z[j2 + jt]);
+#pragma unroll
+            for (int jt = 0; jt < 2; ++jt) Z[j2 + jt] = mfma16h(a[jt], dl[ks], Z[j2 + jt]);
+          }
         }
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt)
@@ -969,6 +977,7 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
             hx[u][v] = R[g4 + u][v] - lam * Dd[g4 + u][v] - egk * hx[u][v];
 #pragma unroll
         for (int jk = 0; jk < 2; ++jk) {
+          if (2 * jk > wave) break;
           f16x8 a[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) a[u] = frag_t_i(sK, LDP, 32 * jk, 16 * (g4 + u), lane);
