@@ -1478,23 +1478,6 @@ __device__ __forceinline__ void block_scalars(const Sc& s, float gv, float bv, i
   }
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dppf(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
-                                                               0xF, 0xF, false));
-}
-// The sums of x[0..3] over the 16 lanes of a DPP row, by a transposing reduction
-// (five DPP additions instead of sixteen): lane l16 receives the sum of x[l16 & 3].
-__device__ __forceinline__ float row16_sum4(const f32x4& x, int l16) {
-  const bool b = l16 & 1, c = l16 & 2;
-  const float y0 = (b ? x[1] : x[0]) + dppf<0xB1>(b ? x[0] : x[1]);   // x[b], lanes l, l ^ 1
-  const float y1 = (b ? x[3] : x[2]) + dppf<0xB1>(b ? x[2] : x[3]);   // x[b + 2]
-  float z = (c ? y1 : y0) + dppf<0x4E>(c ? y0 : y1);                   // x[l & 3], l ^ 2 too
-  z += dppf<0x124>(z);                                                  // row_ror:4
-  z += dppf<0x128>(z);                                                  // row_ror:8
-  return z;
-}
-
 // rows 16 mt + 4 q4 .. +3 of a per-token LDS array (one 16-byte read)
 __device__ __forceinline__ f32x4 row4(const float* a, int mt, int q4) {
   return *reinterpret_cast<const f32x4*>(a + 16 * mt + 4 * q4);

@@ -138,6 +138,20 @@ __device__ __forceinline__ SegInfo load_seg(const int* seg, int s) {
   return SegInfo{r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7]};
 }
 
+// The segment of block gb: the last s with segblk[s] <= gb (segblk is non-decreasing),
+// counted 64 segments at a time across the wave's lanes -- one round trip to memory
+// where a binary search takes one per halving.
+__device__ __forceinline__ int segment_of(const Params& p, int gb, int lane) {
+  int n = 0;
+  for (int s0 = 0; s0 < p.nseg_total; s0 += 64) {
+    const int s = s0 + lane;
+    const int c = __builtin_popcountll(__ballot(s < p.nseg_total && p.segblk[min(s, p.nseg_total - 1)] <= gb));
+    n += c;
+    if (c < 64) break;
+  }
+  return __builtin_amdgcn_readfirstlane(n - 1);
+}
+
 // Sum of squares of an 8-feature slice over the 16 lanes of its DPP row.
 __device__ __forceinline__ float row_sumsq(const bf16x8& x) {
   float s = 0.f;
@@ -694,12 +708,7 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
   const int64_t DD = (int64_t)D * D;
 
   // ---- which segment / block -------------------------------------------------
-  int lo = 0, hi = p.nseg_total;        // last s with segblk[s] <= gb
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (p.segblk[mid] <= gb) lo = mid; else hi = mid;
-  }
-  const int s_id = lo;
+  const int s_id = segment_of(p, gb, lane);
   const SegInfo si = load_seg(p.seg, s_id);
   const int lb = gb - p.segblk[s_id];                 // block index within the segment
   const int tok0 = si.bos + (si.c_start + lb) * CB;
@@ -749,7 +758,7 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
   }
   float* red = sc + SC_HN * CB;           // 4 partial sums
   if constexpr (SOLVE) {
-    const float ss = wave_sum(state_store<true>(sH, hst, fast_exp(off_gk), tid));
+    const float ss = wave_sum_v(state_store<true>(sH, hst, fast_exp(off_gk), tid));
     if (lane == 0) red[wave] = ss;
   }
   // this lane's token t (16 per wave) and its q^ slice: Q[nt][v] = q^[t][16 nt + 4 q4 + v]
@@ -774,8 +783,7 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) ss += Q[nt][v] * Q[nt][v];
     }
-    ss += __shfl_xor(ss, 16, 64);
-    ss += __shfl_xor(ss, 32, 64);
+    ss = q4_sum(ss);
     rq = (!tok_ok) ? 0.f : (p.l2norm ? 1.0f / sqrtf(ss) : 1.f);
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt)
@@ -809,8 +817,7 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) d += Pd[nt][v] * (float)kk[v];
       }
-      d += __shfl_xor(d, 16, 64);
-      d += __shfl_xor(d, 32, 64);
+      d = q4_sum(d);
       if (q4 == 0) SC(SC_D, tb) = d;
     }
     // Gram part of |H_t|^2: g2_t = sum_{i,j<=t} a_ti a_tj (k~_i.k~_j)^2, a_tj = e^{Gk_t-Gk_j},
@@ -870,9 +877,15 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
         f = tok_ok ? p.fro[(int64_t)(tok0 + tb) * H + h] : 0.f;
       } else {
         float cross = 0.f;
-        for (int j = q4; j <= tb; j += 4) cross += fast_exp(GkT - SC(SC_GK, j)) * SC(SC_D, j);
-        cross += __shfl_xor(cross, 16, 64);
-        cross += __shfl_xor(cross, 32, 64);
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) {
+          const f32x4 gkj = *reinterpret_cast<const f32x4*>(&SC(SC_GK, 16 * jt + 4 * q4));
+          const f32x4 dj = *reinterpret_cast<const f32x4*>(&SC(SC_D, 16 * jt + 4 * q4));
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            cross += (16 * jt + 4 * q4 + v <= tb) ? fast_exp(GkT - gkj[v]) * dj[v] : 0.f;
+        }
+        cross = q4_sum(cross);
         const float e = fast_exp(GkT);
         f = sqrtf(fmaxf(e * e * hn + 2.f * e * cross + SC(SC_G2, tb), 0.f));
         if ((MODE == SM_X || MODE == SM_GLA_SAVE) && tok_ok && q4 == 0)
@@ -1127,8 +1140,7 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
           O[nt][v] = y;
           ss += y * y;
         }
-      ss += __shfl_xor(ss, 16, 64);
-      ss += __shfl_xor(ss, 32, 64);
+      ss = q4_sum(ss);
       rstd = 1.0f / sqrtf(ss * (1.0f / D) + p.on_eps);
     }
     const bf16* zr = (NORM && p.zg) ? p.zg + (int64_t)(tok0 + tb) * p.zg_ts + (int64_t)h * p.zg_hs + 4 * q4
@@ -1339,16 +1351,12 @@ struct Bwd {
 };
 
 struct Blk { int s_id, lb, tok0, nval; };
-__device__ __forceinline__ Blk block_of(const Params& p, int gb) {
-  int lo = 0, hi = p.nseg_total;         // last s with segblk[s] <= gb
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (p.segblk[mid] <= gb) lo = mid; else hi = mid;
-  }
-  const SegInfo si = load_seg(p.seg, lo);
-  const int lb = gb - p.segblk[lo];
+__device__ __forceinline__ Blk block_of(const Params& p, int gb, int lane) {
+  const int s_id = segment_of(p, gb, lane);
+  const SegInfo si = load_seg(p.seg, s_id);
+  const int lb = gb - p.segblk[s_id];
   const int tok0 = si.bos + (si.c_start + lb) * CB;
-  return Blk{lo, lb, tok0, min(CB, si.eos - tok0)};
+  return Blk{s_id, lb, tok0, min(CB, si.eos - tok0)};
 }
 
 // h_c of block gb into sH (fp16, interleaved rows, both triangles), as the solve
@@ -1398,9 +1406,59 @@ __device__ __forceinline__ float pow2_scale(float m) {
   return e > 8 ? ldexpf(1.f, 8 - e) : 1.f;
 }
 __device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x = fmaxf(x, __shfl_xor(x, m, 64));
-  return x;
+  x = fmaxf(x, dppf<0xB1>(x));
+  x = fmaxf(x, dppf<0x4E>(x));
+  x = fmaxf(x, dppf<0x141>(x));
+  x = fmaxf(x, dppf<0x140>(x));
+  const unsigned u = __builtin_bit_cast(unsigned, x);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  x = fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+  const unsigned w = __builtin_bit_cast(unsigned, x);
+  const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)q[0]), __builtin_bit_cast(float, (unsigned)q[1]));
+}
+// Suffix sums over the 64 lanes of a wave (lane l: lanes l..63), within each row of 16
+// by lane shifts, then the later rows' totals.
+template <int N>
+__device__ __forceinline__ float shl_row(float v) {   // lane l of a row receives lane l + N (0 past it)
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + N,
+                                                               0xF, 0xF, true));
+}
+__device__ __forceinline__ float lane_val(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+__device__ __forceinline__ float suffix_sum64(float x, int lane) {
+  x += shl_row<1>(x);
+  x += shl_row<2>(x);
+  x += shl_row<4>(x);
+  x += shl_row<8>(x);
+  const float r3 = lane_val(x, 48), r2 = lane_val(x, 32) + r3, r1 = lane_val(x, 16) + r2;
+  return x + (lane < 16 ? r1 : lane < 32 ? r2 : lane < 48 ? r3 : 0.f);
+}
+// rho_t = sum_{t' >= t} a_t' e^{2 (g_t' - g_t)} over the 64 lanes t (a_t, g_t in lane t):
+// rho over 2n lanes = rho over n + e^{2 (g_{t+n} - g_t)} (rho over n of lane t + n).
+// One wave forms it while the workgroup waits: as a loop over the later tokens (an LDS
+// read and an exponential each, up to 64) it cost, together with the loops of the gates' suffix sums, the binary
+// search for the block's segment and the lane sums through the LDS, 0.67 of training's
+// 7.25 ms at 8 x 4096 tokens, H = 32 (cheb_e_kernel 0.98 -> 0.77, cheb_dk_kernel 1.69 -> 1.45, gla_bwd_kernel
+// 1.58 -> 1.45 ms).
+__device__ __forceinline__ float decayed_suffix(float a, float g, int lane) {
+  const int l16 = lane & 15;
+  float r = a;
+  auto step = [&](float r_n, float g_n, int n) {
+    if (l16 + n < 16) r += fast_exp(2.f * (g_n - g)) * r_n;
+  };
+  step(shl_row<1>(r), shl_row<1>(g), 1);
+  step(shl_row<2>(r), shl_row<2>(g), 2);
+  step(shl_row<4>(r), shl_row<4>(g), 4);
+  step(shl_row<8>(r), shl_row<8>(g), 8);
+  // the later rows: their sums from lanes 16, 32 and 48, the last first
+  const float g1 = lane_val(g, 16), g2 = lane_val(g, 32), g3 = lane_val(g, 48);
+  const float r3 = lane_val(r, 48);
+  const float r2 = lane_val(r, 32) + fast_exp(2.f * (g3 - g2)) * r3;
+  const float r1 = lane_val(r, 16) + fast_exp(2.f * (g2 - g1)) * r2;
+  const float rn = lane < 16 ? r1 : lane < 32 ? r2 : r3, gn = lane < 16 ? g1 : lane < 32 ? g2 : g3;
+  return lane < 48 ? r + fast_exp(2.f * (gn - g)) * rn : r;
 }
 __device__ __forceinline__ float absmax8(const bf16x8& x) {
   float m = 0.f;
@@ -1461,7 +1519,7 @@ __global__ __launch_bounds__(E_NTHR, 1) void cheb_e_kernel(Params p, Bwd w) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q4 = lane >> 4, l16 = lane & 15;
   const int gb = blockIdx.x, h = blockIdx.y, H = p.H;
-  const Blk b = block_of(p, gb);
+  const Blk b = block_of(p, gb, lane);
   if (b.nval <= 0) return;
   constexpr int NP = CB * 16 / E_NTHR;     // staging passes of 32 rows
 
@@ -1490,9 +1548,8 @@ __global__ __launch_bounds__(E_NTHR, 1) void cheb_e_kernel(Params p, Bwd w) {
   // rho_t = sum_{t'>=t} a_t' e^{2(g_t'-g_t)} (lane t of wave 0), beta_t = e^{g_t} rho_t
   float alpha = 0.f;
   if (wave == 0) {
-    float rho = 0.f;
     const float gt = sG[lane];
-    for (int t2 = lane; t2 < b.nval; ++t2) rho += sA[t2] * fast_exp(2.f * (sG[t2] - gt));
+    const float rho = decayed_suffix(sA[lane], gt, lane);
     sB[lane] = lane < b.nval ? 2.f * fast_exp(gt) * rho : 0.f;
     alpha = __builtin_bit_cast(float, __builtin_amdgcn_readlane(
                                           __builtin_bit_cast(int, fast_exp(2.f * gt) * rho), 0));
@@ -1617,7 +1674,7 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
   const int cg = wave & 3, fh = wave >> 2;   // column group, feature half (nt 4 fh .. 4 fh + 3)
   const int q4 = lane >> 4, l16 = lane & 15;
   const int gb = blockIdx.x, h = blockIdx.y, H = p.H;
-  const Blk b = block_of(p, gb);
+  const Blk b = block_of(p, gb, lane);
   if (b.nval <= 0) return;
   const int64_t DD = (int64_t)D * D;
   constexpr int NP = CB * 16 / C_NTHR;     // staging passes of 32 rows
@@ -1685,13 +1742,10 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
     for (int v = 0; v < 4; ++v) dnh += u[2 * j][v] * (float)h0[v] + u[2 * j + 1][v] * (float)h1[v];
     store8_i(sDn + dr * LDP, c, h8_of(u[2 * j], u[2 * j + 1], sd));
   }
-  dnh = wave_sum(dnh);
+  dnh = wave_sum_v(dnh);
   // rho_t (lane t of wave 0)
   if (wave == 0) {
-    float rho = 0.f;
-    const float gt = SC(CS_G, lane);
-    for (int t2 = lane; t2 < b.nval; ++t2) rho += SC(CS_A, t2) * fast_exp(2.f * (SC(CS_G, t2) - gt));
-    SC(CS_RHO, lane) = rho;
+    SC(CS_RHO, lane) = decayed_suffix(SC(CS_A, lane), SC(CS_G, lane), lane);
   }
   if (lane == 0) red[wave] = dnh;
   lds_barrier();
@@ -1787,8 +1841,7 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
       wk[jk] = h8_of(WK[2 * jk], WK[2 * jk + 1], sw);
     }
   }
-  rowdm += __shfl_xor(rowdm, 16, 64);
-  rowdm += __shfl_xor(rowdm, 32, 64);
+  rowdm = q4_sum(rowdm);
   // dk^T accumulators over this wave's feature half: in-block terms, then the lambda terms L
   f32x4 DK[4], L[4];
   const float beta2 = 2.f * fast_exp(gs) * rho_s;
@@ -1834,12 +1887,9 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
         qhx += dq[v] * HX[i][v];
       }
     }
-    kl += __shfl_xor(kl, 16, 64);
-    kl += __shfl_xor(kl, 32, 64);
-    kp += __shfl_xor(kp, 16, 64);
-    kp += __shfl_xor(kp, 32, 64);
-    qhx += __shfl_xor(qhx, 16, 64);
-    qhx += __shfl_xor(qhx, 32, 64);
+    kl = q4_sum(kl);
+    kp = q4_sum(kp);
+    qhx = q4_sum(qhx);
     if (q4 == 0) {
       float* xo = xch + (fh * CB + s) * 4;
       xo[0] = kl; xo[1] = kp; xo[2] = qhx;
@@ -1878,8 +1928,7 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
   }
   // sum of phi over the block (for the last token)
   float ph = phi;
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1) ph += __shfl_xor(ph, m, 64);
+  ph = row16_sum(ph);
   float dnh_all = 0.f;
 #pragma unroll
   for (int j = 0; j < C_NTHR / 64; ++j) dnh_all += red[j];
@@ -1891,10 +1940,9 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
   // dgk_u = sum_{t >= u} dL/dg_t within the block
   if (fh == 0 && q4 == 0) SC(CS_DG, s) = s_ok ? dg : 0.f;
   lds_barrier();
-  if (w.dgk && wave == 0 && lane < b.nval) {
-    float acc = 0.f;
-    for (int t2 = lane; t2 < b.nval; ++t2) acc += SC(CS_DG, t2);
-    w.dgk[(int64_t)(b.tok0 + lane) * H + h] = acc;
+  if (w.dgk && wave == 0) {
+    const float acc = suffix_sum64(SC(CS_DG, lane), lane);
+    if (lane < b.nval) w.dgk[(int64_t)(b.tok0 + lane) * H + h] = acc;
   }
 }
 
@@ -1942,7 +1990,7 @@ __global__ __launch_bounds__(NTHR, 2) void gla_e_kernel(Params p, GlaBwd w) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q4 = lane >> 4, l16 = lane & 15;
   const int gb = blockIdx.x, h = blockIdx.y, H = p.H;
-  const Blk b = block_of(p, gb);
+  const Blk b = block_of(p, gb, lane);
   if (b.nval <= 0) return;
   if (wave == 0) {
     const bool ok = lane < b.nval;
@@ -2038,7 +2086,7 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
   const int cg = wave & 3, fh = wave >> 2;   // column group, feature half (nt 4 fh .. 4 fh + 3)
   const int q4 = lane >> 4, l16 = lane & 15;
   const int gb = blockIdx.x, h = blockIdx.y, H = p.H;
-  const Blk b = block_of(p, gb);
+  const Blk b = block_of(p, gb, lane);
   if (b.nval <= 0) return;
   const int64_t DD = (int64_t)D * D;
   constexpr int NP = CB * 16 / GB_NTHR;    // staging passes of 32 rows
@@ -2111,7 +2159,7 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     store8_i(sDS + drw * LDP, dc0 + 8 * j, h8_of(dsv[2 * j], dsv[2 * j + 1], sds));
-  dss = wave_sum(dss);
+  dss = wave_sum_v(dss);
   if (lane == 0) red[wave] = dss;
   lds_barrier();
 
@@ -2193,10 +2241,8 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
         if (w.solve) *reinterpret_cast<f32x4*>(w.dx + ro + 16 * nt) = dxo;
       }
     }
-    dal += __shfl_xor(dal, 16, 64);
-    dal += __shfl_xor(dal, 32, 64);
-    udu += __shfl_xor(udu, 16, 64);
-    udu += __shfl_xor(udu, 32, 64);
+    dal = q4_sum(dal);
+    udu = q4_sum(udu);
     if (q4 == 0) {
       xo[0] = udu;
       xo[1] = dal;
@@ -2265,10 +2311,8 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
         else *reinterpret_cast<bf16x4*>(w.dk_bf + ro + 16 * nt) = bf4(y);
       }
     }
-    kdk += __shfl_xor(kdk, 16, 64);
-    kdk += __shfl_xor(kdk, 32, 64);
-    kdkx += __shfl_xor(kdkx, 16, 64);
-    kdkx += __shfl_xor(kdkx, 32, 64);
+    kdk = q4_sum(kdk);
+    kdkx = q4_sum(kdkx);
     if (q4 == 0) {
       xo[2] = kdk;
       xo[3] = kdkx;
@@ -2339,8 +2383,7 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
     kx = xa[3] + xb[3];
     if (q4 == 0 && w.solve) w.dalpha[ti] = xa[1] + xb[1];
   }
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1) kx += __shfl_xor(kx, m, 64);
+  kx = row16_sum(kx);
   float dss_all = 0.f;
 #pragma unroll
   for (int j = 0; j < GB_NTHR / 64; ++j) dss_all += red[j];
@@ -2353,10 +2396,9 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
     SC(GS_DG, s) = d;
   }
   lds_barrier();
-  if (wave == 0 && lane < b.nval) {
-    float acc = 0.f;
-    for (int t2 = lane; t2 < b.nval; ++t2) acc += SC(GS_DG, t2);
-    w.dg[(int64_t)(b.tok0 + lane) * H + h] = acc;
+  if (wave == 0) {
+    const float acc = suffix_sum64(lane < b.nval ? SC(GS_DG, lane) : 0.f, lane);
+    if (lane < b.nval) w.dg[(int64_t)(b.tok0 + lane) * H + h] = acc;
   }
 }
 }  // namespace train

@@ -152,6 +152,44 @@ __device__ __forceinline__ float pow2f(int n) {
   return __builtin_bit_cast(float, (uint32_t)(127 + n) << 23);
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dppf(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                                               0xF, 0xF, false));
+}
+// The sums of x[0..3] over the 16 lanes of a DPP row, by a transposing reduction
+// (five DPP additions instead of sixteen): lane l16 receives the sum of x[l16 & 3].
+__device__ __forceinline__ float row16_sum4(const f32x4& x, int l16) {
+  const bool b = l16 & 1, c = l16 & 2;
+  const float y0 = (b ? x[1] : x[0]) + dppf<0xB1>(b ? x[0] : x[1]);   // x[b], lanes l, l ^ 1
+  const float y1 = (b ? x[3] : x[2]) + dppf<0xB1>(b ? x[2] : x[3]);   // x[b + 2]
+  float z = (c ? y1 : y0) + dppf<0x4E>(c ? y0 : y1);                   // x[l & 3], l ^ 2 too
+  z += dppf<0x124>(z);                                                  // row_ror:4
+  z += dppf<0x128>(z);                                                  // row_ror:8
+  return z;
+}
+
+// a + b with their halves of 32 lanes exchanged: lanes 0-31 receive a's sums over the
+// lane pairs (l, l + 32), lanes 32-63 b's; with b = a the pair's sum in every lane
+// (lane swaps in the VALU, where __shfl_xor goes through the LDS).
+__device__ __forceinline__ float pair_sum32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a),
+                                                  __builtin_bit_cast(unsigned, b), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+// the same over (l, l + 16): even rows of 16 lanes receive a's sums, odd rows b's
+__device__ __forceinline__ float pair_sum16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a),
+                                                  __builtin_bit_cast(unsigned, b), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+// sum over the four lanes l16, l16 + 16, l16 + 32, l16 + 48
+__device__ __forceinline__ float q4_sum(float x) {
+  x = pair_sum16(x, x);
+  return pair_sum32(x, x);
+}
+__device__ __forceinline__ float wave_sum_v(float x) { return q4_sum(row16_sum(x)); }
+
 // Inclusive prefix sum over lanes 0..31 (two DPP rows) with VALU lane shifts.
 #define HMX_DPP_F(v, ctrl, rmask) \
   __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (v)), (ctrl), \

@@ -442,41 +442,6 @@ struct GLay {
   static_assert(BYTES <= 160 * 1024 && P >= L, "LDS budget");
 };
 
-template <int CTRL>
-__device__ __forceinline__ float dppf(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
-                                                               0xF, 0xF, false));
-}
-// The sums of x[0..3] over the 16 lanes of a DPP row by a transposing reduction: lane
-// l16 receives the sum of x[l16 & 3].
-__device__ __forceinline__ float row16_sum4(const f32x4& x, int l16) {
-  const bool b = l16 & 1, c = l16 & 2;
-  const float y0 = (b ? x[1] : x[0]) + dppf<0xB1>(b ? x[0] : x[1]);
-  const float y1 = (b ? x[3] : x[2]) + dppf<0xB1>(b ? x[2] : x[3]);
-  float z = (c ? y1 : y0) + dppf<0x4E>(c ? y0 : y1);
-  z += dppf<0x124>(z);
-  z += dppf<0x128>(z);
-  return z;
-}
-// a + b with their halves of 32 lanes exchanged: lanes 0-31 receive a over the lane
-// pairs (l, l + 32), lanes 32-63 b; with b = a the sum over the pair in every lane
-__device__ __forceinline__ float pair_sum32(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a),
-                                                  __builtin_bit_cast(unsigned, b), false, false);
-  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-}
-// the same over (l, l + 16): even rows of 16 lanes receive a's sums, odd rows b's
-__device__ __forceinline__ float pair_sum16(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a),
-                                                  __builtin_bit_cast(unsigned, b), false, false);
-  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-}
-__device__ __forceinline__ float wave_sum_v(float x) {
-  x = row16_sum(x);
-  x = pair_sum16(x, x);
-  return pair_sum32(x, x);
-}
-
 // row and transposed fragments of interleaved bf16 rows (mfma.hpp)
 __device__ __forceinline__ bf16x8 fr(const bf16* b, int ld, int r0, int k0, int lane) {
   return __builtin_bit_cast(bf16x8, frag_i(reinterpret_cast<const f16*>(b), ld, r0, k0, lane));
