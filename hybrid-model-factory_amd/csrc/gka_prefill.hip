@@ -107,10 +107,12 @@ struct Params {
   float on_eps;
   // the training solve (SM_X / SM_DQ / SM_GLA_SAVE solve kernels): |H_t|_F per token
   // [tokens][H] (written by SM_X and SM_GLA_SAVE, read by SM_DQ), the fp32 solution
-  // of SM_DQ [tokens][H][D] (added to what it holds when xo32_acc), and the solution
-  // x (before the alpha blend) saved by SM_GLA_SAVE [tokens][H][D] bf16
-  float* fro; float* xo32; int xo32_acc; bf16* xs;
-  const float* rhs32;                     // SM_DQ: an fp32 right-hand side in place of p.q
+  // of SM_DQ [tokens][H][D] and its bf16 copy dq_out, and the solution x (before the
+  // alpha blend) saved by SM_GLA_SAVE [tokens][H][D] bf16
+  float* fro; float* xo32; bf16* dq_out; bf16* xs;
+  // SM_DQ under the alpha blend: the fp32 gradient du of the blended query; the
+  // right-hand side is then alpha du (in place of p.q) and dq_out gains (1 - alpha) du
+  const float* du32;
 };
 
 // The fused gates' raw projection values as bits (one load in either dtype
@@ -592,7 +594,8 @@ __device__ __forceinline__ void h8_hilo(const f32x4& t0, const f32x4& t1, f16x8&
 
 // A block-start state X = dX_b + e^{off} X_seg (both fp16; dX_b is zero for a
 // segment's first block), this thread's 64 elements: row tid/2, half tid&1.
-struct StateLd { f16x8 b[8], s[8]; };
+// The workgroup's first NT threads hold D / NT rows' pieces each (256: as above).
+template <int NT = NTHR> struct StateLd { static constexpr int NPC = 16 * D / NT; f16x8 b[NPC], s[NPC]; };
 
 // The loads of a block-start state (tile-major; null: zero) and of its segment's
 // start state (rows; null: dropped), issued separately so the second can wait for
@@ -603,21 +606,23 @@ template <bool SYM>
 __device__ __forceinline__ bool piece_kept(int r, int c) {
   return !SYM || (r >> 4) <= (c >> 4);
 }
-template <bool SYM>
-__device__ __forceinline__ void state_issue_b(StateLd& L, const f16* xb, int tid) {
-  const int r = tid >> 1, c0 = (tid & 1) * 64;
+template <bool SYM, int NT>
+__device__ __forceinline__ void state_issue_b(StateLd<NT>& L, const f16* xb, int tid) {
+  constexpr int NPC = StateLd<NT>::NPC;
+  const int r = tid / (16 / NPC), c0 = (tid % (16 / NPC)) * 8 * NPC;
   const f16* xbr = xb ? xb + blk_index(r, c0) : nullptr;   // 8-element pieces: fixed offsets
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
+  for (int j = 0; j < NPC; ++j)
     L.b[j] = (xbr && piece_kept<SYM>(r, c0 + 8 * j))
                  ? *reinterpret_cast<const f16x8*>(xbr + (j >> 1) * 256 + (j & 1) * 8)
                  : f16x8{};
 }
-template <bool SYM>
-__device__ __forceinline__ void state_issue_s(StateLd& L, const f16* xs, int tid) {
-  const int r = tid >> 1, c0 = (tid & 1) * 64;
+template <bool SYM, int NT>
+__device__ __forceinline__ void state_issue_s(StateLd<NT>& L, const f16* xs, int tid) {
+  constexpr int NPC = StateLd<NT>::NPC;
+  const int r = tid / (16 / NPC), c0 = (tid % (16 / NPC)) * 8 * NPC;
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
+  for (int j = 0; j < NPC; ++j)
     L.s[j] = (xs && piece_kept<SYM>(r, c0 + 8 * j))
                  ? *reinterpret_cast<const f16x8*>(xs + r * D + c0 + 8 * j)
                  : f16x8{};
@@ -629,12 +634,13 @@ constexpr float SEG_STATE_DROP = -20.f;
 // Writes the state into LDS as fp16 rows; returns this thread's sum of squares.
 // (SYM: of the upper tiles, each off-diagonal tile standing for itself and its
 // mirror in the sum of squares.)
-template <bool SYM>
-__device__ __forceinline__ float state_store(f16* dst, const StateLd& L, float dec, int tid) {
-  const int r = tid >> 1, c0 = (tid & 1) * 64;
+template <bool SYM, int NT>
+__device__ __forceinline__ float state_store(f16* dst, const StateLd<NT>& L, float dec, int tid) {
+  constexpr int NPC = StateLd<NT>::NPC;
+  const int r = tid / (16 / NPC), c0 = (tid % (16 / NPC)) * 8 * NPC;
   float ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < NPC; ++j) {
     const int c = c0 + 8 * j;
     if (!piece_kept<SYM>(r, c)) continue;
     f16x8 y;
@@ -720,7 +726,7 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
   const int64_t bo = ((int64_t)gb * H + h) * 2;
   const int64_t so = ((int64_t)s_id * H + h) * DD;
   const int64_t bso = ((int64_t)gb * H + h) * DD;
-  StateLd hst;
+  StateLd<> hst;
   if constexpr (SOLVE) state_issue_b<true>(hst, lb > 0 ? p.ws_hb + bso : nullptr, tid);
   const float off_gk = p.ws_boff[bo + 0], off_g = p.ws_boff[bo + 1];
   if constexpr (SOLVE)
@@ -765,16 +771,21 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
   const int tb = 16 * wave + l16;
   const bool tok_ok = tb < nval;
   f32x4 Q[8];
+  [[maybe_unused]] f32x4 Du[MODE == SM_DQ ? 8 : 1];
+  const float al_dq = (MODE == SM_DQ && p.du32 && tok_ok)
+                          ? ldsc(p.alpha, (int64_t)(tok0 + tb) * H + h, p.alpha_dt) : 0.f;
   const bf16* qr = p.q + (int64_t)(tok0 + tb) * p.q_ts + (int64_t)h * D + 4 * q4;
   float rq;
   {
     float ss = 0.f;
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt) {
-      if (MODE == SM_DQ && p.rhs32) {
-        Q[nt] = tok_ok ? *reinterpret_cast<const f32x4*>(p.rhs32 + ((int64_t)(tok0 + tb) * H + h) * D +
-                                                         4 * q4 + 16 * nt)
-                       : f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (MODE == SM_DQ) Du[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (MODE == SM_DQ && p.du32) {
+        if (tok_ok)
+          Du[nt] = *reinterpret_cast<const f32x4*>(p.du32 + ((int64_t)(tok0 + tb) * H + h) * D +
+                                                   4 * q4 + 16 * nt);
+        Q[nt] = Du[nt] * al_dq;
       } else {
         const bf16x4 x = tok_ok ? *reinterpret_cast<const bf16x4*>(qr + 16 * nt) : bf16x4{};
 #pragma unroll
@@ -1033,13 +1044,10 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
             for (int v = 0; v < 4; ++v) y[v] = (bf16)X[nt][v];
             *reinterpret_cast<bf16x4*>((MODE == SM_X ? p.o : p.xs) + ro + 16 * nt) = y;
           } else {
-            f32x4 y = X[nt];
-            if (p.xo32_acc) {
-              const f32x4 o0 = *reinterpret_cast<const f32x4*>(p.xo32 + ro + 16 * nt);
-#pragma unroll
-              for (int v = 0; v < 4; ++v) y[v] += o0[v];
-            }
-            *reinterpret_cast<f32x4*>(p.xo32 + ro + 16 * nt) = y;
+            *reinterpret_cast<f32x4*>(p.xo32 + ro + 16 * nt) = X[nt];
+            const f32x4 y = X[nt] + Du[nt] * (1.f - al_dq);
+            *reinterpret_cast<bf16x4*>(p.dq_out + ro + 16 * nt) =
+                bf16x4{(bf16)y[0], (bf16)y[1], (bf16)y[2], (bf16)y[3]};
           }
         }
       }
@@ -1065,7 +1073,7 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
   // ---- GLA output: o^T = scale [e^{G_t} S_c^T x^ + V~^T Z'^T] ---------------
   // The S_c loads go out first; the in-block products (they need only k~) run while
   // they arrive.
-  StateLd sst;
+  StateLd<> sst;
   state_issue_b<false>(sst, lb > 0 ? p.ws_sb + bso : nullptr, tid);
   state_issue_s<false>(sst, (lb == 0 || off_g > SEG_STATE_DROP) ? p.ws_s0 + so : nullptr, tid);
   if constexpr (!SOLVE) lds_barrier();     // the staged k~, v~ and gates
@@ -1344,8 +1352,6 @@ struct Bwd {
   float* gam;             // [nblk][H] block totals of gk
   bf16* dk;               // [tokens][H][D] the gradient of k (+ dk_add when given)
   const float* dk_add;    // null, or [tokens][H][D] fp32 added to dk
-  bf16* dq_out;           // [tokens][H][D] the gradient of the right-hand side (+ dq_add)
-  const float* dq_add;    // null, or [tokens][H][D] fp32 added to dq_out
   float* dgk;             // [tokens][H]
   int bp_lambda;
 };
@@ -1367,7 +1373,7 @@ __device__ __forceinline__ void load_hc(const Params& p, f16* sH, const Blk& b, 
     const int64_t DD = (int64_t)D * D;
     const int64_t so = ((int64_t)b.s_id * p.H + h) * DD;
     const int64_t bso = ((int64_t)gb * p.H + h) * DD;
-    StateLd hst;
+    StateLd<> hst;
     solve::state_issue_b<true>(hst, b.lb > 0 ? p.ws_hb + bso : nullptr, tid);
     const float off_gk = p.ws_boff[((int64_t)gb * p.H + h) * 2];
     solve::state_issue_s<true>(hst, (b.lb == 0 || off_gk > solve::SEG_STATE_DROP) ? p.ws_h0 + so : nullptr, tid);
@@ -1645,24 +1651,31 @@ __global__ __launch_bounds__(256) void cheb_dscan_kernel(Params p, Bwd w) {
   }
 }
 
+constexpr int LDB = CB + 8;               // fp16 [64][LDB] in-block matrices: 36 dwords
 constexpr int C_OFF_K = 0, C_OFF_X = SZ_K, C_OFF_Q = 2 * SZ_K, C_OFF_H = 3 * SZ_K;
 constexpr int C_OFF_DN = C_OFF_H + SZ_H, C_OFF_SC = C_OFF_DN + SZ_H;
-enum { CS_G, CS_A, CS_RHO, CS_DG, CS_COL0, NCS = CS_COL0 + 4 };
+enum { CS_G, CS_A, CS_A1, CS_RHO, CS_DG, CS_COL0, NCS = CS_COL0 + 4 };
 // 8 waves: wave w takes the 16 columns s of group w & 3 and the feature half w >> 2
 constexpr int C_NTHR = 512;
 constexpr int C_OFF_RED = C_OFF_SC + NCS * CB * 4;        // 16 floats of cross-wave sums
 constexpr int C_OFF_MS = C_OFF_RED + 16 * 4;              // 24 floats for block_max
 constexpr int C_OFF_XCH = C_OFF_MS + 24 * 4;              // [2][64][4] feature-half dot products
 constexpr int C_SMEM = C_OFF_XCH + 2 * CB * 4 * 4;
-static_assert(C_SMEM <= 160 * 1024, "LDS budget");
+static_assert(C_SMEM <= 160 * 1024 && 3 * CB * LDB * 2 <= SZ_H, "LDS budget");
 
-// dk and dgk of block gb (see the section comment)
-__global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
+// dk and dgk of block gb (see the section comment).
+// One workgroup per CU (134 KB of LDS): every load of the block is issued before the
+// first wait, x and dq in the layout of dk's tiles (so dq is read once, for its products
+// and for dgk's dot products).  The in-block matrices x_t.k_s, dq_t.k_s and W_st k_t.k_s
+// are formed once, two of each one's sixteen tiles per wave, and shared through the LDS
+// of h_c.
+__global__ __launch_bounds__(C_NTHR, 2) void cheb_dk_kernel(Params p, Bwd w) {
   __shared__ __align__(16) unsigned char smem[C_SMEM];
   f16* sK = reinterpret_cast<f16*>(smem + C_OFF_K);
   f16* sX = reinterpret_cast<f16*>(smem + C_OFF_X);
   f16* sQ = reinterpret_cast<f16*>(smem + C_OFF_Q);
   f16* sH = reinterpret_cast<f16*>(smem + C_OFF_H);
+  f16 *sS1 = sH, *sS2 = sH + CB * LDB, *sWK = sH + 2 * CB * LDB;   // rows s, columns t
   f16* sDn = reinterpret_cast<f16*>(smem + C_OFF_DN);
   float* sc = reinterpret_cast<float*>(smem + C_OFF_SC);
   float* red = reinterpret_cast<float*>(smem + C_OFF_RED);
@@ -1679,90 +1692,111 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
   const int64_t DD = (int64_t)D * D;
   constexpr int NP = CB * 16 / C_NTHR;     // staging passes of 32 rows
 
-  load_hc(p, sH, b, gb, h, tid, wave, lane, C_NTHR / 64);
-  if (wave == 0) SC(CS_G, lane) = block_decay(p, b, h, lane);
-  // the rows (x, dq and Dn scaled into fp16's range) and a_t
-  bf16x8 kr[NP], xr[NP];
-  f32x4 q0[NP], q1[NP];
-  const bf16* dn = w.e + ((int64_t)gb * H + h) * DD;
-  const int dr = tid >> 2, dc0 = (tid & 3) * 32;    // this thread's Dn: row dr, columns dc0..+31
-  f32x4 u[8];
-  float mx[3] = {0.f, 0.f, 0.f};            // max |x|, |dq|, |Dn|
+  const int s = 16 * cg + l16;              // this lane's key / token column
+  const bool s_ok = s < b.nval;
+  const int64_t ts = (int64_t)(b.tok0 + s) * H + h;
+  const int64_t ro = ts * D + 64 * fh + 4 * q4;   // + 16 i: features 64 fh + 16 i + 4 q4 .. +3
+
+  // ---- loads ---------------------------------------------------------------------
+  const int64_t so = ((int64_t)b.s_id * H + h) * DD;
+  const int64_t bso = ((int64_t)gb * H + h) * DD;
+  StateLd<C_NTHR> hst;
+  solve::state_issue_b<true>(hst, b.lb > 0 ? p.ws_hb + bso : nullptr, tid);
+  const float off_gk = p.ws_boff[((int64_t)gb * H + h) * 2];
+  // Dn: wave w's tile row w, column j (rows 16 w + l16, columns 16 j + 4 q4 ..)
+  bf16x4 dn[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    dn[j] = *reinterpret_cast<const bf16x4*>(w.e + bso + blk_index(16 * wave + l16, 16 * j + 4 * q4));
+  bf16x8 kr[NP];
 #pragma unroll
   for (int pass = 0; pass < NP; ++pass) {
     const int row = pass * 32 + (tid >> 4), f0 = (tid & 15) * 8;
-    const bool ok = row < b.nval;
-    const int64_t ro = ((int64_t)(b.tok0 + row) * H + h) * D + f0;
-    kr[pass] = ok ? *reinterpret_cast<const bf16x8*>(p.k + (int64_t)(b.tok0 + row) * p.kv_ts + h * D + f0) : bf16x8{};
-    xr[pass] = ok ? *reinterpret_cast<const bf16x8*>(w.x + ro) : bf16x8{};
-    q0[pass] = ok ? *reinterpret_cast<const f32x4*>(w.dq + ro) : f32x4{0.f, 0.f, 0.f, 0.f};
-    q1[pass] = ok ? *reinterpret_cast<const f32x4*>(w.dq + ro + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-    mx[0] = fmaxf(mx[0], absmax8(xr[pass]));
-    mx[1] = fmaxf(mx[1], fmaxf(absmax4(q0[pass]), absmax4(q1[pass])));
-    const float a = lambda_weight(p, w, b, row, h, q0[pass], q1[pass], xr[pass]);
-    if (l16 == 0) SC(CS_A, row) = a;
-    if (ok) {                             // the caller's dq: this solve's (+ dq_add), bf16
-      f32x4 y0 = q0[pass], y1 = q1[pass];
-      if (w.dq_add) {
-        const f32x4 o0 = *reinterpret_cast<const f32x4*>(w.dq_add + ro);
-        const f32x4 o1 = *reinterpret_cast<const f32x4*>(w.dq_add + ro + 4);
+    kr[pass] = row < b.nval
+                   ? *reinterpret_cast<const bf16x8*>(p.k + (int64_t)(b.tok0 + row) * p.kv_ts + h * D + f0)
+                   : bf16x8{};
+  }
+  bf16x4 xr[4];
+  f32x4 dq[4], dk0[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          y0[v] += o0[v];
-          y1[v] += o1[v];
-        }
-      }
-      *reinterpret_cast<bf16x8*>(w.dq_out + ro) =
-          bf16x8{(bf16)y0[0], (bf16)y0[1], (bf16)y0[2], (bf16)y0[3],
-                 (bf16)y1[0], (bf16)y1[1], (bf16)y1[2], (bf16)y1[3]};
-    }
+  for (int i = 0; i < 4; ++i) {
+    xr[i] = s_ok ? *reinterpret_cast<const bf16x4*>(w.x + ro + 16 * i) : bf16x4{};
+    dq[i] = s_ok ? *reinterpret_cast<const f32x4*>(w.dq + ro + 16 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float fro = s_ok ? w.fro[ts] : 0.f;
+  const float g_l = wave == 0 ? block_decay(p, b, h, lane) : 0.f;
+  solve::state_issue_s<true>(hst, (b.lb == 0 || off_gk > solve::SEG_STATE_DROP) ? p.ws_h0 + so : nullptr, tid);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    dk0[i] = (s_ok && w.dk_add) ? *reinterpret_cast<const f32x4*>(w.dk_add + ro + 16 * i)
+                                : f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // ---- staging (x, dq and Dn scaled into fp16's range) and a_t's halves -----------------
+  if (wave == 0) SC(CS_G, lane) = g_l;
+  float mx[3] = {0.f, 0.f, 0.f};            // max |x|, |dq|, |Dn|
+  float qx = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 xf = f4(xr[i]);
+    mx[0] = fmaxf(mx[0], absmax4(xf));
+    mx[1] = fmaxf(mx[1], absmax4(dq[i]));
+#pragma unroll
+    for (int v = 0; v < 4; ++v) qx += dq[i][v] * xf[v];
   }
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    u[j] = f4(*reinterpret_cast<const bf16x4*>(dn + blk_index(dr, dc0 + 4 * j)));
-    mx[2] = fmaxf(mx[2], absmax4(u[j]));
-  }
-  block_max<3, C_NTHR / 64>(mx, mslot, wave, lane);   // (its barrier also orders h_c's lower tiles)
+  for (int j = 0; j < 8; ++j) mx[2] = fmaxf(mx[2], absmax4(f4(dn[j])));
+  qx = q4_sum(qx);
+  // a_t = -r (dq_t . x_t) / |H_t|_F, this feature half's part (0 without bp_lambda)
+  const float a_half = (w.bp_lambda && fro > 0.f) ? -p.ridge_ratio * qx / fro : 0.f;
+  if (q4 == 0) SC(CS_A + fh, s) = a_half;
+  solve::state_store<true>(sH, hst, fast_exp(off_gk), tid);
+  block_max<3, C_NTHR / 64>(mx, mslot, wave, lane);
   const float sx = pow2_scale(mx[0]), sq = pow2_scale(mx[1]), sd = pow2_scale(mx[2]);
+  solve::state_fill_lower(sH, wave, lane, C_NTHR / 64);
+  if (wave == 0)                            // rho_t (lane t)
+    SC(CS_RHO, lane) = decayed_suffix(SC(CS_A, lane) + SC(CS_A1, lane), g_l, lane);
 #pragma unroll
   for (int pass = 0; pass < NP; ++pass) {
     const int row = pass * 32 + (tid >> 4), f0 = (tid & 15) * 8;
     store8_i(sK + row * LDP, f0, scale_h8(kr[pass], 1.f));
-    store8_i(sX + row * LDP, f0, scale_h8(xr[pass], sx));
-    store8_i(sQ + row * LDP, f0, h8_of(q0[pass], q1[pass], sq));
   }
-  // Dn into LDS and <Dn, h_c> in fp32
-  float dnh = 0.f;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = dc0 + 8 * j;
-    const f16x4 h0 = *reinterpret_cast<const f16x4*>(sH + dr * LDP + icol(c));
-    const f16x4 h1 = *reinterpret_cast<const f16x4*>(sH + dr * LDP + icol(c + 4));
+  for (int i = 0; i < 4; ++i) {
+    const int o = s * LDP + icol(64 * fh + 16 * i + 4 * q4);
+    *reinterpret_cast<f16x4*>(sX + o) = h4(f4(xr[i]) * sx);
+    *reinterpret_cast<f16x4*>(sQ + o) = h4(dq[i] * sq);
+  }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) dnh += u[2 * j][v] * (float)h0[v] + u[2 * j + 1][v] * (float)h1[v];
-    store8_i(sDn + dr * LDP, c, h8_of(u[2 * j], u[2 * j + 1], sd));
-  }
-  dnh = wave_sum_v(dnh);
-  // rho_t (lane t of wave 0)
-  if (wave == 0) {
-    SC(CS_RHO, lane) = decayed_suffix(SC(CS_A, lane), SC(CS_G, lane), lane);
-  }
-  if (lane == 0) red[wave] = dnh;
+  for (int j = 0; j < 8; ++j)
+    *reinterpret_cast<f16x4*>(sDn + (16 * wave + l16) * LDP + icol(16 * j + 4 * q4)) = h4(f4(dn[j]) * sd);
   lds_barrier();
 
-  const int s = 16 * cg + l16;              // this lane's key / token column
-  const bool s_ok = s < b.nval;
+  // <Dn, h_c> in fp32
+  float dnh = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const f32x4 d = f4(dn[j]);
+    const f16x4 hv = *reinterpret_cast<const f16x4*>(sH + (16 * wave + l16) * LDP + icol(16 * j + 4 * q4));
+#pragma unroll
+    for (int v = 0; v < 4; ++v) dnh += d[v] * (float)hv[v];
+  }
+  dnh = wave_sum_v(dnh);
+  if (lane == 0) red[wave] = dnh;
   const float gs = SC(CS_G, s);
   const float Gam = SC(CS_G, b.nval - 1);
   // products with h_c and Dn over this wave's feature half: HK = h_c k_s, HX = h_c x_s,
-  // P = Dn k_s (rows f = 16 (4 fh + i) + 4 q4 + v, column s)
-  f32x4 HK[4], HX[4], P[4];
+  // P = Dn k_s (rows f = 16 (4 fh + i) + 4 q4 + v, column s); and the wave's two tiles
+  // (rows t = 16 (2 fh + j) + 4 q4 + v, column s) of XK = x_t . k_s, QK = dq_t . k_s and
+  // KK = k_t . k_s
+  f32x4 HK[4], HX[4], P[4], XK[2], QK[2], KK[2];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     HK[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     HX[i] = HK[i];
     P[i] = HK[i];
   }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) XK[j] = QK[j] = KK[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
     const f16x8 bk = frag_i(sK, LDP, 16 * cg, 32 * ks, lane);
@@ -1775,73 +1809,57 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
       HX[i] = mfma16h(ah, bx, HX[i]);
       P[i] = mfma16h(frag_i(sDn, LDP, 16 * nt, 32 * ks, lane), bk, P[i]);
     }
-  }
-  // in-block products over the 64 tokens t (rows) for this wave's columns s:
-  // XK = x_t . k_s, QK = dq_t . k_s, KK = k_t . k_s (both feature halves form them)
-  f32x4 XK[4], QK[4], KK[4];
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt) {
-    XK[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    QK[tt] = XK[tt];
-    KK[tt] = XK[tt];
-  }
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    const f16x8 bk = frag_i(sK, LDP, 16 * cg, 32 * ks, lane);
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      XK[tt] = mfma16h(frag_i(sX, LDP, 16 * tt, 32 * ks, lane), bk, XK[tt]);
-      QK[tt] = mfma16h(frag_i(sQ, LDP, 16 * tt, 32 * ks, lane), bk, QK[tt]);
-      KK[tt] = mfma16h(frag_i(sK, LDP, 16 * tt, 32 * ks, lane), bk, KK[tt]);
+    for (int j = 0; j < 2; ++j) {
+      const int t0 = 16 * (2 * fh + j);
+      XK[j] = mfma16h(frag_i(sX, LDP, t0, 32 * ks, lane), bk, XK[j]);
+      QK[j] = mfma16h(frag_i(sQ, LDP, t0, 32 * ks, lane), bk, QK[j]);
+      KK[j] = mfma16h(frag_i(sK, LDP, t0, 32 * ks, lane), bk, KK[j]);
     }
   }
   // masks and the scalar sums: m_ts = e^{g_t - g_s} (t >= s); dm = (x_t.k_s)(dq_t.k_s) m_ts
   // (XK carries the scale sx and QK sq: S1 and S2 keep them, dm is unscaled)
   const float rho_s = SC(CS_RHO, s);
   const float uxq = 1.f / (sx * sq);
-  float rowdm = 0.f, sw;
-  f16x8 s1[2], s2[2], wk[2];
-  {
-    f32x4 S1[4], S2[4], WK[4];
+  float rowdm = 0.f, mw = 0.f;
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      const f32x4 gt4 = *reinterpret_cast<const f32x4*>(&SC(CS_G, 16 * tt + 4 * q4));
-      const f32x4 rt4 = *reinterpret_cast<const f32x4*>(&SC(CS_RHO, 16 * tt + 4 * q4));
-      float col[4];
+  for (int j = 0; j < 2; ++j) {
+    const int tt = 2 * fh + j;
+    const f32x4 gt4 = *reinterpret_cast<const f32x4*>(&SC(CS_G, 16 * tt + 4 * q4));
+    const f32x4 rt4 = *reinterpret_cast<const f32x4*>(&SC(CS_RHO, 16 * tt + 4 * q4));
+    f32x4 col;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int t = 16 * tt + 4 * q4 + v;
-        const float m = (t >= s && t < b.nval) ? fast_exp(gt4[v] - gs) : 0.f;
-        S1[tt][v] = -XK[tt][v] * m;
-        S2[tt][v] = -QK[tt][v] * m;
-        const float dm = XK[tt][v] * QK[tt][v] * m * uxq;
-        rowdm += dm;
-        col[v] = dm;
-        // W_st with mm = max(s, t): e^{(g_mm - g_s) + (g_mm - g_t)} rho_mm
-        const bool sl = t >= s;
-        const float gm = sl ? gt4[v] : gs;
-        const float wst = (t < b.nval && s_ok) ? fast_exp((gm - gs) + (gm - gt4[v])) * (sl ? rt4[v] : rho_s) : 0.f;
-        WK[tt][v] = 2.f * wst * KK[tt][v];
-      }
-      // column sums over this wave's s (the 16 lanes of each row group)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float cs = row16_sum(col[v]);
-        if (fh == 0 && l16 == 0) SC(CS_COL0 + cg, 16 * tt + 4 * q4 + v) = cs;
-      }
+    for (int v = 0; v < 4; ++v) {
+      const int t = 16 * tt + 4 * q4 + v;
+      const float m = (t >= s && t < b.nval) ? fast_exp(gt4[v] - gs) : 0.f;
+      const float dm = XK[j][v] * QK[j][v] * m * uxq;
+      rowdm += dm;
+      col[v] = dm;
+      XK[j][v] *= -m;
+      QK[j][v] *= -m;
+      // W_st with mm = max(s, t): e^{(g_mm - g_s) + (g_mm - g_t)} rho_mm
+      const bool sl = t >= s;
+      const float gm = sl ? gt4[v] : gs;
+      const float wst = (t < b.nval && s_ok) ? fast_exp((gm - gs) + (gm - gt4[v])) * (sl ? rt4[v] : rho_s) : 0.f;
+      KK[j][v] = 2.f * wst * KK[j][v];
     }
-    float mw = 0.f;
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) mw = fmaxf(mw, absmax4(WK[tt]));
-    sw = pow2_scale(wave_max(mw));
-#pragma unroll
-    for (int jk = 0; jk < 2; ++jk) {
-      s1[jk] = h8(S1[2 * jk], S1[2 * jk + 1]);
-      s2[jk] = h8(S2[2 * jk], S2[2 * jk + 1]);
-      wk[jk] = h8_of(WK[2 * jk], WK[2 * jk + 1], sw);
-    }
+    const float cs = row16_sum4(col, l16);   // over this wave's 16 columns s
+    if (l16 < 4) SC(CS_COL0 + cg, 16 * tt + 4 * q4 + l16) = cs;
+    mw = fmaxf(mw, absmax4(KK[j]));
   }
+  mw = wave_max(mw);
+  if (lane == 0) mslot[wave] = mw;
   rowdm = q4_sum(rowdm);
+  lds_barrier();                            // every wave is done with h_c
+  const float sw = pow2_scale(fmaxf(mslot[cg], mslot[cg + 4]));   // the column group's
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int o = s * LDB + icol(16 * (2 * fh + j) + 4 * q4);
+    *reinterpret_cast<f16x4*>(sS1 + o) = h4(XK[j]);
+    *reinterpret_cast<f16x4*>(sS2 + o) = h4(QK[j]);
+    *reinterpret_cast<f16x4*>(sWK + o) = h4(KK[j] * sw);
+  }
+  lds_barrier();
   // dk^T accumulators over this wave's feature half: in-block terms, then the lambda terms L
   f32x4 DK[4], L[4];
   const float beta2 = 2.f * fast_exp(gs) * rho_s;
@@ -1851,68 +1869,46 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
     L[i] = DK[i];
   }
 #pragma unroll
-  for (int jk = 0; jk < 2; ++jk)
+  for (int jk = 0; jk < 2; ++jk) {
+    const f16x8 wk = frag_i(sWK, LDB, 16 * cg, 32 * jk, lane);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) L[i] = mfma16h(frag_t_i(sK, LDP, 32 * jk, 16 * (4 * fh + i), lane), wk, L[i]);
+    if (jk == 0 && cg >= 2) continue;       // the tokens before every key of this column group
+    const f16x8 s1 = frag_i(sS1, LDB, 16 * cg, 32 * jk, lane);
+    const f16x8 s2 = frag_i(sS2, LDB, 16 * cg, 32 * jk, lane);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int nt = 4 * fh + i;
-      DK[i] = mfma16h(frag_t_i(sQ, LDP, 32 * jk, 16 * nt, lane), s1[jk], DK[i]);
-      DK[i] = mfma16h(frag_t_i(sX, LDP, 32 * jk, 16 * nt, lane), s2[jk], DK[i]);
-      L[i] = mfma16h(frag_t_i(sK, LDP, 32 * jk, 16 * nt, lane), wk[jk], L[i]);
+      DK[i] = mfma16h(frag_t_i(sQ, LDP, 32 * jk, 16 * (4 * fh + i), lane), s1, DK[i]);
+      DK[i] = mfma16h(frag_t_i(sX, LDP, 32 * jk, 16 * (4 * fh + i), lane), s2, DK[i]);
     }
-  // unscale: DK (sx sq), L's MFMA part (sw), P (sd), HX (sx)
+  }
+  // unscale: DK (sx sq), L's MFMA part (sw), P (sd), HX (sx); the dot products of column s
+  // with k_s and dq_s (fp32) over this feature half; dk_s = DK + L + e^{Gam - g_s} P
   const float uw = 1.f / sw, ud = 1.f / sd, ux = 1.f / sx;
+  const float ec = fast_exp(Gam - gs);
+  float kl = 0.f, kp = 0.f, qhx = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 4; ++i) {
+    const f16x4 kk = *reinterpret_cast<const f16x4*>(sK + s * LDP + icol(64 * fh + 16 * i + 4 * q4));
+    f32x4 y;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      DK[i][v] *= uxq;
-      L[i][v] = uw * L[i][v] + beta2 * HK[i][v];
-      P[i][v] *= ud;
-      HX[i][v] *= ux;
+      const float l = uw * L[i][v] + beta2 * HK[i][v], pv = P[i][v] * ud;
+      kl += (float)kk[v] * l;
+      kp += (float)kk[v] * pv;
+      qhx += dq[i][v] * (HX[i][v] * ux);
+      y[v] = DK[i][v] * uxq + l + ec * pv + dk0[i][v];
     }
-  // per-column dot products with k_s, dq_s (fp32 from memory) over both feature halves
-  const float ec = fast_exp(Gam - gs);
-  const int64_t ro = ((int64_t)(b.tok0 + s) * H + h) * D + 4 * q4;
-  float kl = 0.f, kp = 0.f, qhx = 0.f;
-  {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int nt = 4 * fh + i;
-      const f16x4 kk = *reinterpret_cast<const f16x4*>(sK + s * LDP + icol(16 * nt + 4 * q4));
-      const f32x4 dq = s_ok ? *reinterpret_cast<const f32x4*>(w.dq + ro + 16 * nt) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        kl += (float)kk[v] * L[i][v];
-        kp += (float)kk[v] * P[i][v];
-        qhx += dq[v] * HX[i][v];
-      }
-    }
-    kl = q4_sum(kl);
-    kp = q4_sum(kp);
-    qhx = q4_sum(qhx);
-    if (q4 == 0) {
-      float* xo = xch + (fh * CB + s) * 4;
-      xo[0] = kl; xo[1] = kp; xo[2] = qhx;
-    }
+    if (s_ok) *reinterpret_cast<bf16x4*>(w.dk + ro + 16 * i) = bf4(y);
   }
-  // store this feature half of dk_s = DK + L + e^{Gam - g_s} P
-  if (s_ok) {
-    const int64_t dko = ((int64_t)(b.tok0 + s) * H + h) * D + 4 * q4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int nt = 4 * fh + i;
-      f32x4 y;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) y[v] = DK[i][v] + L[i][v] + ec * P[i][v];
-      if (w.dk_add) {
-        const f32x4 o0 = *reinterpret_cast<const f32x4*>(w.dk_add + dko + 16 * nt);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) y[v] += o0[v];
-      }
-      *reinterpret_cast<bf16x4*>(w.dk + dko + 16 * nt) = bf4(y);
-    }
+  kl = q4_sum(kl);
+  kp = q4_sum(kp);
+  qhx = q4_sum(qhx);
+  if (q4 == 0) {
+    float* xo = xch + (fh * CB + s) * 4;
+    xo[0] = kl; xo[1] = kp; xo[2] = qhx; xo[3] = rowdm;
   }
-  lds_barrier();       // the column sums, the feature halves' dot products, red[0..7]
+  lds_barrier();       // the column sums, the halves' dot products, red[0..7]
   // dL/dg_s (waves of the first feature half; the second has the same inputs)
   float dg = 0.f, phi = 0.f;
   if (fh == 0 && s_ok) {
@@ -1922,8 +1918,7 @@ __global__ __launch_bounds__(C_NTHR, 1) void cheb_dk_kernel(Params p, Bwd w) {
     kp = xo[1] + xp[1];
     qhx = xo[2] + xp[2];
     phi = 0.5f * ec * kp;
-    const float f = w.fro[(int64_t)(b.tok0 + s) * H + h];
-    dg = rowdm - fast_exp(gs) * qhx + SC(CS_A, s) * f * f - 0.5f * kl - phi;
+    dg = xo[3] + xp[3] - fast_exp(gs) * qhx + (SC(CS_A, s) + SC(CS_A1, s)) * fro * fro - 0.5f * kl - phi;
     dg -= SC(CS_COL0 + 0, s) + SC(CS_COL0 + 1, s) + SC(CS_COL0 + 2, s) + SC(CS_COL0 + 3, s);
   }
   // sum of phi over the block (for the last token)
@@ -1964,10 +1959,9 @@ struct GlaBwd {
   const bf16* q; const bf16* x; const bf16* v; const bf16* dout;   // [tokens][H][D]
   const void* alpha; int alpha_dt;        // [tokens][H]
   bf16* e; float* gam;                    // as Bwd
-  float* dx;                              // [tokens][H][D]: alpha du (the solve's dx)
-  // [tokens][H][D]: dq and dk in fp32 when the solve's backward adds to them
-  // (dq32, dk32), else in bf16 (dq_bf, dk_bf); dv in bf16
-  float* dq32; float* dk32; bf16* dq_bf; bf16* dk_bf; bf16* dv;
+  // [tokens][H][D]: with the solver du and this part of dk in fp32 (its backward forms
+  // dx = alpha du and adds to (1 - alpha) du and dk), else dq and dk in bf16; dv in bf16
+  float* du; float* dk32; bf16* dq_bf; bf16* dk_bf; bf16* dv;
   float* dalpha; float* dg;               // [tokens][H]
   float scale;
   int solve;                              // 0: num_iter == 0 (u = q, no x, alpha unused)
@@ -2065,16 +2059,25 @@ constexpr int GB_OFF_RED = GB_OFF_SC + NGS * CB * 4;       // 16 floats of cross
 constexpr int GB_OFF_MS = GB_OFF_RED + 16 * 4;             // 24 floats for block_max
 constexpr int GB_OFF_XCH = GB_OFF_MS + 24 * 4;             // [2][64][4] feature-half dot products
 constexpr int GB_SMEM = GB_OFF_XCH + 2 * CB * 4 * 4;
-static_assert(GB_SMEM <= 160 * 1024, "LDS budget");
+static_assert(GB_SMEM <= 160 * 1024 && 2 * CB * LDB * 2 <= SZ_H, "LDS budget");
 
-// du (-> dx, dq, dalpha), dk, dv, dg of block gb (see the section comment)
-__global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w) {
+// du (-> dalpha, dq), dk, dv, dg of block gb (see the section comment).
+// One workgroup per CU (150 KB of LDS): every load of the block is issued before the
+// first wait, q and x in the layout of du's tiles (so they are read once, for u and for
+// du's dot products).  The in-block matrices e^{G_t-G_s} (do_t.v_s) and e^{G_t-G_s}
+// (u_t.k_s) are formed once, a pair of tiles per wave, and shared through the LDS of
+// S_c (each wave formed its column of both, and the first one's transpose too).  With
+// the solver du leaves in fp32 once: the solve forms alpha du, its right-hand side, and
+// (1 - alpha) du, the blend's share of dq, from it.
+__global__ __launch_bounds__(GB_NTHR, 2) void gla_bwd_kernel(Params p, GlaBwd w) {
   __shared__ __align__(16) unsigned char smem[GB_SMEM];
   f16* sK = reinterpret_cast<f16*>(smem + GB_OFF_K);
   f16* sV = reinterpret_cast<f16*>(smem + GB_OFF_V);
   f16* sDo = reinterpret_cast<f16*>(smem + GB_OFF_DO);
   f16* sU = reinterpret_cast<f16*>(smem + GB_OFF_U);
   f16* sS = reinterpret_cast<f16*>(smem + GB_OFF_S);      // S_c^T: rows V, columns K
+  f16* sPt = sS;                                           // then do.v: rows t, columns s
+  f16* sUt = sS + CB * LDB;                                // and u.k
   f16* sDS = reinterpret_cast<f16*>(smem + GB_OFF_DS);    // dSn: rows K, columns V
   float* sc = reinterpret_cast<float*>(smem + GB_OFF_SC);
   float* red = reinterpret_cast<float*>(smem + GB_OFF_RED);
@@ -2091,52 +2094,60 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
   const int64_t DD = (int64_t)D * D;
   constexpr int NP = CB * 16 / GB_NTHR;    // staging passes of 32 rows
 
-  // S_c (as the solve forms it: zero-start block state + decayed segment start)
-  if (tid < NTHR) {
-    const int64_t so = ((int64_t)b.s_id * H + h) * DD;
-    const int64_t bso = ((int64_t)gb * H + h) * DD;
-    StateLd sst;
-    solve::state_issue_b<false>(sst, b.lb > 0 ? p.ws_sb + bso : nullptr, tid);
-    const float off_g = p.ws_boff[((int64_t)gb * H + h) * 2 + 1];
-    solve::state_issue_s<false>(sst, (b.lb == 0 || off_g > solve::SEG_STATE_DROP) ? p.ws_s0 + so : nullptr, tid);
-    solve::state_store<false>(sS, sst, fast_exp(off_g), tid);
-  }
-  if (wave == 0) {
-    const bool ok = lane < b.nval;
-    SC(GS_G, lane) = scan64(ok ? ldsc(p.g, (int64_t)(b.tok0 + lane) * H + h, p.g_dt) : 0.f);
-  }
-  lds_barrier();
-  // rows k, v (fp16 as given), do and u (scaled); dSn (scaled) and <dSn, S_c>
+  const int s = 16 * cg + l16;            // this lane's token / key column
+  const bool s_ok = s < b.nval;
+  const int64_t ti = (int64_t)(b.tok0 + s) * H + h;
+  const int64_t ro = ti * D + 64 * fh + 4 * q4;   // + 16 i: features 64 fh + 16 i + 4 q4 .. +3
+
+  // ---- loads ---------------------------------------------------------------------
+  const int64_t so = ((int64_t)b.s_id * H + h) * DD;
+  const int64_t bso = ((int64_t)gb * H + h) * DD;
+  StateLd<GB_NTHR> sst;
+  solve::state_issue_b<false>(sst, b.lb > 0 ? p.ws_sb + bso : nullptr, tid);
+  const float off_g = p.ws_boff[((int64_t)gb * H + h) * 2 + 1];
+  // dSn: wave w's tile row w, column j (rows K = 16 w + l16, columns V = 16 j + 4 q4 ..)
+  bf16x4 dsn[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    dsn[j] = *reinterpret_cast<const bf16x4*>(w.e + bso + blk_index(16 * wave + l16, 16 * j + 4 * q4));
   bf16x8 kr[NP], vr[NP], dr[NP];
-  f32x4 u0[NP], u1[NP];
-  const bf16* dn = w.e + ((int64_t)gb * H + h) * DD;
-  const int drw = tid >> 2, dc0 = (tid & 3) * 32;    // this thread's dSn: row drw, columns dc0..+31
-  f32x4 dsv[8];
-  float mx[3] = {0.f, 0.f, 0.f};          // max |do|, |u|, |dSn|
 #pragma unroll
   for (int pass = 0; pass < NP; ++pass) {
     const int row = pass * 32 + (tid >> 4), f0 = (tid & 15) * 8;
     const bool ok = row < b.nval;
-    const int64_t ti = (int64_t)(b.tok0 + row) * H + h, ro = ti * D + f0;
+    const int64_t rr = ((int64_t)(b.tok0 + row) * H + h) * D + f0;
     kr[pass] = ok ? *reinterpret_cast<const bf16x8*>(p.k + (int64_t)(b.tok0 + row) * p.kv_ts + h * D + f0) : bf16x8{};
-    vr[pass] = ok ? *reinterpret_cast<const bf16x8*>(w.v + ro) : bf16x8{};
-    dr[pass] = ok ? *reinterpret_cast<const bf16x8*>(w.dout + ro) : bf16x8{};
-    const bf16x8 qr = ok ? *reinterpret_cast<const bf16x8*>(w.q + ro) : bf16x8{};
-    const bf16x8 xr = (ok && w.solve) ? *reinterpret_cast<const bf16x8*>(w.x + ro) : bf16x8{};
-    const float al = ok ? gla_alpha(w, ti) : 0.f;
+    vr[pass] = ok ? *reinterpret_cast<const bf16x8*>(w.v + rr) : bf16x8{};
+    dr[pass] = ok ? *reinterpret_cast<const bf16x8*>(w.dout + rr) : bf16x8{};
+  }
+  bf16x4 qv[4], xv[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    qv[i] = s_ok ? *reinterpret_cast<const bf16x4*>(w.q + ro + 16 * i) : bf16x4{};
+    xv[i] = (s_ok && w.solve) ? *reinterpret_cast<const bf16x4*>(w.x + ro + 16 * i) : bf16x4{};
+  }
+  const float al = s_ok ? gla_alpha(w, ti) : 0.f;
+  const float g_l = (wave == 0 && lane < b.nval) ? ldsc(p.g, (int64_t)(b.tok0 + lane) * H + h, p.g_dt) : 0.f;
+  solve::state_issue_s<false>(sst, (b.lb == 0 || off_g > solve::SEG_STATE_DROP) ? p.ws_s0 + so : nullptr, tid);
+
+  // ---- staging: k, v (fp16 as given), do, u and dSn (scaled), S_c as the solve forms it
+  if (wave == 0) SC(GS_G, lane) = scan64(g_l);
+  f32x4 u[4];
+  float mx[3] = {0.f, 0.f, 0.f};          // max |do|, |u|, |dSn|
+#pragma unroll
+  for (int pass = 0; pass < NP; ++pass) mx[0] = fmaxf(mx[0], absmax8(dr[pass]));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      u0[pass][v] = (float)qr[v] + al * ((float)xr[v] - (float)qr[v]);
-      u1[pass][v] = (float)qr[4 + v] + al * ((float)xr[4 + v] - (float)qr[4 + v]);
+      const float qf = (float)qv[i][v];
+      u[i][v] = qf + al * ((float)xv[i][v] - qf);
     }
-    mx[0] = fmaxf(mx[0], absmax8(dr[pass]));
-    mx[1] = fmaxf(mx[1], fmaxf(absmax4(u0[pass]), absmax4(u1[pass])));
+    mx[1] = fmaxf(mx[1], absmax4(u[i]));
   }
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    dsv[j] = f4(*reinterpret_cast<const bf16x4*>(dn + blk_index(drw, dc0 + 4 * j)));
-    mx[2] = fmaxf(mx[2], absmax4(dsv[j]));
-  }
+  for (int j = 0; j < 8; ++j) mx[2] = fmaxf(mx[2], absmax4(f4(dsn[j])));
+  solve::state_store<false>(sS, sst, fast_exp(off_g), tid);
   block_max<3, GB_NTHR / 64>(mx, mslot, wave, lane);
   const float sdo = pow2_scale(mx[0]), su = pow2_scale(mx[1]), sds = pow2_scale(mx[2]);
 #pragma unroll
@@ -2145,100 +2156,100 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
     store8_i(sK + row * LDP, f0, scale_h8(kr[pass], 1.f));
     store8_i(sV + row * LDP, f0, scale_h8(vr[pass], 1.f));
     store8_i(sDo + row * LDP, f0, scale_h8(dr[pass], sdo));
-    store8_i(sU + row * LDP, f0, h8_of(u0[pass], u1[pass], su));
   }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<f16x4*>(sU + s * LDP + icol(64 * fh + 16 * i + 4 * q4)) = h4(u[i] * su);
   float dss = 0.f;                        // <dSn, S_c> over this thread's elements
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
+    const f32x4 d = f4(dsn[j]);
+    const f16x4 sv = ld_tr_i(sS, LDP, 16 * j + 4 * q4, 16 * wave, lane);   // S_c^T[V][K], V = 16 j + 4 q4 ..
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int c = dc0 + 4 * j + v;      // V index; S_c^T[c][drw] in sS
-      dss += dsv[j][v] * (float)sS[c * LDP + icol(drw)];
-    }
+    for (int v = 0; v < 4; ++v) dss += d[v] * (float)sv[v];
+    *reinterpret_cast<f16x4*>(sDS + (16 * wave + l16) * LDP + icol(16 * j + 4 * q4)) = h4(d * sds);
   }
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    store8_i(sDS + drw * LDP, dc0 + 8 * j, h8_of(dsv[2 * j], dsv[2 * j + 1], sds));
   dss = wave_sum_v(dss);
   if (lane == 0) red[wave] = dss;
   lds_barrier();
 
-  const int s = 16 * cg + l16;            // this lane's token / key column
-  const bool s_ok = s < b.nval;
   const float Gs = SC(GS_G, s), Gam = SC(GS_G, b.nval - 1);
   const float ec = fast_exp(Gam - Gs), egs = fast_exp(Gs);
-  const int64_t ti = (int64_t)(b.tok0 + s) * H + h;
-  const int64_t ro = ti * D + 4 * q4;     // + 16 nt: features 16 nt + 4 q4 .. +3
   float* xo = xch + (fh * CB + s) * 4;    // this half's dot products of column s
 
-  // ---- du (rows f = K of this half, column t = s) ---------------------------
+  // ---- S_c do_t (rows f = K of this half, column t = s): A = S_c rows over V, read
+  // transposed from S_c^T; and the wave's two tiles (rows j, column t) of
+  // P[j][t] = e^{G_t-G_j} (do_t.v_j) and U[j][t] = e^{G_t-G_j} (u_t.k_j), j <= t ------
+  f32x4 DQ[4];
+  f16x4 pt[2], ut[2];
   {
-    f32x4 DQ[4], DI[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      DQ[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      DI[i] = DQ[i];
-    }
-    // S_c do_t: A = S_c rows (K) over V, read transposed from S_c^T
+    for (int i = 0; i < 4; ++i) DQ[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 P[2], U[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) P[j] = U[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const f16x8 bd = frag_i(sDo, LDP, 16 * cg, 32 * ks, lane);
+      const f16x8 bu = frag_i(sU, LDP, 16 * cg, 32 * ks, lane);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         DQ[i] = mfma16h(frag_t_i(sS, LDP, 32 * ks, 16 * (4 * fh + i), lane), bd, DQ[i]);
-    }
-    // P[j][t] = e^{G_t-G_j} (do_t.v_j), j <= t: rows j over the block, column t
-    f16x8 pb[2];
-    {
-      f32x4 P[4];
 #pragma unroll
-      for (int jt = 0; jt < 4; ++jt) P[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const f16x8 bd = frag_i(sDo, LDP, 16 * cg, 32 * ks, lane);
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) P[jt] = mfma16h(frag_i(sV, LDP, 16 * jt, 32 * ks, lane), bd, P[jt]);
+      for (int j = 0; j < 2; ++j) {
+        P[j] = mfma16h(frag_i(sV, LDP, 16 * (2 * fh + j), 32 * ks, lane), bd, P[j]);
+        U[j] = mfma16h(frag_i(sK, LDP, 16 * (2 * fh + j), 32 * ks, lane), bu, U[j]);
       }
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt) {
-        const f32x4 gj = *reinterpret_cast<const f32x4*>(&SC(GS_G, 16 * jt + 4 * q4));
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int j = 16 * jt + 4 * q4 + v;
-          P[jt][v] = (j <= s && j < b.nval) ? P[jt][v] * fast_exp(Gs - gj[v]) : 0.f;
-        }
-      }
-      pb[0] = h8(P[0], P[1]);
-      pb[1] = h8(P[2], P[3]);
     }
 #pragma unroll
-    for (int jk = 0; jk < 2; ++jk)
+    for (int j = 0; j < 2; ++j) {
+      const int j0 = 16 * (2 * fh + j) + 4 * q4;
+      const f32x4 gj = *reinterpret_cast<const f32x4*>(&SC(GS_G, j0));
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float e = (j0 + v <= s && j0 + v < b.nval) ? fast_exp(Gs - gj[v]) : 0.f;
+        pt[j][v] = (f16)(P[j][v] * e);
+        ut[j][v] = (f16)(U[j][v] * e);
+      }
+    }
+  }
+  lds_barrier();                          // every wave is done with S_c
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int o = s * LDB + icol(16 * (2 * fh + j) + 4 * q4);
+    *reinterpret_cast<f16x4*>(sPt + o) = pt[j];
+    *reinterpret_cast<f16x4*>(sUt + o) = ut[j];
+  }
+  lds_barrier();
+
+  // ---- du = scale (e^{G_t} S_c do_t + sum_j P[j][t] k_j) / sdo ------------------------
+  {
+    f32x4 DI[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) DI[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int jk = 0; jk < 2; ++jk) {
+      if (2 * jk > cg) break;             // the keys past every token of this column group
+      const f16x8 pb = frag_i(sPt, LDB, 16 * cg, 32 * jk, lane);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        DI[i] = mfma16h(frag_t_i(sK, LDP, 32 * jk, 16 * (4 * fh + i), lane), pb[jk], DI[i]);
-    // du = scale (e^{G_t} DQ + DI) / sdo; dx, dq, dalpha and u.du over this half
+        DI[i] = mfma16h(frag_t_i(sK, LDP, 32 * jk, 16 * (4 * fh + i), lane), pb, DI[i]);
+    }
     const float cu = w.scale / sdo;
-    const float al = s_ok ? gla_alpha(w, ti) : 0.f;
     float dal = 0.f, udu = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int nt = 4 * fh + i;
-      const bf16x4 qv = s_ok ? *reinterpret_cast<const bf16x4*>(w.q + ro + 16 * nt) : bf16x4{};
-      const bf16x4 xv = (s_ok && w.solve) ? *reinterpret_cast<const bf16x4*>(w.x + ro + 16 * nt) : bf16x4{};
-      f32x4 du, dqo, dxo;
+      f32x4 du;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         du[v] = cu * (egs * DQ[i][v] + DI[i][v]);
-        const float qf = (float)qv[v], xf = (float)xv[v];
+        const float qf = (float)qv[i][v], xf = (float)xv[i][v];
         dal += du[v] * (xf - qf);
         udu += du[v] * (qf + al * (xf - qf));
-        dqo[v] = (1.f - al) * du[v];
-        dxo[v] = al * du[v];
       }
       if (s_ok) {
-        if (w.dq32) *reinterpret_cast<f32x4*>(w.dq32 + ro + 16 * nt) = dqo;
-        else *reinterpret_cast<bf16x4*>(w.dq_bf + ro + 16 * nt) = bf4(dqo);
-        if (w.solve) *reinterpret_cast<f32x4*>(w.dx + ro + 16 * nt) = dxo;
+        if (w.solve) *reinterpret_cast<f32x4*>(w.du + ro + 16 * i) = du;
+        else *reinterpret_cast<bf16x4*>(w.dq_bf + ro + 16 * i) = bf4(du);
       }
     }
     dal = q4_sum(dal);
@@ -2256,35 +2267,14 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
       DK[i] = f32x4{0.f, 0.f, 0.f, 0.f};
       DX[i] = DK[i];
     }
-    // R[t][s] = e^{G_t-G_s} (do_t.v_s), t >= s
-    f16x8 rb[2];
-    {
-      f32x4 R[4];
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) R[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const f16x8 bv = frag_i(sV, LDP, 16 * cg, 32 * ks, lane);
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) R[tt] = mfma16h(frag_i(sDo, LDP, 16 * tt, 32 * ks, lane), bv, R[tt]);
-      }
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) {
-        const f32x4 gt = *reinterpret_cast<const f32x4*>(&SC(GS_G, 16 * tt + 4 * q4));
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int t = 16 * tt + 4 * q4 + v;
-          R[tt][v] = (t >= s && t < b.nval) ? R[tt][v] * fast_exp(gt[v] - Gs) : 0.f;
-        }
-      }
-      rb[0] = h8(R[0], R[1]);
-      rb[1] = h8(R[2], R[3]);
-    }
-#pragma unroll
-    for (int jk = 0; jk < 2; ++jk)
+    for (int jk = 0; jk < 2; ++jk) {
+      if (jk == 0 && cg >= 2) continue;   // the tokens before every key of this column group
+      const f16x8 rb = frag_t_i(sPt, LDB, 32 * jk, 16 * cg, lane);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        DK[i] = mfma16h(frag_t_i(sU, LDP, 32 * jk, 16 * (4 * fh + i), lane), rb[jk], DK[i]);
+        DK[i] = mfma16h(frag_t_i(sU, LDP, 32 * jk, 16 * (4 * fh + i), lane), rb, DK[i]);
+    }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const f16x8 bv = frag_i(sV, LDP, 16 * cg, 32 * ks, lane);
@@ -2296,8 +2286,7 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
     float kdk = 0.f, kdkx = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int nt = 4 * fh + i;
-      const f16x4 kk = *reinterpret_cast<const f16x4*>(sK + s * LDP + icol(16 * nt + 4 * q4));
+      const f16x4 kk = *reinterpret_cast<const f16x4*>(sK + s * LDP + icol(64 * fh + 16 * i + 4 * q4));
       f32x4 y;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -2307,8 +2296,8 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
         kdkx += (float)kk[v] * xpart;
       }
       if (s_ok) {
-        if (w.dk32) *reinterpret_cast<f32x4*>(w.dk32 + ro + 16 * nt) = y;
-        else *reinterpret_cast<bf16x4*>(w.dk_bf + ro + 16 * nt) = bf4(y);
+        if (w.dk32) *reinterpret_cast<f32x4*>(w.dk32 + ro + 16 * i) = y;
+        else *reinterpret_cast<bf16x4*>(w.dk_bf + ro + 16 * i) = bf4(y);
       }
     }
     kdk = q4_sum(kdk);
@@ -2326,35 +2315,14 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
       DV[i] = f32x4{0.f, 0.f, 0.f, 0.f};
       DX[i] = DV[i];
     }
-    // U[t][s] = e^{G_t-G_s} (u_t.k_s), t >= s
-    f16x8 ub[2];
-    {
-      f32x4 U[4];
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) U[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const f16x8 bk = frag_i(sK, LDP, 16 * cg, 32 * ks, lane);
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) U[tt] = mfma16h(frag_i(sU, LDP, 16 * tt, 32 * ks, lane), bk, U[tt]);
-      }
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) {
-        const f32x4 gt = *reinterpret_cast<const f32x4*>(&SC(GS_G, 16 * tt + 4 * q4));
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int t = 16 * tt + 4 * q4 + v;
-          U[tt][v] = (t >= s && t < b.nval) ? U[tt][v] * fast_exp(gt[v] - Gs) : 0.f;
-        }
-      }
-      ub[0] = h8(U[0], U[1]);
-      ub[1] = h8(U[2], U[3]);
-    }
-#pragma unroll
-    for (int jk = 0; jk < 2; ++jk)
+    for (int jk = 0; jk < 2; ++jk) {
+      if (jk == 0 && cg >= 2) continue;
+      const f16x8 ub = frag_t_i(sUt, LDB, 32 * jk, 16 * cg, lane);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        DV[i] = mfma16h(frag_t_i(sDo, LDP, 32 * jk, 16 * (4 * fh + i), lane), ub[jk], DV[i]);
+        DV[i] = mfma16h(frag_t_i(sDo, LDP, 32 * jk, 16 * (4 * fh + i), lane), ub, DV[i]);
+    }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const f16x8 bk = frag_i(sK, LDP, 16 * cg, 32 * ks, lane);
@@ -2369,7 +2337,7 @@ __global__ __launch_bounds__(GB_NTHR, 1) void gla_bwd_kernel(Params p, GlaBwd w)
         f32x4 y;
 #pragma unroll
         for (int v = 0; v < 4; ++v) y[v] = ci * DV[i][v] + cx * DX[i][v];
-        *reinterpret_cast<bf16x4*>(w.dv + ro + 16 * (4 * fh + i)) = bf4(y);
+        *reinterpret_cast<bf16x4*>(w.dv + ro + 16 * i) = bf4(y);
       }
     }
   }
@@ -2524,7 +2492,7 @@ extern "C" int hmx_gka_cheb_bwd(const void* k, int64_t k_token_stride, const voi
   w.dq = dq32; w.fro = fro;
   w.e = reinterpret_cast<bf16*>(bw);
   w.gam = reinterpret_cast<float*>(bw + e_bytes);
-  w.dk = static_cast<bf16*>(dk); w.dq_out = static_cast<bf16*>(dq);
+  w.dk = static_cast<bf16*>(dk); p.dq_out = static_cast<bf16*>(dq);
   w.dgk = gk ? dgk : nullptr;
   w.bp_lambda = bp_lambda;
   hipStream_t s = (hipStream_t)stream;
@@ -2602,12 +2570,12 @@ extern "C" int hmx_gka_train_fwd(const void* q, const void* k, const void* v, in
   return check_launch("hmx_gka_train_fwd");
 }
 
-// backward workspace: the solve's backward workspace (with its dq), then dx, the
-// GLA's dq and dk (fp32)
+// backward workspace: the solve's backward workspace (with its dq), then du and the
+// GLA's dk (fp32)
 extern "C" size_t hmx_gka_train_bwd_workspace_bytes(int32_t nblock_total, int32_t H,
                                                     int64_t tokens) {
   return hmx_gka_cheb_bwd_workspace_bytes(nblock_total, H, tokens) +
-         3 * al256((size_t)tokens * H * D * sizeof(float));
+         2 * al256((size_t)tokens * H * D * sizeof(float));
 }
 
 extern "C" int hmx_gka_train_bwd(const void* q, const void* k, const void* v, int32_t dtype,
@@ -2649,12 +2617,11 @@ extern "C" int hmx_gka_train_bwd(const void* q, const void* k, const void* v, in
   gw.alpha = alpha; gw.alpha_dt = alpha_dtype;
   gw.e = reinterpret_cast<bf16*>(bw);
   gw.gam = reinterpret_cast<float*>(bw + e_bytes);
-  gw.dx = reinterpret_cast<float*>(bw + cb_bytes);
   float* dq_cheb = reinterpret_cast<float*>(bw + e_bytes + al256((size_t)nblock_total * H * sizeof(float)));
-  float* dq_gla = reinterpret_cast<float*>(bw + cb_bytes + tok_bytes);
-  float* dk_gla = reinterpret_cast<float*>(bw + cb_bytes + 2 * tok_bytes);
+  float* du = reinterpret_cast<float*>(bw + cb_bytes);
+  float* dk_gla = reinterpret_cast<float*>(bw + cb_bytes + tok_bytes);
   if (solve_) {           // the solve's backward adds its dq and dk, then writes bf16
-    gw.dq32 = dq_gla; gw.dk32 = dk_gla;
+    gw.du = du; gw.dk32 = dk_gla;
   } else {
     gw.dq_bf = static_cast<bf16*>(dq); gw.dk_bf = static_cast<bf16*>(dk);
   }
@@ -2670,12 +2637,11 @@ extern "C" int hmx_gka_train_bwd(const void* q, const void* k, const void* v, in
   if (solve_) {
     // the solve's backward on dx = alpha du: its dq is added to dq, its dk to dk
     Params pc = p;
-    pc.rhs32 = gw.dx;
+    pc.du32 = du; pc.dq_out = static_cast<bf16*>(dq);
     pc.fro = const_cast<float*>(fro);
-    pc.xo32 = dq_cheb; pc.xo32_acc = 0;
+    pc.xo32 = dq_cheb;
     cw.x = gw.x; cw.dq = dq_cheb; cw.fro = fro;
     cw.dk = static_cast<bf16*>(dk); cw.dk_add = dk_gla;
-    cw.dq_out = static_cast<bf16*>(dq); cw.dq_add = dq_gla;
     cw.dgk = gk ? dgk : nullptr;
     cw.bp_lambda = bp_lambda;
     hipLaunchKernelGGL((solve::gka_solve_kernel<true, false, solve::SM_DQ>), grid, dim3(NTHR), 0, s, pc);
