@@ -113,6 +113,9 @@ struct Params {
   // SM_DQ under the alpha blend: the fp32 gradient du of the blended query; the
   // right-hand side is then alpha du (in place of p.q) and dq_out gains (1 - alpha) du
   const float* du32;
+  // SM_DQ: the saved solution x, and the block's share E_c of the state gradient
+  // [nblk][H][D][D] (bf16, tile-major) with its log decay [nblk][H]
+  const bf16* xsol; bf16* eout; float* gam; int bp_lambda;
 };
 
 // The fused gates' raw projection values as bits (one load in either dtype
@@ -544,6 +547,110 @@ __global__ __launch_bounds__(256) void gka_combine_kernel(Params p, int track_h)
   }
 }
 
+// ---- helpers of the training kernels, the solve's backward mode included -------------
+namespace train {
+// x, dq and the ridge weights grow like 1 / |H_t|_F, which is small at a
+// sequence's start: the fp16 operands built from them are scaled by a power of two
+// (exact) chosen from their largest magnitude, and the products unscaled in fp32.
+// pow2_scale(m): 2^j with m 2^j < 2^8 (1 when m is below that already)
+__device__ __forceinline__ float pow2_scale(float m) {
+  int e;
+  (void)frexpf(m, &e);                   // m < 2^e
+  return e > 8 ? ldexpf(1.f, 8 - e) : 1.f;
+}
+__device__ __forceinline__ float wave_max(float x) {
+  x = fmaxf(x, dppf<0xB1>(x));
+  x = fmaxf(x, dppf<0x4E>(x));
+  x = fmaxf(x, dppf<0x141>(x));
+  x = fmaxf(x, dppf<0x140>(x));
+  const unsigned u = __builtin_bit_cast(unsigned, x);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  x = fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+  const unsigned w = __builtin_bit_cast(unsigned, x);
+  const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)q[0]), __builtin_bit_cast(float, (unsigned)q[1]));
+}
+// Suffix sums over the 64 lanes of a wave (lane l: lanes l..63), within each row of 16
+// by lane shifts, then the later rows' totals.
+template <int N>
+__device__ __forceinline__ float shl_row(float v) {   // lane l of a row receives lane l + N (0 past it)
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + N,
+                                                               0xF, 0xF, true));
+}
+__device__ __forceinline__ float lane_val(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+__device__ __forceinline__ float suffix_sum64(float x, int lane) {
+  x += shl_row<1>(x);
+  x += shl_row<2>(x);
+  x += shl_row<4>(x);
+  x += shl_row<8>(x);
+  const float r3 = lane_val(x, 48), r2 = lane_val(x, 32) + r3, r1 = lane_val(x, 16) + r2;
+  return x + (lane < 16 ? r1 : lane < 32 ? r2 : lane < 48 ? r3 : 0.f);
+}
+// rho_t = sum_{t' >= t} a_t' e^{2 (g_t' - g_t)} over the 64 lanes t (a_t, g_t in lane t):
+// rho over 2n lanes = rho over n + e^{2 (g_{t+n} - g_t)} (rho over n of lane t + n).
+// One wave forms it while the workgroup waits: as a loop over the later tokens (an LDS
+// read and an exponential each, up to 64) it cost, together with the loops of the
+// gates' suffix sums, a binary search for each block's segment and lane sums through
+// the LDS, 0.67 of training's 7.25 ms at 8 x 4096 tokens, H = 32.
+__device__ __forceinline__ float decayed_suffix(float a, float g, int lane) {
+  const int l16 = lane & 15;
+  float r = a;
+  auto step = [&](float r_n, float g_n, int n) {
+    if (l16 + n < 16) r += fast_exp(2.f * (g_n - g)) * r_n;
+  };
+  step(shl_row<1>(r), shl_row<1>(g), 1);
+  step(shl_row<2>(r), shl_row<2>(g), 2);
+  step(shl_row<4>(r), shl_row<4>(g), 4);
+  step(shl_row<8>(r), shl_row<8>(g), 8);
+  // the later rows: their sums from lanes 16, 32 and 48, the last first
+  const float g1 = lane_val(g, 16), g2 = lane_val(g, 32), g3 = lane_val(g, 48);
+  const float r3 = lane_val(r, 48);
+  const float r2 = lane_val(r, 32) + fast_exp(2.f * (g3 - g2)) * r3;
+  const float r1 = lane_val(r, 16) + fast_exp(2.f * (g2 - g1)) * r2;
+  const float rn = lane < 16 ? r1 : lane < 32 ? r2 : r3, gn = lane < 16 ? g1 : lane < 32 ? g2 : g3;
+  return lane < 48 ? r + fast_exp(2.f * (gn - g)) * rn : r;
+}
+__device__ __forceinline__ float absmax8(const bf16x8& x) {
+  float m = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf((float)x[j]));
+  return m;
+}
+__device__ __forceinline__ float absmax4(const f32x4& x) {
+  return fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+}
+// The workgroup's maxima of NV per-thread values over NW waves: slot[NV * NW] of
+// LDS scratch; includes a barrier.
+template <int NV, int NW = 4>
+__device__ __forceinline__ void block_max(float (&v)[NV], float* slot, int wave, int lane) {
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    v[i] = wave_max(v[i]);
+    if (lane == 0) slot[NW * i + wave] = v[i];
+  }
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float m = slot[NW * i];
+#pragma unroll
+    for (int j = 1; j < NW; ++j) m = fmaxf(m, slot[NW * i + j]);
+    v[i] = m;
+  }
+}
+__device__ __forceinline__ bf16x4 bf4(const f32x4& x) {
+  return bf16x4{(bf16)x[0], (bf16)x[1], (bf16)x[2], (bf16)x[3]};
+}
+__device__ __forceinline__ f32x4 f4(const bf16x4& x) {
+  return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+}
+__device__ __forceinline__ f16x8 h8_of(const f32x4& a, const f32x4& b, float s) {
+  return f16x8{(f16)(s * a[0]), (f16)(s * a[1]), (f16)(s * a[2]), (f16)(s * a[3]),
+               (f16)(s * b[0]), (f16)(s * b[1]), (f16)(s * b[2]), (f16)(s * b[3])};
+}
+}  // namespace train
+
 // ===========================================================================
 // Pass B: the parallel solve and GLA output
 // ===========================================================================
@@ -690,7 +797,8 @@ __device__ __forceinline__ void with_wave(int wave, F&& f) {
 // What the solve kernel produces: the GLA output (serving prefill), or the solution
 // x of the Chebyshev solve itself (training): SM_X writes x (bf16, into p.o) and
 // |H_t|_F; SM_DQ solves for the right-hand side in p.q with the |H_t|_F of the
-// forward read back (the backward's dq) and writes fp32 (p.xo32); SM_GLA_SAVE is
+// forward read back (the backward's dq), writes fp32 (p.xo32) and bf16 (p.dq_out) and
+// forms the block's share of the state gradient (p.eout); SM_GLA_SAVE is
 // the GLA output that also saves x (p.xs) and |H_t|_F for the training backward.
 enum SolveMode { SM_GLA = 0, SM_X = 1, SM_DQ = 2, SM_GLA_SAVE = 3 };
 
@@ -1051,6 +1159,133 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
           }
         }
       }
+      if constexpr (MODE == SM_DQ) {
+      // ---- E_c = -(Ql^T X + X^T Ql) + 2 (alpha h_c + K^T diag(beta) K), Ql = e^{g} dq: the
+      // block's share of dL/dh_c (see the training section), while dq, h_c and k are on
+      // chip: as a launch of its own (0.77 ms at 8 x 4096 tokens, H = 32, one workgroup per
+      // CU) it read them back, 1.7 of its 2.2 GB; here the solve takes 1.04 -> 1.38 ms, the
+      // training step 6.19 -> 5.76.  2 beta k, then dq, take v's LDS and x takes h_c's.
+      // The saved x in dq's layout (this lane's token) -------------------------------------
+      using train::bf4; using train::f4; using train::absmax4; using train::pow2_scale;
+      const int64_t ro = ((int64_t)(tok0 + tb) * H + h) * D + 4 * q4;
+      bf16x4 xr[8];
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt)
+        xr[nt] = tok_ok ? *reinterpret_cast<const bf16x4*>(p.xsol + ro + 16 * nt) : bf16x4{};
+      float mx[3] = {0.f, 0.f, 0.f};      // max |x|, |e^g dq|, |2 beta k|
+      {
+        // a_t = -r (dq_t . x_t) / |H_t|_F (0 without bp_lambda)
+        float qx = 0.f;
+        const float eg = tok_ok ? -fast_exp(GkT) : 0.f;
+#pragma unroll
+        for (int nt = 0; nt < 8; ++nt) {
+          const f32x4 xf = f4(xr[nt]);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) qx += X[nt][v] * xf[v];
+          X[nt] *= eg;
+          mx[0] = fmaxf(mx[0], absmax4(xf));
+          mx[1] = fmaxf(mx[1], absmax4(X[nt]));
+        }
+        qx = q4_sum(qx);
+        const float f = (tok_ok && p.bp_lambda) ? p.fro[(int64_t)(tok0 + tb) * H + h] : 0.f;
+        if (q4 == 0) SC(SC_D, tb) = f > 0.f ? -p.ridge_ratio * qx / f : 0.f;
+      }
+      lds_barrier();                      // a_t; every wave is done iterating
+      if (wave == 0) {
+        // rho_t = sum_{t'>=t} a_t' e^{2(g_t'-g_t)}; 2 beta_t = 2 e^{g_t} rho_t; alpha = rho_0 e^{2 g_0}
+        const float gt = SC(SC_GK, lane);
+        const float rho = train::decayed_suffix(SC(SC_D, lane), gt, lane);
+        SC(SC_G2, lane) = lane < nval ? 2.f * fast_exp(gt) * rho : 0.f;
+        if (lane == 0) SC(SC_AL, 0) = fast_exp(2.f * gt) * rho;
+        if (lane == nval - 1) p.gam[(int64_t)gb * H + h] = gt;
+      }
+      lds_barrier();
+      const float b2 = SC(SC_G2, tb), a2 = 2.f * SC(SC_AL, 0);
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt) {
+        const f16x4 kk = *reinterpret_cast<const f16x4*>(sK + tb * LDP + icol(16 * nt + 4 * q4));
+        mx[2] = fmaxf(mx[2], fabsf(b2) * absmax4(f32x4{(float)kk[0], (float)kk[1], (float)kk[2], (float)kk[3]}));
+      }
+      train::block_max<3, 4>(mx, &SC(SC_HN, 0), wave, lane);
+      const float sx = pow2_scale(mx[0]), sq = pow2_scale(mx[1]), sb = pow2_scale(mx[2]);
+      const float u12 = 1.f / (sx * sq), u3 = 1.f / sb;
+      const auto put = [&](f16* base, int nt, f16x4 y) {
+        *reinterpret_cast<f16x4*>(base + tb * LDP + icol(16 * nt + 4 * q4)) = y;
+      };
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt) {
+        const f16x4 kk = *reinterpret_cast<const f16x4*>(sK + tb * LDP + icol(16 * nt + 4 * q4));
+        const float m = sb * b2;
+        put(sV, nt, f16x4{(f16)((float)kk[0] * m), (f16)((float)kk[1] * m), (f16)((float)kk[2] * m),
+                          (f16)((float)kk[3] * m)});
+      }
+      lds_barrier();
+      // wave w: tile rows 2w, 2w + 1 (state rows), all 8 tile columns.  First K^T (2 beta K)
+      // and h_c, rescaled (by powers of two) to the units of the products that follow.
+      f32x4 E[2][8];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int jt = 0; jt < 8; ++jt) E[i][jt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int jk = 0; jk < 2; ++jk) {
+        f16x8 ab[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) ab[i] = frag_t_i(sV, LDP, 32 * jk, 16 * (2 * wave + i), lane);
+#pragma unroll
+        for (int jt = 0; jt < 8; ++jt) {
+          const f16x8 bk = frag_t_i(sK, LDP, 32 * jk, 16 * jt, lane);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) E[i][jt] = mfma16h(ab[i], bk, E[i][jt]);
+        }
+      }
+      const float c3 = u3 * (sx * sq), ch = a2 * (sx * sq);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int jt = 0; jt < 8; ++jt) {
+          // E[i][jt][v] is element (16 (2w + i) + 4 q4 + v, 16 jt + l16); E_c is symmetric
+          const f16x4 hc = *reinterpret_cast<const f16x4*>(sH + (16 * jt + l16) * LDP +
+                                                           icol(16 * (2 * wave + i) + 4 * q4));
+#pragma unroll
+          for (int v = 0; v < 4; ++v) E[i][jt][v] = c3 * E[i][jt][v] + ch * (float)hc[v];
+        }
+      lds_barrier();                      // h_c and 2 beta k are read
+      f16* sXs = sH;
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt) {
+        put(sV, nt, h4(X[nt] * sq));
+        put(sXs, nt, h4(f4(xr[nt]) * sx));
+      }
+      lds_barrier();
+#pragma unroll
+      for (int jk = 0; jk < 2; ++jk) {
+        f16x8 aq[2], ax[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          aq[i] = frag_t_i(sV, LDP, 32 * jk, 16 * (2 * wave + i), lane);
+          ax[i] = frag_t_i(sXs, LDP, 32 * jk, 16 * (2 * wave + i), lane);
+        }
+#pragma unroll
+        for (int jt = 0; jt < 8; ++jt) {
+          const f16x8 bx = frag_t_i(sXs, LDP, 32 * jk, 16 * jt, lane);
+          const f16x8 bq = frag_t_i(sV, LDP, 32 * jk, 16 * jt, lane);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            E[i][jt] = mfma16h(aq[i], bx, E[i][jt]);
+            E[i][jt] = mfma16h(ax[i], bq, E[i][jt]);
+          }
+        }
+      }
+      // the lane writes row 16 jt + l16, columns 16 (2w + i) + 4 q4 .. of the tile-major store
+      bf16* eo = p.eout + ((int64_t)gb * H + h) * DD;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int jt = 0; jt < 8; ++jt)
+          *reinterpret_cast<bf16x4*>(eo + blk_index(16 * jt + l16, 16 * (2 * wave + i) + 4 * q4)) =
+              bf4(E[i][jt] * u12);
+    }
       if constexpr (!GLA) return;
     }
     // alpha blend (q read again: the iterations keep x, d and rho in registers)
@@ -1365,265 +1600,10 @@ __device__ __forceinline__ Blk block_of(const Params& p, int gb, int lane) {
   return Blk{s_id, lb, tok0, min(CB, si.eos - tok0)};
 }
 
-// h_c of block gb into sH (fp16, interleaved rows, both triangles), as the solve
-// forms it; the first 256 threads load, all nw waves mirror
-__device__ __forceinline__ void load_hc(const Params& p, f16* sH, const Blk& b, int gb, int h,
-                                        int tid, int wave, int lane, int nw = 4) {
-  if (tid < NTHR) {
-    const int64_t DD = (int64_t)D * D;
-    const int64_t so = ((int64_t)b.s_id * p.H + h) * DD;
-    const int64_t bso = ((int64_t)gb * p.H + h) * DD;
-    StateLd<> hst;
-    solve::state_issue_b<true>(hst, b.lb > 0 ? p.ws_hb + bso : nullptr, tid);
-    const float off_gk = p.ws_boff[((int64_t)gb * p.H + h) * 2];
-    solve::state_issue_s<true>(hst, (b.lb == 0 || off_gk > solve::SEG_STATE_DROP) ? p.ws_h0 + so : nullptr, tid);
-    solve::state_store<true>(sH, hst, fast_exp(off_gk), tid);
-  }
-  lds_barrier();
-  solve::state_fill_lower(sH, wave, lane, nw);
-}
-
 // in-block inclusive cumsum of gk for lanes 0-63 (wave 0); 0 past the block's tokens
 __device__ __forceinline__ float block_decay(const Params& p, const Blk& b, int h, int lane) {
   const bool ok = lane < b.nval;
   return scan64((ok && p.gk) ? ldsc(p.gk, (int64_t)(b.tok0 + lane) * p.H + h, p.gk_dt) : 0.f);
-}
-
-// a_t = -r (dq_t . x_t) / |H_t|_F for token row `row` from the row's staged
-// pieces (features 8 l16 .. 8 l16 + 7 in each lane of its 16-lane group)
-__device__ __forceinline__ float lambda_weight(const Params& p, const Bwd& w, const Blk& b, int row,
-                                               int h, const f32x4& q0, const f32x4& q1,
-                                               const bf16x8& xv) {
-  float d = 0.f;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) d += q0[v] * (float)xv[v] + q1[v] * (float)xv[4 + v];
-  d = row16_sum(d);
-  const float f = (row < b.nval && w.bp_lambda) ? w.fro[(int64_t)(b.tok0 + row) * p.H + h] : 0.f;
-  return f > 0.f ? -p.ridge_ratio * d / f : 0.f;
-}
-
-// x, dq and the ridge weights grow like 1 / |H_t|_F, which is small at a
-// sequence's start: the fp16 operands built from them are scaled by a power of two
-// (exact) chosen from their largest magnitude, and the products unscaled in fp32.
-// pow2_scale(m): 2^j with m 2^j < 2^8 (1 when m is below that already)
-__device__ __forceinline__ float pow2_scale(float m) {
-  int e;
-  (void)frexpf(m, &e);                   // m < 2^e
-  return e > 8 ? ldexpf(1.f, 8 - e) : 1.f;
-}
-__device__ __forceinline__ float wave_max(float x) {
-  x = fmaxf(x, dppf<0xB1>(x));
-  x = fmaxf(x, dppf<0x4E>(x));
-  x = fmaxf(x, dppf<0x141>(x));
-  x = fmaxf(x, dppf<0x140>(x));
-  const unsigned u = __builtin_bit_cast(unsigned, x);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  x = fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
-  const unsigned w = __builtin_bit_cast(unsigned, x);
-  const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return fmaxf(__builtin_bit_cast(float, (unsigned)q[0]), __builtin_bit_cast(float, (unsigned)q[1]));
-}
-// Suffix sums over the 64 lanes of a wave (lane l: lanes l..63), within each row of 16
-// by lane shifts, then the later rows' totals.
-template <int N>
-__device__ __forceinline__ float shl_row(float v) {   // lane l of a row receives lane l + N (0 past it)
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + N,
-                                                               0xF, 0xF, true));
-}
-__device__ __forceinline__ float lane_val(float v, int l) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-__device__ __forceinline__ float suffix_sum64(float x, int lane) {
-  x += shl_row<1>(x);
-  x += shl_row<2>(x);
-  x += shl_row<4>(x);
-  x += shl_row<8>(x);
-  const float r3 = lane_val(x, 48), r2 = lane_val(x, 32) + r3, r1 = lane_val(x, 16) + r2;
-  return x + (lane < 16 ? r1 : lane < 32 ? r2 : lane < 48 ? r3 : 0.f);
-}
-// rho_t = sum_{t' >= t} a_t' e^{2 (g_t' - g_t)} over the 64 lanes t (a_t, g_t in lane t):
-// rho over 2n lanes = rho over n + e^{2 (g_{t+n} - g_t)} (rho over n of lane t + n).
-// One wave forms it while the workgroup waits: as a loop over the later tokens (an LDS
-// read and an exponential each, up to 64) it cost, together with the loops of the gates' suffix sums, the binary
-// search for the block's segment and the lane sums through the LDS, 0.67 of training's
-// 7.25 ms at 8 x 4096 tokens, H = 32 (cheb_e_kernel 0.98 -> 0.77, cheb_dk_kernel 1.69 -> 1.45, gla_bwd_kernel
-// 1.58 -> 1.45 ms).
-__device__ __forceinline__ float decayed_suffix(float a, float g, int lane) {
-  const int l16 = lane & 15;
-  float r = a;
-  auto step = [&](float r_n, float g_n, int n) {
-    if (l16 + n < 16) r += fast_exp(2.f * (g_n - g)) * r_n;
-  };
-  step(shl_row<1>(r), shl_row<1>(g), 1);
-  step(shl_row<2>(r), shl_row<2>(g), 2);
-  step(shl_row<4>(r), shl_row<4>(g), 4);
-  step(shl_row<8>(r), shl_row<8>(g), 8);
-  // the later rows: their sums from lanes 16, 32 and 48, the last first
-  const float g1 = lane_val(g, 16), g2 = lane_val(g, 32), g3 = lane_val(g, 48);
-  const float r3 = lane_val(r, 48);
-  const float r2 = lane_val(r, 32) + fast_exp(2.f * (g3 - g2)) * r3;
-  const float r1 = lane_val(r, 16) + fast_exp(2.f * (g2 - g1)) * r2;
-  const float rn = lane < 16 ? r1 : lane < 32 ? r2 : r3, gn = lane < 16 ? g1 : lane < 32 ? g2 : g3;
-  return lane < 48 ? r + fast_exp(2.f * (gn - g)) * rn : r;
-}
-__device__ __forceinline__ float absmax8(const bf16x8& x) {
-  float m = 0.f;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf((float)x[j]));
-  return m;
-}
-__device__ __forceinline__ float absmax4(const f32x4& x) {
-  return fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
-}
-// The workgroup's maxima of NV per-thread values over NW waves: slot[NV * NW] of
-// LDS scratch; includes a barrier.
-template <int NV, int NW = 4>
-__device__ __forceinline__ void block_max(float (&v)[NV], float* slot, int wave, int lane) {
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    v[i] = wave_max(v[i]);
-    if (lane == 0) slot[NW * i + wave] = v[i];
-  }
-  lds_barrier();
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    float m = slot[NW * i];
-#pragma unroll
-    for (int j = 1; j < NW; ++j) m = fmaxf(m, slot[NW * i + j]);
-    v[i] = m;
-  }
-}
-__device__ __forceinline__ bf16x4 bf4(const f32x4& x) {
-  return bf16x4{(bf16)x[0], (bf16)x[1], (bf16)x[2], (bf16)x[3]};
-}
-__device__ __forceinline__ f32x4 f4(const bf16x4& x) {
-  return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
-}
-__device__ __forceinline__ f16x8 h8_of(const f32x4& a, const f32x4& b, float s) {
-  return f16x8{(f16)(s * a[0]), (f16)(s * a[1]), (f16)(s * a[2]), (f16)(s * a[3]),
-               (f16)(s * b[0]), (f16)(s * b[1]), (f16)(s * b[2]), (f16)(s * b[3])};
-}
-
-constexpr int E_OFF_K = 0, E_OFF_KB = SZ_K, E_OFF_Q = 2 * SZ_K, E_OFF_X = 3 * SZ_K;
-constexpr int E_OFF_H = 4 * SZ_K, E_OFF_SC = E_OFF_H + SZ_H;
-constexpr int E_SMEM = E_OFF_SC + 3 * CB * 4 + 32 * 4;
-constexpr int E_NTHR = 512;             // 8 waves: wave w forms tile row w of E_c
-static_assert(E_SMEM <= 160 * 1024, "LDS budget");
-
-// E_c = -(Ql^T X + X^T Ql) + 2 (alpha h_c + K^T diag(beta) K), Ql = e^{g} dq, of block gb
-__global__ __launch_bounds__(E_NTHR, 1) void cheb_e_kernel(Params p, Bwd w) {
-  __shared__ __align__(16) unsigned char smem[E_SMEM];
-  f16* sK = reinterpret_cast<f16*>(smem + E_OFF_K);
-  f16* sKb = reinterpret_cast<f16*>(smem + E_OFF_KB);
-  f16* sQ = reinterpret_cast<f16*>(smem + E_OFF_Q);
-  f16* sX = reinterpret_cast<f16*>(smem + E_OFF_X);
-  f16* sH = reinterpret_cast<f16*>(smem + E_OFF_H);
-  float* sG = reinterpret_cast<float*>(smem + E_OFF_SC);     // g_t
-  float* sA = sG + CB;                                        // a_t
-  float* sB = sA + CB;                                        // 2 beta_t, then [CB-1 + 1] unused
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q4 = lane >> 4, l16 = lane & 15;
-  const int gb = blockIdx.x, h = blockIdx.y, H = p.H;
-  const Blk b = block_of(p, gb, lane);
-  if (b.nval <= 0) return;
-  constexpr int NP = CB * 16 / E_NTHR;     // staging passes of 32 rows
-
-  load_hc(p, sH, b, gb, h, tid, wave, lane, E_NTHR / 64);
-  if (wave == 0) {
-    const float g = block_decay(p, b, h, lane);
-    sG[lane] = g;
-    if (lane == b.nval - 1) w.gam[(int64_t)gb * H + h] = g;
-  }
-  // the rows, and a_t from them
-  bf16x8 kr[NP], xr[NP];
-  f32x4 q0[NP], q1[NP];
-#pragma unroll
-  for (int pass = 0; pass < NP; ++pass) {
-    const int row = pass * 32 + (tid >> 4), f0 = (tid & 15) * 8;
-    const bool ok = row < b.nval;
-    const int64_t ro = ((int64_t)(b.tok0 + row) * H + h) * D + f0;
-    kr[pass] = ok ? *reinterpret_cast<const bf16x8*>(p.k + (int64_t)(b.tok0 + row) * p.kv_ts + h * D + f0) : bf16x8{};
-    xr[pass] = ok ? *reinterpret_cast<const bf16x8*>(w.x + ro) : bf16x8{};
-    q0[pass] = ok ? *reinterpret_cast<const f32x4*>(w.dq + ro) : f32x4{0.f, 0.f, 0.f, 0.f};
-    q1[pass] = ok ? *reinterpret_cast<const f32x4*>(w.dq + ro + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-    const float a = lambda_weight(p, w, b, row, h, q0[pass], q1[pass], xr[pass]);
-    if (l16 == 0) sA[row] = a;
-  }
-  lds_barrier();
-  // rho_t = sum_{t'>=t} a_t' e^{2(g_t'-g_t)} (lane t of wave 0), beta_t = e^{g_t} rho_t
-  float alpha = 0.f;
-  if (wave == 0) {
-    const float gt = sG[lane];
-    const float rho = decayed_suffix(sA[lane], gt, lane);
-    sB[lane] = lane < b.nval ? 2.f * fast_exp(gt) * rho : 0.f;
-    alpha = __builtin_bit_cast(float, __builtin_amdgcn_readlane(
-                                          __builtin_bit_cast(int, fast_exp(2.f * gt) * rho), 0));
-  }
-  __shared__ float s_alpha;
-  if (tid == 0) s_alpha = alpha;
-  lds_barrier();
-  // stage k, 2 beta k, -e^{g} dq, x (fp16, interleaved; the last three scaled)
-  float mx[3] = {0.f, 0.f, 0.f};            // max |x|, |e^g dq|, |2 beta k|
-#pragma unroll
-  for (int pass = 0; pass < NP; ++pass) {
-    const int row = pass * 32 + (tid >> 4);
-    const float eg = row < b.nval ? -fast_exp(sG[row]) : 0.f;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      q0[pass][v] *= eg;
-      q1[pass][v] *= eg;
-    }
-    mx[0] = fmaxf(mx[0], absmax8(xr[pass]));
-    mx[1] = fmaxf(mx[1], fmaxf(absmax4(q0[pass]), absmax4(q1[pass])));
-    mx[2] = fmaxf(mx[2], fabsf(sB[row]) * absmax8(kr[pass]));
-  }
-  block_max<3, E_NTHR / 64>(mx, reinterpret_cast<float*>(smem + E_OFF_SC + 3 * CB * 4), wave, lane);
-  const float sx = pow2_scale(mx[0]), sq = pow2_scale(mx[1]), sb = pow2_scale(mx[2]);
-#pragma unroll
-  for (int pass = 0; pass < NP; ++pass) {
-    const int row = pass * 32 + (tid >> 4), f0 = (tid & 15) * 8;
-    store8_i(sK + row * LDP, f0, scale_h8(kr[pass], 1.f));
-    store8_i(sKb + row * LDP, f0, scale_h8(kr[pass], sb * sB[row]));
-    store8_i(sX + row * LDP, f0, scale_h8(xr[pass], sx));
-    store8_i(sQ + row * LDP, f0, h8_of(q0[pass], q1[pass], sq));
-  }
-  lds_barrier();
-  const float a2 = 2.f * s_alpha;
-  const float u12 = 1.f / (sx * sq), u3 = 1.f / sb;
-  // wave w: tile row w (state rows 16w..16w+15), all 8 tile columns
-  bf16* eo = w.e + ((int64_t)gb * H + h) * D * D;
-  {
-    const int it = wave;
-    f32x4 E[8], E3[8];
-#pragma unroll
-    for (int jt = 0; jt < 8; ++jt) {
-      E[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      E3[jt] = E[jt];
-    }
-#pragma unroll
-    for (int jk = 0; jk < 2; ++jk) {
-      const f16x8 aq = frag_t_i(sQ, LDP, 32 * jk, 16 * it, lane);
-      const f16x8 ax = frag_t_i(sX, LDP, 32 * jk, 16 * it, lane);
-      const f16x8 ab = frag_t_i(sKb, LDP, 32 * jk, 16 * it, lane);
-#pragma unroll
-      for (int jt = 0; jt < 8; ++jt) {
-        E[jt] = mfma16h(aq, frag_t_i(sX, LDP, 32 * jk, 16 * jt, lane), E[jt]);
-        E[jt] = mfma16h(ax, frag_t_i(sQ, LDP, 32 * jk, 16 * jt, lane), E[jt]);
-        E3[jt] = mfma16h(ab, frag_t_i(sK, LDP, 32 * jk, 16 * jt, lane), E3[jt]);
-      }
-    }
-    // E[jt][v] = E_c[16 it + 4 q4 + v][16 jt + l16]; E_c is symmetric, so the lane
-    // writes it as row 16 jt + l16, columns 16 it + 4 q4 .. +3 of the tile-major store
-#pragma unroll
-    for (int jt = 0; jt < 8; ++jt) {
-      const f16x4 hc = *reinterpret_cast<const f16x4*>(sH + (16 * jt + l16) * LDP + icol(16 * it + 4 * q4));
-      f32x4 y;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) y[v] = u12 * E[jt][v] + u3 * E3[jt][v] + a2 * (float)hc[v];
-      *reinterpret_cast<bf16x4*>(eo + blk_index(16 * jt + l16, 16 * it + 4 * q4)) = bf4(y);
-    }
-  }
 }
 
 // Dn_c = sum over the later blocks of the sequence: one workgroup per (sequence,
@@ -1668,7 +1648,8 @@ static_assert(C_SMEM <= 160 * 1024 && 3 * CB * LDB * 2 <= SZ_H, "LDS budget");
 // first wait, x and dq in the layout of dk's tiles (so dq is read once, for its products
 // and for dgk's dot products).  The in-block matrices x_t.k_s, dq_t.k_s and W_st k_t.k_s
 // are formed once, two of each one's sixteen tiles per wave, and shared through the LDS
-// of h_c.
+// of h_c: 1.45 -> 1.13 ms at 8 x 4096 tokens, H = 32 (3 GB, 0.6 ms at the rate of a copy;
+// the load, product and store phases of the CU's one workgroup do not overlap).
 __global__ __launch_bounds__(C_NTHR, 2) void cheb_dk_kernel(Params p, Bwd w) {
   __shared__ __align__(16) unsigned char smem[C_SMEM];
   f16* sK = reinterpret_cast<f16*>(smem + C_OFF_K);
@@ -2066,7 +2047,8 @@ static_assert(GB_SMEM <= 160 * 1024 && 2 * CB * LDB * 2 <= SZ_H, "LDS budget");
 // first wait, q and x in the layout of du's tiles (so they are read once, for u and for
 // du's dot products).  The in-block matrices e^{G_t-G_s} (do_t.v_s) and e^{G_t-G_s}
 // (u_t.k_s) are formed once, a pair of tiles per wave, and shared through the LDS of
-// S_c (each wave formed its column of both, and the first one's transpose too).  With
+// S_c (each wave formed its column of both, and the first one's transpose too):
+// 1.45 -> 1.19 ms at 8 x 4096 tokens, H = 32 (4.4 GB, 0.87 ms at the rate of a copy).  With
 // the solver du leaves in fp32 once: the solve forms alpha du, its right-hand side, and
 // (1 - alpha) du, the blend's share of dq, from it.
 __global__ __launch_bounds__(GB_NTHR, 2) void gla_bwd_kernel(Params p, GlaBwd w) {
@@ -2495,10 +2477,10 @@ extern "C" int hmx_gka_cheb_bwd(const void* k, int64_t k_token_stride, const voi
   w.dk = static_cast<bf16*>(dk); p.dq_out = static_cast<bf16*>(dq);
   w.dgk = gk ? dgk : nullptr;
   w.bp_lambda = bp_lambda;
+  p.xsol = w.x; p.eout = w.e; p.gam = w.gam; p.bp_lambda = bp_lambda;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(nblock_total, H);
   hipLaunchKernelGGL((solve::gka_solve_kernel<true, false, solve::SM_DQ>), grid, dim3(NTHR), 0, s, p);
-  hipLaunchKernelGGL(train::cheb_e_kernel, grid, dim3(train::E_NTHR), 0, s, p, w);
   hipLaunchKernelGGL(train::cheb_dscan_kernel, dim3(N * H, 16), dim3(256), 0, s, p, w);
   hipLaunchKernelGGL(train::cheb_dk_kernel, grid, dim3(train::C_NTHR), 0, s, p, w);
   return check_launch("hmx_gka_cheb_bwd");
@@ -2644,8 +2626,8 @@ extern "C" int hmx_gka_train_bwd(const void* q, const void* k, const void* v, in
     cw.dk = static_cast<bf16*>(dk); cw.dk_add = dk_gla;
     cw.dgk = gk ? dgk : nullptr;
     cw.bp_lambda = bp_lambda;
+    pc.xsol = cw.x; pc.eout = cw.e; pc.gam = cw.gam; pc.bp_lambda = bp_lambda;
     hipLaunchKernelGGL((solve::gka_solve_kernel<true, false, solve::SM_DQ>), grid, dim3(NTHR), 0, s, pc);
-    hipLaunchKernelGGL(train::cheb_e_kernel, grid, dim3(train::E_NTHR), 0, s, pc, cw);
     hipLaunchKernelGGL(train::cheb_dscan_kernel, sgrid, dim3(256), 0, s, pc, cw);
     hipLaunchKernelGGL(train::cheb_dk_kernel, grid, dim3(train::C_NTHR), 0, s, pc, cw);
   }
