@@ -1914,13 +1914,14 @@ __global__ __launch_bounds__(BNTHR, 3) void gdn_bwd_chain_kernel(Bwd p, int mode
 
 // ---- the per-block gradients -------------------------------------------------
 constexpr int SZR = C * LR * 2, SZS = D * LR * 2, SZL = C * LL * 2;
+constexpr int LG = 36;         // fp32 row stride of the [32][32] arrays (16-byte rows)
 constexpr int G_OFF_K = 0, G_OFF_Q = SZR, G_OFF_DO = 2 * SZR, G_OFF_X = 3 * SZR;
 constexpr int G_OFF_W = 4 * SZR, G_OFF_Z = 5 * SZR;
 constexpr int G_OFF_S0 = 6 * SZR, G_OFF_DS = G_OFF_S0 + SZS;
 constexpr int G_OFF_T = G_OFF_DS + SZS, G_OFF_PM = G_OFF_T + SZL;
 constexpr int G_OFF_DP = G_OFF_PM + SZL, G_OFF_DM = G_OFF_DP + SZL;
-constexpr int G_OFF_QK = G_OFF_DM + SZL, G_OFF_KK = G_OFF_QK + C * LF * 4;
-constexpr int G_OFF_SC = G_OFF_KK + C * LF * 4;            // G, E, F, B, rq, rk
+constexpr int G_OFF_QK = G_OFF_DM + SZL, G_OFF_KK = G_OFF_QK + C * LG * 4;
+constexpr int G_OFF_SC = G_OFF_KK + C * LG * 4;            // G, E, F, B, rq, rk
 constexpr int NPG = 16, NPB = 10;
 constexpr int G_OFF_PG = G_OFF_SC + 6 * C * 4;             // [16][32] dgamma pieces
 constexpr int G_OFF_PB = G_OFF_PG + NPG * C * 4;           // [10][32] dbeta pieces
@@ -1941,12 +1942,20 @@ struct GradPre {
   float g, b;
 };
 
+// the row of ld_row without a branch: a missing row reads the block's first one and
+// becomes zeros
+__device__ __forceinline__ bf16x8 ld_row_nb(const bf16* src, int64_t ts, int tok0, int nval, int tid) {
+  const int row = tid >> 4, f0 = (tid & 15) * 8;
+  const bool ok = row < nval;
+  const bf16x8 x = *reinterpret_cast<const bf16x8*>(src + (int64_t)(tok0 + (ok ? row : 0)) * ts + f0);
+  return ok ? x : bf16x8{};
+}
 __device__ __forceinline__ void grad_load(const Bwd& p, GradPre& r, int64_t bh, int h, int tok0,
                                           int nval, int tid, int wave, int lane) {
-  r.k = ld_row(p.k + (int64_t)h * D, p.kv_ts, tok0, nval, tid);
-  r.q = ld_row(p.q + (int64_t)h * D, p.q_ts, tok0, nval, tid);
-  r.o = ld_row(p.dout + (int64_t)h * D, p.do_ts, tok0, nval, tid);
-  r.v = ld_row(p.v + (int64_t)h * D, p.kv_ts, tok0, nval, tid);
+  r.k = ld_row_nb(p.k + (int64_t)h * D, p.kv_ts, tok0, nval, tid);
+  r.q = ld_row_nb(p.q + (int64_t)h * D, p.q_ts, tok0, nval, tid);
+  r.o = ld_row_nb(p.dout + (int64_t)h * D, p.do_ts, tok0, nval, tid);
+  r.v = ld_row_nb(p.v + (int64_t)h * D, p.kv_ts, tok0, nval, tid);
   const int64_t DD = (int64_t)D * D;
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass) {
@@ -1959,10 +1968,43 @@ __device__ __forceinline__ void grad_load(const Bwd& p, GradPre& r, int64_t bh, 
   r.g = r.b = 0.f;
   if (wave == 0) ld_gates(p, tok0, nval, h, lane, r.g, r.b);
 }
+// put_row in the interleaved feature order
+__device__ __forceinline__ void put_row_i(f16* dst, const bf16x8& x, bool l2, float* rnorm, int tid) {
+  const int row = tid >> 4, f0 = (tid & 15) * 8;
+  const float r = l2 ? row_inv_norm(x) : 1.f;
+  store8_i(dst + row * LR, f0, scale_h8(x, r));
+  if (rnorm && (tid & 15) == 0) rnorm[row] = r;
+}
+// a raw buffer resource over a block's nval rows of a [tokens][H][D] bf16 output: stores
+// past them are dropped, so the rows need no branch around a store (a wait after one
+// would drain every store before it)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t out_rows(const bf16* o, int64_t tok, int h, int H, int nval) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(o) + (tok * H + h) * D, 0,
+                                           (uint32_t)(((int64_t)(nval - 1) * H * D + D) * 2), 0x00020000);
+}
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void st_row4(__amdgpu_buffer_rsrc_t r, uint32_t off, const f32x4& x) {
+  const bf16x4 y = {(bf16)x[0], (bf16)x[1], (bf16)x[2], (bf16)x[3]};
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, y), r, off, 0, 0);
+}
+__device__ __forceinline__ f32x4 ld4_h(const f16* a) {
+  const f16x4 x = *reinterpret_cast<const f16x4*>(a);
+  return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+}
+__device__ __forceinline__ float sum4(const f32x4& x) { return (x[0] + x[1]) + (x[2] + x[3]); }
 
 // Persistent: workgroup w takes blocks (block, head) = w, w + gridDim.x, ... and
 // loads each one's inputs while it processes the one before.
-__global__ __launch_bounds__(BNTHR, 1) void gdn_bwd_grad_kernel(Bwd p) {
+// Tiles are formed transposed (features x tokens; the MFMA operands exchanged), so a
+// lane holds four consecutive features of one token: LDS and memory take one 8-byte
+// access where the token-major tiles took four 2-byte ones, a token's scalars are one
+// value per lane, and row sums take two lane swaps.  The arrays are in the interleaved
+// feature order (mfma.hpp): row and transposing fragments are single, conflict-free
+// reads.  dW alone is token-major: as it is the operand of Z = T^T dW.
+// 8 x 4096 tokens, H = 32: 1.34 -> 1.26 ms (3.4 GB read, 0.9 GB written, 0.85 ms at the
+// rate of a copy).  Latency bounds it: six barriers and the chains between them at two
+// waves per SIMD; with S0 and dS read from cache it takes 1.22 ms, without its stores 1.25.
+__global__ __launch_bounds__(BNTHR, 2) void gdn_bwd_grad_kernel(Bwd p) {
   __shared__ __align__(16) unsigned char smem[G_SMEM];
   f16* sK = reinterpret_cast<f16*>(smem + G_OFF_K);
   f16* sQ = reinterpret_cast<f16*>(smem + G_OFF_Q);
@@ -1993,6 +2035,7 @@ __global__ __launch_bounds__(BNTHR, 1) void gdn_bwd_grad_kernel(Bwd p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q4 = lane >> 4, l16 = lane & 15;
   const int c0 = 16 * wave;      // this wave's value columns (P1-P2) / key features (P3-P5)
+  const int ic = icol4(wave, q4);   // features c0 + 4 q4 .. +3 of a row
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   int it = blockIdx.x;
   if (it >= total) return;
@@ -2009,42 +2052,47 @@ __global__ __launch_bounds__(BNTHR, 1) void gdn_bwd_grad_kernel(Bwd p) {
       ntok0 = p.ctab[ncb * 4];
       nnval = p.ctab[ncb * 4 + 1];
     }
-    const int64_t bh = (int64_t)cb * H + h;
 
-    // ---- P0: stage this block from registers; the next block's loads go out -------
+    // ---- P0: stage this block from registers, with each wave's share of <dS, S0>; the
+    // next block's loads go out -----------------------------------------------------
     lds_barrier();   // the previous block's LDS reads are done
     {
-      put_row(sK, pre.k, p.l2norm, sRk, tid);
-      put_row(sQ, pre.q, p.l2norm, sRq, tid);
-      put_row(sDO, pre.o, false, nullptr, tid);
-      put_row(sX, pre.v, false, nullptr, tid);
+      put_row_i(sK, pre.k, p.l2norm, sRk, tid);
+      put_row_i(sQ, pre.q, p.l2norm, sRq, tid);
+      put_row_i(sDO, pre.o, false, nullptr, tid);
+      put_row_i(sX, pre.v, false, nullptr, tid);
       if (wave == 0) block_scalars(sc, pre.g, pre.b, lane);
+      float d = 0.f;
 #pragma unroll
       for (int pass = 0; pass < 4; ++pass) {
         const int e = (pass * BNTHR + tid) * 8, row = e >> 7, col = e & 127;
-        *reinterpret_cast<f16x8*>(sS0 + row * LR + col) = pre.s0[pass];
-        *reinterpret_cast<f16x8*>(sDS + row * LR + col) = pre.ds[pass];
+        store8_i(sS0 + row * LR, col, pre.s0[pass]);
+        store8_i(sDS + row * LR, col, pre.ds[pass]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) d += (float)pre.s0[pass][j] * (float)pre.ds[pass][j];
       }
+      d = wave_sum_v(d);
+      if (lane == 0) sPD[wave] = d;
       const int e2 = 2 * tid, i = e2 >> 5, j = e2 & 31;
-      *reinterpret_cast<uint32_t*>(sT + i * LL + j) = pre.t;
-      *reinterpret_cast<uint32_t*>(sPm + i * LL + j) = pre.pm;
+      *reinterpret_cast<uint32_t*>(sT + i * LL + icol(j)) = pre.t;
+      *reinterpret_cast<uint32_t*>(sPm + i * LL + icol(j)) = pre.pm;
     }
     if (nxt < total) grad_load(p, pre, (int64_t)ncb * H + nh, nh, ntok0, nnval, tid, wave, lane);
     lds_barrier();
 
-    // ---- P1: K^ S0 and K^ dS (tokens x this wave's value columns), a tile of Q^K^T
-    // or K^K^T, this wave's share of <dS, S0>; Ut = V - E K^ S0, beta Ut over V ----
+    // ---- P1: (K^ S0)^T and K^ dS (this wave's value columns), a tile of Q^K^T or
+    // K^K^T; Ut = V - E K^ S0, beta Ut over V -----------------------------------------
     f32x4 Ut[2], KD[2];
     {
       f32x4 KS[2] = {zero, zero};
       KD[0] = KD[1] = zero;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        const f16x8 bs = frag_col(sS0, LR, 32 * ks, c0, lane), bd = frag_col(sDS, LR, 32 * ks, c0, lane);
+        const f16x8 bs = frag_t_i(sS0, LR, 32 * ks, c0, lane), bd = frag_t_i(sDS, LR, 32 * ks, c0, lane);
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
-          const f16x8 a = frag_h(sK, LR, 16 * mt, 32 * ks, lane);
-          KS[mt] = mfma16h(a, bs, KS[mt]);
+          const f16x8 a = frag_i(sK, LR, 16 * mt, 32 * ks, lane);
+          KS[mt] = mfma16h(bs, a, KS[mt]);
           KD[mt] = mfma16h(a, bd, KD[mt]);
         }
       }
@@ -2054,70 +2102,46 @@ __global__ __launch_bounds__(BNTHR, 1) void gdn_bwd_grad_kernel(Bwd p) {
         f32x4 acc = zero;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
-          acc = mfma16h(frag_h(A, LR, 16 * mt, 32 * ks, lane), frag_h(sK, LR, 16 * nt, 32 * ks, lane), acc);
+          acc = mfma16h(frag_i(sK, LR, 16 * nt, 32 * ks, lane), frag_i(A, LR, 16 * mt, 32 * ks, lane), acc);
         float* dst = wave < 4 ? sQK : sKK;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) dst[(16 * mt + 4 * q4 + v) * LF + 16 * nt + l16] = acc[v];
-      }
-      {
-        float d = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int row = 16 * wave + 4 * i + q4, col = 8 * l16;
-          const f16x8 a = *reinterpret_cast<const f16x8*>(sS0 + row * LR + col);
-          const f16x8 b = *reinterpret_cast<const f16x8*>(sDS + row * LR + col);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) d += (float)a[j] * (float)b[j];
-        }
-        d = wave_sum(d);
-        if (lane == 0) sPD[wave] = d;
+        *reinterpret_cast<f32x4*>(dst + (16 * mt + l16) * LG + 16 * nt + 4 * q4) = acc;
       }
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        const f32x4 e4 = row4(sc.E, mt, q4), b4 = row4(sc.B, mt, q4);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = 16 * mt + 4 * q4 + v, idx = r * LR + c0 + l16;
-          Ut[mt][v] = (float)sX[idx] - e4[v] * KS[mt][v];
-          sX[idx] = (f16)(b4[v] * Ut[mt][v]);
-        }
+        const int r = 16 * mt + l16;
+        f16* x = sX + r * LR + ic;
+        Ut[mt] = ld4_h(x) - KS[mt] * sc.E[r];
+        *reinterpret_cast<f16x4*>(x) = h4(Ut[mt] * sc.B[r]);
       }
     }
     lds_barrier();
 
     // ---- P2: W = T (beta Ut); dW = P^T dO + F K^ dS; Z = T^T dW; dv; rowdot(Z, Ut) --
     {
-      const f16x8 bx = frag_col(sX, LR, 0, c0, lane), bdo = frag_col(sDO, LR, 0, c0, lane);
+      const f16x8 bx = frag_t_i(sX, LR, 0, c0, lane), bdo = frag_t_i(sDO, LR, 0, c0, lane);
+      const auto ov = out_rows(p.dv, tok0, h, H, nval);
       f32x4 W[2], dW[2];
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        W[mt] = mfma16h(frag_h(sT, LL, 16 * mt, 0, lane), bx, zero);
-        const f32x4 f4r = row4(sc.F, mt, q4);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) dW[mt][v] = f4r[v] * KD[mt][v];
-        dW[mt] = mfma16h(frag_col(sPm, LL, 0, 16 * mt, lane), bdo, dW[mt]);
+        W[mt] = mfma16h(bx, frag_i(sT, LL, 16 * mt, 0, lane), zero);
+        dW[mt] = row4(sc.F, mt, q4) * KD[mt];
+        dW[mt] = mfma16h(frag_t_i(sPm, LL, 0, 16 * mt, lane), bdo, dW[mt]);
       }
       const f16x8 bw = h8(dW[0], dW[1]);
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        const f32x4 Z = mfma16h(frag_t_perm_h(sT, LL, 0, 16 * mt, lane), bw, zero);
-        const f32x4 b4 = row4(sc.B, mt, q4);
-        f32x4 zu;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = 16 * mt + 4 * q4 + v, idx = r * LR + c0 + l16;
-          sW[idx] = (f16)W[mt][v];
-          sZ[idx] = (f16)Z[v];
-          if (r < nval) p.dv[((int64_t)(tok0 + r) * H + h) * D + c0 + l16] = (bf16)(b4[v] * Z[v]);
-          zu[v] = Z[v] * Ut[mt][v];
-        }
-        const float zs = row16_sum4(zu, l16);
-        if (l16 < 4) sPB[wave * C + 16 * mt + 4 * q4 + l16] = zs;
+        const int r = 16 * mt + l16;
+        const f32x4 Z = mfma16h(bw, frag_t_i(sT, LL, 0, 16 * mt, lane), zero);
+        *reinterpret_cast<f16x4*>(sW + r * LR + ic) = h4(W[mt]);
+        *reinterpret_cast<f16x4*>(sZ + r * LR + ic) = h4(Z);
+        st_row4(ov, (uint32_t)((r * H * D + c0 + 4 * q4) * 2), Z * sc.B[r]);
+        const float zs = q4_sum(sum4(Z * Ut[mt]));
+        if (q4 == 0) sPB[wave * C + r] = zs;
       }
     }
     lds_barrier();
 
-    // ---- P3: dO S0^T, Z S0^T, W dS^T (tokens x this wave's key features); a tile of
+    // ---- P3: dO S0^T, Z S0^T, W dS^T (this wave's key features x tokens); a tile of
     // Z W^T (-> dN, Dm) or dO W^T (-> Dp) with their row and column sums -------------
     f32x4 DQ[2], DK[2];
     f32x4 qh[2], kh[2];      // q^, k^ at this lane's accumulator positions
@@ -2126,138 +2150,113 @@ __global__ __launch_bounds__(BNTHR, 1) void gdn_bwd_grad_kernel(Bwd p) {
       f32x4 A0[2] = {zero, zero}, A1[2] = {zero, zero}, A2[2] = {zero, zero};
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        const f16x8 bs = frag_h(sS0, LR, c0, 32 * ks, lane), bd = frag_h(sDS, LR, c0, 32 * ks, lane);
+        const f16x8 bs = frag_i(sS0, LR, c0, 32 * ks, lane), bd = frag_i(sDS, LR, c0, 32 * ks, lane);
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
-          A0[mt] = mfma16h(frag_h(sDO, LR, 16 * mt, 32 * ks, lane), bs, A0[mt]);
-          A1[mt] = mfma16h(frag_h(sZ, LR, 16 * mt, 32 * ks, lane), bs, A1[mt]);
-          A2[mt] = mfma16h(frag_h(sW, LR, 16 * mt, 32 * ks, lane), bd, A2[mt]);
+          A0[mt] = mfma16h(bs, frag_i(sDO, LR, 16 * mt, 32 * ks, lane), A0[mt]);
+          A1[mt] = mfma16h(bs, frag_i(sZ, LR, 16 * mt, 32 * ks, lane), A1[mt]);
+          A2[mt] = mfma16h(bd, frag_i(sW, LR, 16 * mt, 32 * ks, lane), A2[mt]);
         }
       }
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        const f32x4 e4 = row4(sc.E, mt, q4), b4 = row4(sc.B, mt, q4), f4r = row4(sc.F, mt, q4);
-        f32x4 gq;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = 16 * mt + 4 * q4 + v, idx = r * LR + c0 + l16;
-          const float qt = p.scale * e4[v] * A0[mt][v];
-          const float ut = -e4[v] * b4[v] * A1[mt][v];
-          const float st = f4r[v] * A2[mt][v];
-          qh[mt][v] = (float)sQ[idx];
-          kh[mt][v] = (float)sK[idx];
-          DQ[mt][v] = qt;
-          DK[mt][v] = ut + st;
-          gq[v] = qh[mt][v] * qt + kh[mt][v] * (ut - st);
-          cs += kh[mt][v] * st;
-        }
-        const float gs = row16_sum4(gq, l16);
-        if (l16 < 4) sPG[(8 + wave) * C + 16 * mt + 4 * q4 + l16] = gs;
+        const int r = 16 * mt + l16;
+        const float e = sc.E[r], eb = -e * sc.B[r], f = sc.F[r];
+        qh[mt] = ld4_h(sQ + r * LR + ic);
+        kh[mt] = ld4_h(sK + r * LR + ic);
+        DQ[mt] = A0[mt] * (p.scale * e);
+        const f32x4 ut = A1[mt] * eb, st = A2[mt] * f;
+        DK[mt] = ut + st;
+        const float gs = q4_sum(sum4(qh[mt] * DQ[mt] + kh[mt] * (ut - st)));
+        cs += sum4(kh[mt] * st);
+        if (q4 == 0) sPG[(8 + wave) * C + r] = gs;
       }
-      cs = wave_sum(cs);
+      cs = wave_sum_v(cs);
       if (lane == 0) sPC[wave] = cs;
     }
     {
       const int t = wave & 3, mt = t >> 1, nt = t & 1;
       const f16* A = wave < 4 ? sZ : sDO;
-      f32x4 acc = zero;
+      f32x4 acc = zero;        // rows j = 16 nt + 4 q4 + v, column i = 16 mt + l16
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
-        acc = mfma16h(frag_h(A, LR, 16 * mt, 32 * ks, lane), frag_h(sW, LR, 16 * nt, 32 * ks, lane), acc);
-      const int j = 16 * nt + l16;
-      const float gj = sc.G[j];
-      const f32x4 gi4 = row4(sc.G, mt, q4), bi4 = row4(sc.B, mt, q4);
-      float csum = 0.f;
-      f32x4 xs, dbs;
+        acc = mfma16h(frag_i(sW, LR, 16 * nt, 32 * ks, lane), frag_i(A, LR, 16 * mt, 32 * ks, lane), acc);
+      const int i = 16 * mt + l16, j0 = 16 * nt + 4 * q4;
+      const float gi = sc.G[i], bi = sc.B[i];
+      const f32x4 gj = row4(sc.G, nt, q4);
+      const f32x4 m4 = *reinterpret_cast<const f32x4*>((wave < 4 ? sKK : sQK) + i * LG + j0);
+      f32x4 xs, d;
+      float dbs = 0.f;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int i = 16 * mt + 4 * q4 + v;
-        const float gm = j <= i ? fast_exp(gi4[v] - gj) : 0.f;
-        float x;
+        const float gm = j0 + v <= i ? fast_exp(gi - gj[v]) : 0.f;
         if (wave < 4) {   // dN = -strict_lower(Z W^T), Dm = beta dN . Gm
-          const float dn = j < i ? -acc[v] : 0.f;
-          const float kk = sKK[i * LF + j];
-          const float d = bi4[v] * dn * gm;
-          sDm[i * LL + j] = (f16)d;
-          x = d * kk;
-          dbs[v] = dn * kk * gm;
+          const float dn = j0 + v < i ? -acc[v] : 0.f;
+          d[v] = bi * dn * gm;
+          dbs += dn * m4[v] * gm;
         } else {          // Dp = scale lower(dO W^T) . Gm
-          const float d = p.scale * acc[v] * gm;
-          sDp[i * LL + j] = (f16)d;
-          x = d * sQK[i * LF + j];
-          dbs[v] = 0.f;
+          d[v] = p.scale * acc[v] * gm;
         }
-        xs[v] = x;
-        csum += x;
+        xs[v] = d[v] * m4[v];
       }
-      const int ri = 16 * mt + 4 * q4 + l16;   // the row whose sums this lane holds (l16 < 4)
+      *reinterpret_cast<f16x4*>((wave < 4 ? sDm : sDp) + i * LL + icol4(nt, q4)) = h4(d);
       if (wave < 4) {
-        const float db = row16_sum4(dbs, l16);
-        if (l16 < 4) sPB[(8 + nt) * C + ri] = db;
+        const float db = q4_sum(dbs);
+        if (q4 == 0) sPB[(8 + nt) * C + i] = db;
       }
-      const float rs = row16_sum4(xs, l16);
-      if (l16 < 4) sPG[((wave < 4 ? 0 : 2) + nt) * C + ri] = rs;
-      csum += __shfl_xor(csum, 16, 64);
-      csum += __shfl_xor(csum, 32, 64);
-      if (q4 == 0) sPG[((wave < 4 ? 4 : 6) + mt) * C + j] = -csum;
+      const float rs = q4_sum(sum4(xs));
+      if (q4 == 0) sPG[((wave < 4 ? 0 : 2) + nt) * C + i] = rs;
+      const float csum = row16_sum4(xs, l16);   // l16 < 4: column j0 + l16
+      if (l16 < 4) sPG[((wave < 4 ? 4 : 6) + mt) * C + j0 + l16] = -csum;
     }
     lds_barrier();
 
     // ---- P4: dQ^ += Dp K^; dK^ += Dp^T Q^ + (Dm + Dm^T) K^; the L2 backward's row dots
     {
-      const f16x8 bk = frag_col(sK, LR, 0, c0, lane), bq = frag_col(sQ, LR, 0, c0, lane);
+      const f16x8 bk = frag_t_i(sK, LR, 0, c0, lane), bq = frag_t_i(sQ, LR, 0, c0, lane);
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        DQ[mt] = mfma16h(frag_h(sDp, LL, 16 * mt, 0, lane), bk, DQ[mt]);
-        DK[mt] = mfma16h(frag_col(sDp, LL, 0, 16 * mt, lane), bq, DK[mt]);
-        DK[mt] = mfma16h(frag_h(sDm, LL, 16 * mt, 0, lane), bk, DK[mt]);
-        DK[mt] = mfma16h(frag_col(sDm, LL, 0, 16 * mt, lane), bk, DK[mt]);
+        DQ[mt] = mfma16h(bk, frag_i(sDp, LL, 16 * mt, 0, lane), DQ[mt]);
+        DK[mt] = mfma16h(bq, frag_t_i(sDp, LL, 0, 16 * mt, lane), DK[mt]);
+        DK[mt] = mfma16h(bk, frag_i(sDm, LL, 16 * mt, 0, lane), DK[mt]);
+        DK[mt] = mfma16h(bk, frag_t_i(sDm, LL, 0, 16 * mt, lane), DK[mt]);
       }
+      if (p.l2norm) {
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        f32x4 xq, xk;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          xq[v] = qh[mt][v] * DQ[mt][v];
-          xk[v] = kh[mt][v] * DK[mt][v];
-        }
-        const float sq = row16_sum4(xq, l16), sk = row16_sum4(xk, l16);
-        if (l16 < 4) {
-          sPQ[wave * C + 16 * mt + 4 * q4 + l16] = sq;
-          sPK[wave * C + 16 * mt + 4 * q4 + l16] = sk;
+        for (int mt = 0; mt < 2; ++mt) {
+          const float sq = q4_sum(sum4(qh[mt] * DQ[mt])), sk = q4_sum(sum4(kh[mt] * DK[mt]));
+          if (q4 == 0) {
+            sPQ[wave * C + 16 * mt + l16] = sq;
+            sPK[wave * C + 16 * mt + l16] = sk;
+          }
         }
       }
     }
     lds_barrier();
 
     // ---- P5: dq, dk (through the L2 normalisation); dg, dbeta --------------------
+    {
+      const auto oq = out_rows(p.dq, tok0, h, H, nval), ok = out_rows(p.dk, tok0, h, H, nval);
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      f32x4 sq = zero, sk = zero;
-      if (p.l2norm) {
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-          sq += row4(sPQ + w * C, mt, q4);
-          sk += row4(sPK + w * C, mt, q4);
-        }
-      }
-      const f32x4 rq4 = row4(sRq, mt, q4), rk4 = row4(sRk, mt, q4);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = 16 * mt + 4 * q4 + v;
-        float dq = DQ[mt][v], dk = DK[mt][v];
+      for (int mt = 0; mt < 2; ++mt) {
+        const int r = 16 * mt + l16;
+        f32x4 dq = DQ[mt], dk = DK[mt];
         if (p.l2norm) {
-          dq = rq4[v] * (dq - qh[mt][v] * sq[v]);
-          dk = rk4[v] * (dk - kh[mt][v] * sk[v]);
+          float sq = 0.f, sk = 0.f;
+#pragma unroll
+          for (int w = 0; w < 8; ++w) {
+            sq += sPQ[w * C + r];
+            sk += sPK[w * C + r];
+          }
+          dq = (dq - qh[mt] * sq) * sRq[r];
+          dk = (dk - kh[mt] * sk) * sRk[r];
         }
-        if (r < nval) {
-          const int64_t o = ((int64_t)(tok0 + r) * H + h) * D + c0 + l16;
-          p.dq[o] = (bf16)dq;
-          p.dk[o] = (bf16)dk;
-        }
+        const uint32_t o = (uint32_t)((r * H * D + c0 + 4 * q4) * 2);
+        st_row4(oq, o, dq);
+        st_row4(ok, o, dk);
       }
     }
-    if (wave == 0) {
+    if (wave == 7) {
       float dgam = 0.f, db = 0.f, ctot = 0.f, dd = 0.f;
       if (lane < C) {
 #pragma unroll
@@ -2271,12 +2270,7 @@ __global__ __launch_bounds__(BNTHR, 1) void gdn_bwd_grad_kernel(Bwd p) {
         ctot += sPC[w];
       }
       if (lane == C - 1) dgam += sc.E[C - 1] * dd + ctot;
-      // in-block reverse inclusive cumsum over lanes 0-31
-#pragma unroll
-      for (int off = 1; off < C; off <<= 1) {
-        const float y = __shfl_down(dgam, off, 64);
-        if (lane + off < C) dgam += y;
-      }
+      dgam = suffix_sum64(dgam, lane);   // in-block reverse inclusive cumsum (lanes 0-31)
       if (lane < nval) {
         const int64_t o = (int64_t)(tok0 + lane) * H + h;
         p.dg[o] = dgam;

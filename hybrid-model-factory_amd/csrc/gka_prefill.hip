@@ -570,24 +570,6 @@ __device__ __forceinline__ float wave_max(float x) {
   const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
   return fmaxf(__builtin_bit_cast(float, (unsigned)q[0]), __builtin_bit_cast(float, (unsigned)q[1]));
 }
-// Suffix sums over the 64 lanes of a wave (lane l: lanes l..63), within each row of 16
-// by lane shifts, then the later rows' totals.
-template <int N>
-__device__ __forceinline__ float shl_row(float v) {   // lane l of a row receives lane l + N (0 past it)
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + N,
-                                                               0xF, 0xF, true));
-}
-__device__ __forceinline__ float lane_val(float v, int l) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-__device__ __forceinline__ float suffix_sum64(float x, int lane) {
-  x += shl_row<1>(x);
-  x += shl_row<2>(x);
-  x += shl_row<4>(x);
-  x += shl_row<8>(x);
-  const float r3 = lane_val(x, 48), r2 = lane_val(x, 32) + r3, r1 = lane_val(x, 16) + r2;
-  return x + (lane < 16 ? r1 : lane < 32 ? r2 : lane < 48 ? r3 : 0.f);
-}
 // rho_t = sum_{t' >= t} a_t' e^{2 (g_t' - g_t)} over the 64 lanes t (a_t, g_t in lane t):
 // rho over 2n lanes = rho over n + e^{2 (g_{t+n} - g_t)} (rho over n of lane t + n).
 // One wave forms it while the workgroup waits: as a loop over the later tokens (an LDS

@@ -190,6 +190,25 @@ __device__ __forceinline__ float q4_sum(float x) {
 }
 __device__ __forceinline__ float wave_sum_v(float x) { return q4_sum(row16_sum(x)); }
 
+// Suffix sums over the 64 lanes of a wave (lane l: lanes l..63), within each row of 16
+// by lane shifts, then the later rows' totals.
+template <int N>
+__device__ __forceinline__ float shl_row(float v) {   // lane l of a row receives lane l + N (0 past it)
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + N,
+                                                               0xF, 0xF, true));
+}
+__device__ __forceinline__ float lane_val(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+__device__ __forceinline__ float suffix_sum64(float x, int lane) {
+  x += shl_row<1>(x);
+  x += shl_row<2>(x);
+  x += shl_row<4>(x);
+  x += shl_row<8>(x);
+  const float r3 = lane_val(x, 48), r2 = lane_val(x, 32) + r3, r1 = lane_val(x, 16) + r2;
+  return x + (lane < 16 ? r1 : lane < 32 ? r2 : lane < 48 ? r3 : 0.f);
+}
+
 // Inclusive prefix sum over lanes 0..31 (two DPP rows) with VALU lane shifts.
 #define HMX_DPP_F(v, ctrl, rmask) \
   __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (v)), (ctrl), \
@@ -285,6 +304,8 @@ __device__ __forceinline__ f16x8 frag_t_i(const f16* b, int ld, int t0, int c0, 
   const f16x4 y = ld_tr_i(b, ld, tq + 16, c0, lane);
   return f16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
 }
+// icol(16 blk + 4 m), the position of the 4-feature chunk m of 16-feature block `blk`
+__device__ __forceinline__ int icol4(int blk, int m) { return ((blk >> 1) << 5) + ((blk & 1) << 2) + 8 * m; }
 // stores features f0..f0+7 (f0 a multiple of 8) of an interleaved row
 __device__ __forceinline__ void store8_i(f16* row, int f0, const f16x8& y) {
   *reinterpret_cast<f16x4*>(row + icol(f0)) = f16x4{y[0], y[1], y[2], y[3]};

@@ -446,10 +446,8 @@ struct GLay {
 __device__ __forceinline__ bf16x8 fr(const bf16* b, int ld, int r0, int k0, int lane) {
   return __builtin_bit_cast(bf16x8, frag_i(reinterpret_cast<const f16*>(b), ld, r0, k0, lane));
 }
-// position of the 4-feature chunk m of 16-feature block `blk`, icol(16 blk + 4 m): written
-// so that a compile-time block of an even first block stays an immediate offset
-__device__ __forceinline__ int icol4(int blk, int m) { return ((blk >> 1) << 5) + ((blk & 1) << 2) + 8 * m; }
-// transposed fragment (frag_t_i) of rows t0.., 16-column block c0 + c (c0 even)
+// transposed fragment (frag_t_i) of rows t0.., 16-column block c0 + c (c0 even, or c 0):
+// a compile-time c stays an immediate offset
 __device__ __forceinline__ bf16x8 fr_t(const bf16* b, int ld, int t0, int c0, int c, int lane) {
   const bf16* a = b + (4 * (lane >> 4) + ((lane & 15) >> 2)) * ld + icol4(c0, lane & 3) +
                   t0 * ld + icol4(c, 0);
