@@ -40,7 +40,10 @@ class ProjGates:
     gk_from_g: bool = False
 
     def tokens(self, lo: int, hi: int) -> "ProjGates":
-        """The gates of tokens [lo, hi) (views of the projections)."""
+        """The gates of tokens [lo, hi) (views of the projections; itself for all)."""
+        whole = [t for t in (self.a, self.b, self.alpha_in) if t is not None]
+        if lo == 0 and all(t.shape[0] == hi for t in whole):
+            return self
         cut = lambda t: None if t is None else t[lo:hi]
         return replace(self, a=cut(self.a), b=cut(self.b), alpha_in=cut(self.alpha_in))
 

@@ -32,6 +32,14 @@ def _i32(t: torch.Tensor | None) -> torch.Tensor | None:
     return t.contiguous()
 
 
+def _rows_contiguous(t: torch.Tensor) -> bool:
+    """Whether row 0 of a [rows, H, K, V] pool (and so every row) is contiguous; the
+    strides of the common case are compared without making a view of the row."""
+    if t.dim() == 4 and t.shape[0] and t.stride()[1:] == (t.shape[2] * t.shape[3], t.shape[3], 1):
+        return True
+    return t[0].is_contiguous()
+
+
 def _token_rows(t: torch.Tensor, mult: int) -> tuple[torch.Tensor, int]:
     """(t, token stride) for a [B, T, heads, dim] tensor whose B*T tokens sit at one
     stride with each token's heads contiguous -- the column slices of a fused
@@ -144,7 +152,7 @@ def fused_recurrent_gated_delta_rule_gqa(
         sdt = torch.float32 if initial_state is None else initial_state.dtype
         final_state = q.new_empty(B, T, H, K, V, dtype=sdt)
     if initial_state is not None:
-        if tuple(initial_state.shape[1:]) != (H, K, V) or not initial_state[0].is_contiguous():
+        if tuple(initial_state.shape[1:]) != (H, K, V) or not _rows_contiguous(initial_state):
             raise ValueError(f"initial_state must be [rows,{H},{K},{V}] with contiguous rows, "
                              f"got {tuple(initial_state.shape)}")
         if initial_state.dtype != final_state.dtype:
@@ -375,7 +383,7 @@ def chunk_gated_delta_rule_gqa(
         if idx.shape != (N,):
             raise ValueError(f"ssm_state_indices must hold {N} slots, got {tuple(idx.shape)}")
         pool = initial_state
-        if (pool.dim() != 4 or tuple(pool.shape[1:]) != (H, K, V) or not pool[0].is_contiguous()
+        if (pool.dim() != 4 or tuple(pool.shape[1:]) != (H, K, V) or not _rows_contiguous(pool)
                 or pool.dtype not in (torch.float32, torch.bfloat16)):
             raise ValueError(f"the state pool must be [slots,{H},{K},{V}] fp32/bf16 with "
                              f"contiguous slots, got {tuple(pool.shape)} {pool.dtype}")

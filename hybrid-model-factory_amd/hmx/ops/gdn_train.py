@@ -20,6 +20,8 @@ and the per-block gradients.  bf16 q/k/v with head dim 128 only.
 """
 from __future__ import annotations
 
+import functools
+
 import numpy as np
 import torch
 
@@ -37,6 +39,22 @@ def block_table(bounds: list[tuple[int, int]]):
             rows.append((t0, min(CHUNK, eos - t0), n, c))
         cu.append(len(rows))
     return np.asarray(rows, dtype=np.int32).reshape(-1, 4), np.asarray(cu, dtype=np.int32)
+
+
+@functools.lru_cache(maxsize=64)
+def _block_plan(bounds: tuple):
+    """block_table, kept for the last few distinct sizes (it depends on them alone and
+    takes 0.5 ms at 1024 blocks)."""
+    return block_table(bounds)
+
+
+@functools.lru_cache(maxsize=64)
+def _chain_plan(bounds: tuple, H: int, cu_count: int, seg_blocks):
+    """The checked chain_segments of ``bounds``, kept like _block_plan."""
+    cu = _block_plan(bounds)[1]
+    rows = chain_segments(cu, H, cu_count, seg_blocks)
+    check_chain_segments(rows, cu)
+    return rows
 
 
 def chain_segments(cu_blocks: np.ndarray, H: int, cu_count: int, seg_blocks: int | None = None):
@@ -108,7 +126,7 @@ def block_states(q, k, v, g, beta, scale, h0, bounds, l2norm, segment_chunks=Non
     (host rows, device table, device cu_blocks, host cu_blocks)."""
     B, T, H, D = q.shape
     N = len(bounds)
-    rows_np, cu_np = block_table(bounds)
+    rows_np, cu_np = _block_plan(tuple(bounds))
     nblk = rows_np.shape[0]
     hc = torch.empty(max(nblk, 1), H, D, D, dtype=torch.float16, device=q.device)
     cu_dev = _device_table(cu_np, q.device)
@@ -143,8 +161,7 @@ def chunk_backward(q, k, v, g, beta, scale, h0, do, dht, bounds, l2norm, segment
     hc, rows_np, tab, cu_dev, cu_np = block_states(q, k, v, g, beta, scale, h0, bounds, l2norm,
                                                    segment_chunks)
     nblk = rows_np.shape[0]
-    cseg_np = chain_segments(cu_np, H, _cu_count(q.device), segment_chunks)
-    check_chain_segments(cseg_np, cu_np)
+    cseg_np = _chain_plan(tuple(bounds), H, _cu_count(q.device), segment_chunks)
     cseg = _device_table(cseg_np, q.device)
     covered = sum(e - b for b, e in bounds) == B * T
     alloc = torch.empty if covered else torch.zeros

@@ -19,8 +19,8 @@ import torch
 
 from .. import _lib
 from .gates import ProjGates
-from .gdn import (_cu_count, _device_table, _gate_rows, _i32, _segment_table, _token_rows,
-                  seq_bounds)
+from .gdn import (_cu_count, _device_table, _gate_rows, _i32, _rows_contiguous, _segment_table,
+                  _token_rows, seq_bounds)
 
 GKA_BLOCK = 64              # tokens per block: the solve kernel's unit and the planner's chunk
 _warned_num_iter_zero = False
@@ -104,7 +104,7 @@ def chebyshev_iteration_gqa(k, q, v, alpha, gk=None, beta=None, num_iter: int = 
     if initial_state_kk.dtype != torch.float32:
         raise NotImplementedError("h_kk state must be float32 (primed_gka_layer.py:424-430)")
     for st, last in ((initial_state_kk, D), (initial_state_kv, V)):
-        if tuple(st.shape[1:]) != (H, D, last) or not st[0].is_contiguous():
+        if tuple(st.shape[1:]) != (H, D, last) or not _rows_contiguous(st):
             raise ValueError(f"state must be [rows,{H},{D},{last}] with contiguous rows, "
                              f"got {tuple(st.shape)}")
     alpha = None if alpha is None else alpha.contiguous()
@@ -249,7 +249,7 @@ def _gka_prefill(q, k, v, alpha, g, gk, beta, gla_scale, ridge_ratio, num_iter, 
         for st, last, name in ((h_kk_initial, D, "h_kk_initial"),
                                (h_kv_initial, V, "h_kv_initial")):
             if (st is None or st.dim() != 4 or tuple(st.shape[1:]) != (H, D, last)
-                    or not st[0].is_contiguous() or st.dtype not in (torch.float32, torch.bfloat16)):
+                    or not _rows_contiguous(st) or st.dtype not in (torch.float32, torch.bfloat16)):
                 raise ValueError(f"{name} must be the state pool [slots,{H},{D},{last}] fp32/bf16 "
                                  f"with contiguous slots")
             pools.append(st)

@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from .gdn import _cu_count, _device_table, _segment_table, seq_bounds
+from .gdn import _cu_count, _device_table, _rows_contiguous, _segment_table, seq_bounds
 
 SSD_CHUNK = 64                 # the kernel's internal chunk length (tokens)
 PAD_SLOT_ID = -1
@@ -235,7 +235,9 @@ def mamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bia
     hT = _ssd_scan(xf, _tokens_view(dt), A, _tokens_view(B), _tokens_view(C), D, zf, dt_bias,
                    dt_softplus, dt_limit, bounds, h0, y.view(b * l, H, P), want, _segment_chunks)
     out = [y]
-    if return_final_states:
+    if return_final_states and last_of_row == list(range(b)) and len(bounds) == b:
+        out.append(hT)      # one sequence a row: the end states as the scan wrote them
+    elif return_final_states:
         fin = torch.zeros(b, H, P, N, dtype=torch.float32, device=x.device)
         for r, i in enumerate(last_of_row):
             if i >= 0:
@@ -299,7 +301,7 @@ def mamba_chunk_scan_combined_varlen(x, dt, A, B, C, chunk_size, cu_seqlens, cu_
         _lib.require_gpu(ssm_state_indices, has_initial_state)
         pool = initial_states
         if (pool is None or pool.dim() != 4 or tuple(pool.shape[1:]) != (H, P, N)
-                or not pool[0].is_contiguous() or pool.dtype not in (torch.float32, torch.bfloat16)):
+                or not _rows_contiguous(pool) or pool.dtype not in (torch.float32, torch.bfloat16)):
             raise ValueError(f"with ssm_state_indices, initial_states must be the state pool "
                              f"[slots,{H},{P},{N}] fp32/bf16 with contiguous slots")
         idx = ssm_state_indices.to(torch.int32).contiguous()

@@ -10,6 +10,9 @@ gradients, then the per-chunk gradient kernel.
 """
 from __future__ import annotations
 
+import functools
+
+import numpy as np
 import torch
 
 from .. import _lib
@@ -31,6 +34,15 @@ def _chunk_table(bounds):
     return rows, seqs
 
 
+@functools.lru_cache(maxsize=64)
+def _chunk_arrays(bounds: tuple):
+    """_chunk_table as int32 arrays (a plan of the sizes alone: building and converting it
+    takes 0.3 ms at 512 chunks)."""
+    rows, seqs = _chunk_table(bounds)
+    return (np.asarray(rows, dtype=np.int32).reshape(-1, 8),
+            np.asarray(seqs, dtype=np.int32).reshape(-1, 2))
+
+
 def ssd_chunk_scan_bwd(x, dt, A, B, C, D, z, dt_bias, dt_softplus, dt_limit, bounds, h0, dy,
                        d_final=None, want_dh0=False):
     """Gradients of the flattened scan (the _ssd_scan layout: x [T,HX,P], dt [T,H],
@@ -48,7 +60,7 @@ def ssd_chunk_scan_bwd(x, dt, A, B, C, D, z, dt_bias, dt_softplus, dt_limit, bou
     if P == 128 and z is not None:
         raise NotImplementedError("hmx SSD backward: the z gate needs headdim 64 (the training "
                                   "layer with its RMSNorm passes z = None)")
-    rows, seqs = _chunk_table(bounds)
+    rows, seqs = _chunk_arrays(tuple(bounds))
     nseq, nrows = len(bounds), len(rows)
     x, B, C = _prep3(x), _prep3(B), _prep3(C)
     z = None if z is None else _prep3(z.to(torch.bfloat16))
@@ -77,8 +89,8 @@ def ssd_chunk_scan_bwd(x, dt, A, B, C, D, z, dt_bias, dt_softplus, dt_limit, bou
     dh0 = torch.empty(nseq, H, P, N, **f32) if want_dh0 and nseq else None
     if d_final is not None:
         d_final = d_final.to(torch.float32).contiguous()
-    seg = _device_table(rows if rows else [(0,) * 8], dev)
-    sq = _device_table(seqs if seqs else [(0, 0)], dev)
+    seg = _device_table(rows if nrows else [(0,) * 8], dev)
+    sq = _device_table(seqs if nseq else [(0, 0)], dev)
     lib = _lib.load()
     ws_bytes = int(lib.hmx_ssd_chunk_bwd_workspace_bytes(nrows, H, P, N))
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)

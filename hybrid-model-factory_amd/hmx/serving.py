@@ -204,11 +204,18 @@ def _by_spec(md, n, rows, core_attn_out, o_norm, run_spec, run_rest):
         core_attn_out.index_copy_(0, idx, out)
 
 
+def _cut(t, lo, hi, dim=0):
+    """t[lo:hi] along ``dim``; t itself when that is all of it."""
+    if lo == 0 and hi == t.shape[dim]:
+        return t
+    return t[lo:hi] if dim == 0 else t[:, lo:hi]
+
+
 def _norm_args(o_norm, lo, hi):
     if o_norm is None:
         return {}
     w, z, eps = o_norm
-    return dict(o_norm_weight=w, o_norm_gate=None if z is None else z[lo:hi].unsqueeze(0),
+    return dict(o_norm_weight=w, o_norm_gate=None if z is None else _cut(z, lo, hi).unsqueeze(0),
                 o_norm_eps=eps)
 
 
@@ -224,7 +231,7 @@ def gdn_forward_core(layer, mixed_qkv: torch.Tensor, b: torch.Tensor, a: torch.T
         return
     _check(layer, md)
     n = md.num_actual_tokens
-    mixed_qkv, b, a = mixed_qkv[:n], b[:n], a[:n]
+    mixed_qkv, b, a = _cut(mixed_qkv, 0, n), _cut(b, 0, n), _cut(a, 0, n)
     beta_scale = 2.0 if getattr(layer, "allow_neg_eigval", False) else 1.0
 
     def rest(rows, out, on, qsl_cpu=None):
@@ -240,17 +247,17 @@ def gdn_forward_core(layer, mixed_qkv: torch.Tensor, b: torch.Tensor, a: torch.T
         if dec is not None:
             cu_d, idx_d = dec
             ops.fused_recurrent_gated_delta_rule_gqa(
-                q[:, :ndt], k[:, :ndt], v[:, :ndt], None, None,
+                _cut(q, 0, ndt, 1), _cut(k, 0, ndt, 1), _cut(v, 0, ndt, 1), None, None,
                 initial_state=ssm_state, inplace_final_state=True, cu_seqlens=cu_d,
-                ssm_state_indices=idx_d, use_qk_l2norm_in_kernel=True, out=o[:, :ndt],
+                ssm_state_indices=idx_d, use_qk_l2norm_in_kernel=True, out=_cut(o, 0, ndt, 1),
                 gates=gates.tokens(0, ndt), **_norm_args(on, 0, ndt))
         if pre is not None:
             cu_p, idx_p, has_p = pre
             ops.chunk_gated_delta_rule_gqa(
-                q[:, ndt:], k[:, ndt:], v[:, ndt:], None, None,
+                _cut(q, ndt, m, 1), _cut(k, ndt, m, 1), _cut(v, ndt, m, 1), None, None,
                 initial_state=ssm_state, output_final_state=True, cu_seqlens=cu_p,
                 use_qk_l2norm_in_kernel=True, ssm_state_indices=idx_p, has_initial_state=has_p,
-                out=o[:, ndt:], gates=gates.tokens(ndt, m), **_norm_args(on, ndt, m))
+                out=_cut(o, ndt, m, 1), gates=gates.tokens(ndt, m), **_norm_args(on, ndt, m))
 
     def spec(rows, out, on):
         mq, aa, bb = rows
@@ -265,7 +272,7 @@ def gdn_forward_core(layer, mixed_qkv: torch.Tensor, b: torch.Tensor, a: torch.T
             out=out.unsqueeze(0), gates=gates, **_norm_args(on, 0, mq.shape[0]))
 
     if md.spec_sequence_masks is None:
-        rest((mixed_qkv, a, b), core_attn_out[:n], o_norm, query_start_loc_cpu)
+        rest((mixed_qkv, a, b), _cut(core_attn_out, 0, n), o_norm, query_start_loc_cpu)
     else:
         _by_spec(md, n, (mixed_qkv, a, b), core_attn_out, o_norm, spec, rest)
 
@@ -282,7 +289,7 @@ def gka_forward_core(layer, mixed_qkv: torch.Tensor, a: torch.Tensor, alpha_in: 
         return
     _check(layer, md)
     n = md.num_actual_tokens
-    mixed_qkv, a, alpha_in = mixed_qkv[:n], a[:n], alpha_in[:n]
+    mixed_qkv, a, alpha_in = _cut(mixed_qkv, 0, n), _cut(a, 0, n), _cut(alpha_in, 0, n)
     use_beta = layer.use_beta_gate
     if use_beta:
         b = b[:n]
@@ -310,17 +317,17 @@ def gka_forward_core(layer, mixed_qkv: torch.Tensor, a: torch.Tensor, alpha_in: 
         if dec is not None:
             cu_d, idx_d = dec
             ops.gka_chebyshev_gla_decode(
-                q[:, :ndt], k[:, :ndt], v[:, :ndt], None, None, None, None,
+                _cut(q, 0, ndt, 1), _cut(k, 0, ndt, 1), _cut(v, 0, ndt, 1), None, None, None, None,
                 h_kk=h_kk_state, h_kv=h_kv_state, cu_seqlens=cu_d, ssm_state_indices=idx_d,
-                out=o[:, :ndt], gates=gates.tokens(0, ndt), **common,
+                out=_cut(o, 0, ndt, 1), gates=gates.tokens(0, ndt), **common,
                 **_norm_args(on, 0, ndt))
         if pre is not None:
             cu_p, idx_p, has_p = pre
             ops.gka_chebyshev_gla_prefill(
-                q[:, ndt:], k[:, ndt:], v[:, ndt:], None, None, None, None,
+                _cut(q, ndt, m, 1), _cut(k, ndt, m, 1), _cut(v, ndt, m, 1), None, None, None, None,
                 h_kk_initial=h_kk_state, h_kv_initial=h_kv_state, output_final_state=True,
                 cu_seqlens=cu_p, ssm_state_indices=idx_p, has_initial_state=has_p,
-                out=o[:, ndt:], gates=gates.tokens(ndt, m), **common, **_norm_args(on, ndt, m))
+                out=_cut(o, ndt, m, 1), gates=gates.tokens(ndt, m), **common, **_norm_args(on, ndt, m))
 
     def spec(rows, out, on):
         mq, aa, ai, bb = rows
