@@ -173,39 +173,14 @@ __device__ __forceinline__ float scan64(float x) {
   return (threadIdx.x & 63) >= 32 ? lo + carry : lo;
 }
 
-// Gate reads: the op's gate tensors, or (fused) the gates formed from the raw
-// projections in gp.  Token tok is the op's flattened token index.
+// The gates come from the op's gate tensors, or (fused) are formed from the raw
+// projections in gp.
 __device__ __forceinline__ bool has_beta(const Params& p) {
   return p.fused ? p.gp.b != nullptr : p.beta != nullptr;
 }
 __device__ __forceinline__ bool has_gk(const Params& p) {
   return p.fused ? p.gp.gk_from_g != 0 : p.gk != nullptr;
 }
-__device__ __forceinline__ float beta_at(const Params& p, int64_t tok, int h) {
-  return p.fused ? gp_beta(p.gp, tok, h) : ldsc(p.beta, tok * p.H + h, p.beta_dt);
-}
-__device__ __forceinline__ float g_at(const Params& p, int64_t tok, int h) {
-  return p.fused ? gp_g(p.gp, tok, h) : ldsc(p.g, tok * p.H + h, p.g_dt);
-}
-__device__ __forceinline__ float gk_at(const Params& p, int64_t tok, int h) {   // has_gk(p)
-  return p.fused ? gp_g(p.gp, tok, h) : ldsc(p.gk, tok * p.H + h, p.gk_dt);
-}
-__device__ __forceinline__ float alpha_at(const Params& p, int64_t tok, int h) {
-  return p.fused ? gp_alpha(p.gp, tok, h) : ldsc(p.alpha, tok * p.H + h, p.alpha_dt);
-}
-
-// The k~ scale of a row: (beta+1e-6) / |k| (or without the norm / without beta).
-__device__ __forceinline__ float key_scale(const Params& p, float ss, int64_t tok, int h, bool ok) {
-  if (!ok) return 0.f;
-  const float be = has_beta(p) ? beta_at(p, tok, h) + EPS : 1.f;
-  return p.l2norm ? be / sqrtf(ss) : be;
-}
-
-__device__ __forceinline__ float beta_eps(const Params& p, int64_t tok, int h, bool ok) {
-  if (!ok) return 0.f;
-  return has_beta(p) ? beta_at(p, tok, h) + EPS : 1.f;
-}
-
 __device__ __forceinline__ f16x8 scale_h8(const bf16x8& x, float s) {
   f16x8 y;
 #pragma unroll
@@ -691,30 +666,38 @@ template <int NT = NTHR> struct StateLd { static constexpr int NPC = 16 * D / NT
 // the decay that decides whether it is needed.
 // SYM (H): only the pieces in upper 16x16 tiles (tile row <= tile column) are
 // loaded; state_fill_lower mirrors the rest in LDS.
+// Buffer loads whose offset masks a piece (past the resource's end: zero, no traffic)
+// rather than branches: a load that may have been skipped cannot be counted, so every
+// wait for an earlier load would wait for the whole state.
 template <bool SYM>
 __device__ __forceinline__ bool piece_kept(int r, int c) {
   return !SYM || (r >> 4) <= (c >> 4);
 }
-template <bool SYM, int NT>
-__device__ __forceinline__ void state_issue_b(StateLd<NT>& L, const f16* xb, int tid) {
-  constexpr int NPC = StateLd<NT>::NPC;
-  const int r = tid / (16 / NPC), c0 = (tid % (16 / NPC)) * 8 * NPC;
-  const f16* xbr = xb ? xb + blk_index(r, c0) : nullptr;   // 8-element pieces: fixed offsets
-#pragma unroll
-  for (int j = 0; j < NPC; ++j)
-    L.b[j] = (xbr && piece_kept<SYM>(r, c0 + 8 * j))
-                 ? *reinterpret_cast<const f16x8*>(xbr + (j >> 1) * 256 + (j & 1) * 8)
-                 : f16x8{};
+constexpr int PIECE_OFF = 1 << 30;        // past any state
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t state_rsrc(const f16* x, const f16* any) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(x ? x : any), 0, x ? D * D * 2 : 0, 0x00020000);
 }
 template <bool SYM, int NT>
-__device__ __forceinline__ void state_issue_s(StateLd<NT>& L, const f16* xs, int tid) {
+__device__ __forceinline__ void state_issue_b(StateLd<NT>& L, const f16* xb, const f16* any, int tid) {
   constexpr int NPC = StateLd<NT>::NPC;
   const int r = tid / (16 / NPC), c0 = (tid % (16 / NPC)) * 8 * NPC;
+  const auto rs = state_rsrc(xb, any);
+  const int o = blk_index(r, c0) * 2;     // 8-element pieces: fixed offsets
 #pragma unroll
   for (int j = 0; j < NPC; ++j)
-    L.s[j] = (xs && piece_kept<SYM>(r, c0 + 8 * j))
-                 ? *reinterpret_cast<const f16x8*>(xs + r * D + c0 + 8 * j)
-                 : f16x8{};
+    L.b[j] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+        rs, piece_kept<SYM>(r, c0 + 8 * j) ? o + ((j >> 1) * 256 + (j & 1) * 8) * 2 : PIECE_OFF, 0, 0));
+}
+template <bool SYM, int NT>
+__device__ __forceinline__ void state_issue_s(StateLd<NT>& L, const f16* xs, const f16* any, int tid) {
+  constexpr int NPC = StateLd<NT>::NPC;
+  const int r = tid / (16 / NPC), c0 = (tid % (16 / NPC)) * 8 * NPC;
+  const auto rs = state_rsrc(xs, any);
+  const int o = (r * D + c0) * 2;
+#pragma unroll
+  for (int j = 0; j < NPC; ++j)
+    L.s[j] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+        rs, piece_kept<SYM>(r, c0 + 8 * j) ? o + 16 * j : PIECE_OFF, 0, 0));
 }
 // A segment's start state enters a block's state decayed by e^{off}; below e^-20
 // (2e-9 of its norm, under fp32 rounding) it is dropped and not loaded.
@@ -776,6 +759,60 @@ __device__ __forceinline__ void with_wave(int wave, F&& f) {
   }
 }
 
+// A gate value as stored, in either width: two 16-bit loads (of an fp32, its halves),
+// so no branch on the type and no conversion that would wait stands at the load.
+struct Raw2 { uint16_t lo, hi; };
+__device__ __forceinline__ Raw2 ld_raw2(const void* x, int64_t i, int dt) {
+  const uint16_t* u = static_cast<const uint16_t*>(x);
+  const bool f32 = dt == HMX_F32;
+  return Raw2{u[f32 ? 2 * i : i], u[f32 ? 2 * i + 1 : i]};
+}
+__device__ __forceinline__ float raw2_f(const Raw2& r, int dt) {
+  const uint32_t lo = r.lo, hi = r.hi;
+  return dt == HMX_F32    ? __builtin_bit_cast(float, lo | (hi << 16))
+         : dt == HMX_BF16 ? __builtin_bit_cast(float, lo << 16)
+                          : (float)__builtin_bit_cast(f16, r.lo);
+}
+// The gates of token tok: beta, g, gk and alpha (fused: b, a, none and alpha_in, with
+// the head's A_log and dt_bias).  An absent one reads p.ws_boff, and is not used.
+struct GateRaw { Raw2 b, g, gk, al, A, dtb; };
+template <bool GLA>
+__device__ __forceinline__ GateRaw load_gates(const Params& p, int64_t tok, int h) {
+  const auto raw = [&](bool have, const void* x, int64_t i, int dt) {
+    return ld_raw2(have ? x : p.ws_boff, have ? i : 0, have ? dt : HMX_F32);
+  };
+  const bool fu = p.fused;
+  const int64_t i = tok * p.H + h;
+  GateRaw r = {};
+  r.b = raw(has_beta(p), fu ? p.gp.b : p.beta, fu ? tok * p.gp.b_token_stride + h * p.gp.b_head_stride : i,
+            fu ? p.gp.in_dtype : p.beta_dt);
+  r.gk = raw(!fu && p.gk, p.gk, i, p.gk_dt);
+  if constexpr (GLA) {
+    const bool fg = fu && p.gp.A_log;
+    r.g = raw(!fu || fg, fu ? p.gp.a : p.g, fu ? tok * p.gp.a_token_stride + h * p.gp.a_head_stride : i,
+              fu ? p.gp.in_dtype : p.g_dt);
+    r.A = raw(fg, p.gp.A_log, h, p.gp.A_log_dtype);
+    r.dtb = raw(fg, p.gp.dt_bias, h, p.gp.dt_bias_dtype);
+    r.al = raw(!fu || !p.gp.alpha_zero, fu ? p.gp.alpha_in : p.alpha,
+               fu ? tok * p.gp.alpha_token_stride + h * p.gp.alpha_head_stride : i,
+               fu ? p.gp.in_dtype : p.alpha_dt);
+  }
+  return r;
+}
+__device__ __forceinline__ float beta_of(const Params& p, const GateRaw& r) {     // beta + 1e-6, or 1
+  if (!has_beta(p)) return 1.f;
+  return (p.fused ? gp_beta_of(p.gp, raw2_f(r.b, p.gp.in_dtype)) : raw2_f(r.b, p.beta_dt)) + EPS;
+}
+__device__ __forceinline__ float g_of(const Params& p, const GateRaw& r) {
+  if (!p.fused) return raw2_f(r.g, p.g_dt);
+  if (!p.gp.A_log) return 0.f;
+  return gp_g_of(p.gp, raw2_f(r.g, p.gp.in_dtype), gate_exp(raw2_f(r.A, p.gp.A_log_dtype)),
+                 raw2_f(r.dtb, p.gp.dt_bias_dtype));
+}
+__device__ __forceinline__ float alpha_of(const Params& p, const GateRaw& r) {
+  return p.fused ? gp_alpha_of(p.gp, raw2_f(r.al, p.gp.in_dtype)) : raw2_f(r.al, p.alpha_dt);
+}
+
 // What the solve kernel produces: the GLA output (serving prefill), or the solution
 // x of the Chebyshev solve itself (training): SM_X writes x (bf16, into p.o) and
 // |H_t|_F; SM_DQ solves for the right-hand side in p.q with the |H_t|_F of the
@@ -804,6 +841,9 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
   const int64_t DD = (int64_t)D * D;
 
   // ---- which segment / block -------------------------------------------------
+  // block-start decay offsets (segment start -> this block)
+  const int64_t bo = ((int64_t)gb * H + h) * 2;
+  const float off_gk = p.ws_boff[bo + 0], off_g = p.ws_boff[bo + 1];
   const int s_id = segment_of(p, gb, lane);
   const SegInfo si = load_seg(p.seg, s_id);
   const int lb = gb - p.segblk[s_id];                 // block index within the segment
@@ -811,78 +851,122 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
   const int nval = min(CB, si.eos - tok0);
   if (nval <= 0) return;
 
-  // block-start decay offsets (segment start -> this block); the state loads go
-  // out first so their latency overlaps the staging below
-  const int64_t bo = ((int64_t)gb * H + h) * 2;
+  // ---- every load of the block, in the order of use -------------------------------
+  // Held as loaded: a conversion, a norm or a gate formed at its load would wait there
+  // for all loads before it.  Rows past the block's tokens load its last one; they
+  // are zeroed where they are staged.  Loaded where each was used, four rows of k and v
+  // and their beta at a time, then q, then h_c, a block waited 36 of its 79 thousand
+  // cycles (8 iterations; of 168 with 30) before its first step, a third of it for
+  // memory four times over; now h_c, v and q arrive under the staging of k~ and the
+  // Gram products.  32768 tokens, H = 32, 30 iterations: 3.13 -> 3.06 ms; a training
+  // step at 8 x 4096 tokens, 8 iterations, which solves twice: 5.76 -> 5.27.
+  const bool lane_ok = lane < nval;       // the gates are those of token `lane`
+  const GateRaw gr = load_gates<GLA>(p, tok0 + min(lane, nval - 1), h);
+  bf16x8 kr[CB / 16], vr[GLA ? CB / 16 : 1];
+  const auto row_at = [&](int pass) { return pass * 16 + (tid >> 4); };
+  const int f0 = (tid & 15) * 8;
+#pragma unroll
+  for (int pass = 0; pass < CB / 16; ++pass)
+    kr[pass] = *reinterpret_cast<const bf16x8*>(p.k + (int64_t)(tok0 + min(row_at(pass), nval - 1)) * p.kv_ts +
+                                                hk * D + f0);
   const int64_t so = ((int64_t)s_id * H + h) * DD;
   const int64_t bso = ((int64_t)gb * H + h) * DD;
   StateLd<> hst;
-  if constexpr (SOLVE) state_issue_b<true>(hst, lb > 0 ? p.ws_hb + bso : nullptr, tid);
-  const float off_gk = p.ws_boff[bo + 0], off_g = p.ws_boff[bo + 1];
-  if constexpr (SOLVE)
-    state_issue_s<true>(hst, (lb == 0 || off_gk > SEG_STATE_DROP) ? p.ws_h0 + so : nullptr, tid);
-
-  // ---- stage k~, v~ (fp16), gates; q rows into registers --------------------
-#pragma unroll
-  for (int pass = 0; pass < CB / 16; ++pass) {
-    const int row = pass * 16 + (tid >> 4), f0 = (tid & 15) * 8;
-    const bool ok = row < nval;
-    const int64_t tok = tok0 + row;
-    const bf16x8 kr = ok ? *reinterpret_cast<const bf16x8*>(p.k + tok * p.kv_ts + hk * D + f0) : bf16x8{};
-    const bf16x8 vr = ok ? *reinterpret_cast<const bf16x8*>(p.v + tok * p.kv_ts + hk * D + f0) : bf16x8{};
-    const float sk = key_scale(p, row_sumsq(kr), tok, h, ok);
-    store8_i(sK + row * LDP, f0, scale_h8(kr, sk));
-    if constexpr (GLA)
-      *reinterpret_cast<f16x8*>(sV + row * LDP + f0) = scale_h8(vr, beta_eps(p, tok, h, ok));
-  }
-  if (wave == 0) {
-    const bool ok = lane < nval;
-    const int64_t tk = tok0 + lane;
-    const float gt = (GLA && ok) ? g_at(p, tk, h) : 0.f;
-    const float G = scan64(gt);
-    const float Gk = scan64((ok && has_gk(p)) ? (p.fused ? gt : gk_at(p, tk, h)) : 0.f);
-    SC(SC_G, lane) = G;
-    SC(SC_GK, lane) = Gk;
-    SC(SC_AL, lane) = (GLA && ok) ? alpha_at(p, tk, h) : 0.f;
-  }
-  if (NORM && tid < D) {
-    float wv;
-    if (p.onw_dt == HMX_F32) wv = static_cast<const float*>(p.onw)[tid];
-    else if (p.onw_dt == HMX_BF16) wv = (float)static_cast<const bf16*>(p.onw)[tid];
-    else wv = (float)static_cast<const f16*>(p.onw)[tid];
-    reinterpret_cast<float*>(smem + OFF_NW)[tid] = wv;
-  }
-  float* red = sc + SC_HN * CB;           // 4 partial sums
   if constexpr (SOLVE) {
-    const float ss = wave_sum_v(state_store<true>(sH, hst, fast_exp(off_gk), tid));
-    if (lane == 0) red[wave] = ss;
+    state_issue_b<true>(hst, lb > 0 ? p.ws_hb + bso : nullptr, p.ws_hb, tid);
+    state_issue_s<true>(hst, (lb == 0 || off_gk > SEG_STATE_DROP) ? p.ws_h0 + so : nullptr, p.ws_h0, tid);
+  }
+  if constexpr (GLA) {
+#pragma unroll
+    for (int pass = 0; pass < CB / 16; ++pass)
+      vr[pass] = *reinterpret_cast<const bf16x8*>(p.v + (int64_t)(tok0 + min(row_at(pass), nval - 1)) * p.kv_ts +
+                                                  hk * D + f0);
   }
   // this lane's token t (16 per wave) and its q^ slice: Q[nt][v] = q^[t][16 nt + 4 q4 + v]
   const int tb = 16 * wave + l16;
   const bool tok_ok = tb < nval;
+  const int64_t tkb = tok0 + min(tb, nval - 1);
   f32x4 Q[8];
   [[maybe_unused]] f32x4 Du[MODE == SM_DQ ? 8 : 1];
-  const float al_dq = (MODE == SM_DQ && p.du32 && tok_ok)
-                          ? ldsc(p.alpha, (int64_t)(tok0 + tb) * H + h, p.alpha_dt) : 0.f;
-  const bf16* qr = p.q + (int64_t)(tok0 + tb) * p.q_ts + (int64_t)h * D + 4 * q4;
-  float rq;
+  [[maybe_unused]] float f_dq = 0.f, al_dq = 0.f;
+  const bf16* qr = p.q + tkb * p.q_ts + (int64_t)h * D + 4 * q4;
+  bf16x4 qraw[8];
+  const bool from_du = MODE == SM_DQ && p.du32;
+  if (!from_du) {
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) qraw[nt] = *reinterpret_cast<const bf16x4*>(qr + 16 * nt);
+  }
+  if constexpr (MODE == SM_DQ) {
+    f_dq = p.fro[tkb * H + h];
+    if (from_du) {
+#pragma unroll
+      for (int nt = 0; nt < 8; ++nt)
+        Du[nt] = *reinterpret_cast<const f32x4*>(p.du32 + (tkb * H + h) * D + 4 * q4 + 16 * nt);
+      al_dq = ldsc(p.alpha, tkb * H + h, p.alpha_dt);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- stage k~ (fp16) and the gates' sums -----------------------------------------
+  // k~, v~ scales: be = beta + 1e-6 of token `lane` (1 without beta), handed to the rows'
+  // lanes by a lane permute
+  float be[CB / 16];
   {
+    const float x = beta_of(p, gr);
+#pragma unroll
+    for (int pass = 0; pass < CB / 16; ++pass) {
+      be[pass] = __builtin_bit_cast(
+          float, __builtin_amdgcn_ds_bpermute(row_at(pass) << 2, __builtin_bit_cast(int, x)));
+      // not to be moved under a row's condition: a permute reads 0 from a masked lane
+      asm volatile("" : "+v"(be[pass]));
+    }
+  }
+#pragma unroll
+  for (int pass = 0; pass < CB / 16; ++pass) {
+    const int row = row_at(pass);
+    const float ss = row_sumsq(kr[pass]);
+    const float sk = p.l2norm ? be[pass] / sqrtf(ss) : be[pass];
+    store8_i(sK + row * LDP, f0, row < nval ? scale_h8(kr[pass], sk) : f16x8{});
+  }
+  if (wave == 0) {
+    const float gt = (GLA && lane_ok) ? g_of(p, gr) : 0.f;
+    const float G = scan64(gt);
+    const float Gk = scan64((lane_ok && has_gk(p)) ? (p.fused ? gt : raw2_f(gr.gk, p.gk_dt)) : 0.f);
+    SC(SC_G, lane) = G;
+    SC(SC_GK, lane) = Gk;
+    SC(SC_AL, lane) = (GLA && lane_ok) ? alpha_of(p, gr) : 0.f;
+  }
+  const auto stage_v = [&]() {
+    if constexpr (GLA) {
+#pragma unroll
+      for (int pass = 0; pass < CB / 16; ++pass) {
+        const int row = row_at(pass);
+        *reinterpret_cast<f16x8*>(sV + row * LDP + f0) =
+            row < nval ? scale_h8(vr[pass], be[pass]) : f16x8{};
+      }
+    }
+    if (NORM && tid < D) {
+      float wv;
+      if (p.onw_dt == HMX_F32) wv = static_cast<const float*>(p.onw)[tid];
+      else if (p.onw_dt == HMX_BF16) wv = (float)static_cast<const bf16*>(p.onw)[tid];
+      else wv = (float)static_cast<const f16*>(p.onw)[tid];
+      reinterpret_cast<float*>(smem + OFF_NW)[tid] = wv;
+    }
+  };
+  float rq;
+  const auto form_q = [&]() {
     float ss = 0.f;
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt) {
-      if constexpr (MODE == SM_DQ) Du[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (MODE == SM_DQ && p.du32) {
-        if (tok_ok)
-          Du[nt] = *reinterpret_cast<const f32x4*>(p.du32 + ((int64_t)(tok0 + tb) * H + h) * D +
-                                                   4 * q4 + 16 * nt);
-        Q[nt] = Du[nt] * al_dq;
-      } else {
-        const bf16x4 x = tok_ok ? *reinterpret_cast<const bf16x4*>(qr + 16 * nt) : bf16x4{};
-#pragma unroll
-        for (int v = 0; v < 4; ++v) Q[nt][v] = (float)x[v];
+      if constexpr (MODE == SM_DQ) {
+        if (!from_du || !tok_ok) Du[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
 #pragma unroll
-      for (int v = 0; v < 4; ++v) ss += Q[nt][v] * Q[nt][v];
+      for (int v = 0; v < 4; ++v) {
+        if (from_du) Q[nt][v] = Du[MODE == SM_DQ ? nt : 0][v] * al_dq;
+        else Q[nt][v] = tok_ok ? (float)qraw[nt][v] : 0.f;
+        ss += Q[nt][v] * Q[nt][v];
+      }
     }
     ss = q4_sum(ss);
     rq = (!tok_ok) ? 0.f : (p.l2norm ? 1.0f / sqrtf(ss) : 1.f);
@@ -890,15 +974,84 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
     for (int nt = 0; nt < 8; ++nt)
 #pragma unroll
       for (int v = 0; v < 4; ++v) Q[nt][v] *= rq;
-  }
+  };
 
+  StateLd<> sst;
+  const auto issue_s = [&]() {
+    state_issue_b<false>(sst, lb > 0 ? p.ws_sb + bso : nullptr, p.ws_hb, tid);
+    state_issue_s<false>(sst, (lb == 0 || off_g > SEG_STATE_DROP) ? p.ws_s0 + so : nullptr, p.ws_h0, tid);
+  };
   f32x4 X[8];                             // the query fed to the GLA, transposed C layout
   if constexpr (SOLVE) {
+    float* red = sc + SC_HN * CB;           // 4 partial sums
+    // in-block decays m_tj = e^{Gk_t-Gk_j} (j <= t, else 0) of this lane's token, key tile jt
+    f32x4 mz[4];
+    float GkT;
+    const auto decays = [&]() {
+      GkT = SC(SC_GK, tb);
+#pragma unroll
+      for (int jt = 0; jt < 4; ++jt) {
+        const f32x4 gkj = *reinterpret_cast<const f32x4*>(&SC(SC_GK, 16 * jt + 4 * q4));
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float e = fast_exp(GkT - gkj[v]);
+          mz[jt][v] = (16 * jt + 4 * q4 + v <= tb) ? e : 0.f;
+        }
+      }
+    };
+    // Gram part of |H_t|^2: g2_t = sum_{i,j<=t} m_ti m_tj (k~_i.k~_j)^2 as the column sums of
+    // m^T . (B m^T) with B = (K K^T)^2 over this wave's key range, while h_c, v and q arrive
+    float g2 = 0.f;
+    if constexpr (MODE != SM_DQ) {
+      lds_barrier();
+      decays();
+      with_wave(wave, [&](auto Wc) {
+        constexpr int W = decltype(Wc)::value;
+        f32x4 U[W + 1];
+#pragma unroll
+        for (int I = 0; I <= W; ++I) U[I] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int J = 0; J <= W; ++J) {
+          f32x4 kk[W + 1];
+#pragma unroll
+          for (int I = 0; I <= W; ++I) kk[I] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) {
+            const f16x8 aj = frag_i(sK, LDP, 16 * J, 32 * ks, lane);
+#pragma unroll
+            for (int I = 0; I <= W; ++I)
+              kk[I] = mfma16h(aj, I == J ? aj : frag_i(sK, LDP, 16 * I, 32 * ks, lane), kk[I]);
+          }
+#pragma unroll
+          for (int I = 0; I <= W; ++I) {
+            f32x4 sq;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sq[v] = kk[I][v] * kk[I][v];
+            // U[I][v]: row i = 16 I + 4 q4 + v, column t = tb
+            U[I] = mfma16h_k16(h4(sq), h4(mz[J]), U[I]);
+          }
+          __builtin_amdgcn_sched_barrier(0);   // one J's operands at a time
+        }
+#pragma unroll
+        for (int I = 0; I <= W; ++I)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            g2 += (I < W || 4 * q4 + v <= l16) ? U[I][v] * mz[I][v] : 0.f;
+      });
+      g2 = q4_sum(g2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    {
+      const float ss = wave_sum_v(state_store<true>(sH, hst, fast_exp(off_gk), tid));
+      if (lane == 0) red[wave] = ss;
+    }
+    stage_v();
+    form_q();
     lds_barrier();
     state_fill_lower(sH, wave, lane);
     lds_barrier();
     const float hn = red[0] + red[1] + red[2] + red[3];   // |H_c|^2
-    const float GkT = SC(SC_GK, tb);
+    if constexpr (MODE == SM_DQ) decays();
 
     // d_j = k~_j^T H_c k~_j for this wave's tokens j = 16 wave + l16
     if constexpr (MODE != SM_DQ) {
@@ -920,75 +1073,26 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
       }
       d = q4_sum(d);
       if (q4 == 0) SC(SC_D, tb) = d;
+      lds_barrier();
     }
-    // Gram part of |H_t|^2: g2_t = sum_{i,j<=t} a_ti a_tj (k~_i.k~_j)^2, a_tj = e^{Gk_t-Gk_j},
-    // as the row sums of a . (A B) with B = (K K^T)^2 over this wave's key range
-    if constexpr (MODE != SM_DQ) with_wave(wave, [&](auto Wc) {
-      constexpr int W = decltype(Wc)::value;
-      f32x4 U[4];
-#pragma unroll
-      for (int I = 0; I < 4; ++I) U[I] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int J = 0; J < 4; ++J) {
-        if (J > W) break;
-        // a[t = tb][j = 16J + 4q4 + v]
-        f16x4 aJ;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int j = 16 * J + 4 * q4 + v;
-          aJ[v] = (f16)(j <= tb ? fast_exp(GkT - SC(SC_GK, j)) : 0.f);
-        }
-#pragma unroll
-        for (int I = 0; I < 4; ++I) {
-          if (I > W) break;
-          f32x4 kk = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < 4; ++ks)
-            kk = mfma16h(frag_i(sK, LDP, 16 * J, 32 * ks, lane), frag_i(sK, LDP, 16 * I, 32 * ks, lane), kk);
-          f32x4 sq;
-#pragma unroll
-          for (int v = 0; v < 4; ++v) sq[v] = kk[v] * kk[v];
-          U[I] = mfma16h_k16(aJ, h4(sq), U[I]);
-        }
-      }
-      // U[I][v]: row t = 16 wave + 4 q4 + v, column i = 16 I + l16
-      float g2[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int I = 0; I < 4; ++I) {
-        if (I > W) break;
-        const int i = 16 * I + l16;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int t = 16 * W + 4 * q4 + v;
-          g2[v] += (i <= t) ? U[I][v] * fast_exp(SC(SC_GK, t) - SC(SC_GK, i)) : 0.f;
-        }
-      }
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float s = row16_sum(g2[v]);
-        if (l16 == 0) SC(SC_G2, 16 * W + 4 * q4 + v) = s;
-      }
-    });
-    lds_barrier();
     // f_t, lam, tau, c for this lane's token
     float tau, lam, cc;
     {
       float f;
       if constexpr (MODE == SM_DQ) {
-        f = tok_ok ? p.fro[(int64_t)(tok0 + tb) * H + h] : 0.f;
+        f = tok_ok ? f_dq : 0.f;
       } else {
         float cross = 0.f;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
-          const f32x4 gkj = *reinterpret_cast<const f32x4*>(&SC(SC_GK, 16 * jt + 4 * q4));
           const f32x4 dj = *reinterpret_cast<const f32x4*>(&SC(SC_D, 16 * jt + 4 * q4));
 #pragma unroll
           for (int v = 0; v < 4; ++v)
-            cross += (16 * jt + 4 * q4 + v <= tb) ? fast_exp(GkT - gkj[v]) * dj[v] : 0.f;
+            cross += (16 * jt + 4 * q4 + v <= tb) ? mz[jt][v] * dj[v] : 0.f;
         }
         cross = q4_sum(cross);
         const float e = fast_exp(GkT);
-        f = sqrtf(fmaxf(e * e * hn + 2.f * e * cross + SC(SC_G2, tb), 0.f));
+        f = sqrtf(fmaxf(e * e * hn + 2.f * e * cross + g2, 0.f));
         if ((MODE == SM_X || MODE == SM_GLA_SAVE) && tok_ok && q4 == 0)
           p.fro[(int64_t)(tok0 + tb) * H + h] = f;
       }
@@ -1022,15 +1126,8 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
         X[nt][v] = Dd[nt][v];
         R[nt][v] = Q[nt][v];
       }
-    // minus the in-block decays -m_tj = -e^{Gk_t-Gk_j} (j <= t, else 0) of the four key tiles
-    f32x4 mz[4];
 #pragma unroll
-    for (int jt = 0; jt < 4; ++jt) {
-      const f32x4 gkj = *reinterpret_cast<const f32x4*>(&SC(SC_GK, 16 * jt + 4 * q4));
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        mz[jt][v] = (16 * jt + 4 * q4 + v <= tb) ? -fast_exp(GkT - gkj[v]) : 0.f;
-    }
+    for (int jt = 0; jt < 4; ++jt) mz[jt] = -mz[jt];
     const float egk = fast_exp(GkT);
     // R <- R - A d: R - lam d - e^{Gk_t} H_c d first, then the in-block part
     // accumulates on top through -Z~ (eight 16-row tiles in two groups of four, four
@@ -1270,30 +1367,33 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
     }
       if constexpr (!GLA) return;
     }
-    // alpha blend (q read again: the iterations keep x, d and rho in registers)
+    // alpha blend (q read again: the iterations keep x, d and rho in registers); the S_c
+    // loads go out behind q's
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) qraw[nt] = *reinterpret_cast<const bf16x4*>(qr + 16 * nt);
+    issue_s();
+    __builtin_amdgcn_sched_barrier(0);
     const float al = SC(SC_AL, tb);
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt) {
-      const bf16x4 xq = tok_ok ? *reinterpret_cast<const bf16x4*>(qr + 16 * nt) : bf16x4{};
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const float qv = (float)xq[v] * rq;
+        const float qv = tok_ok ? (float)qraw[nt][v] * rq : 0.f;
         X[nt][v] = qv + al * (X[nt][v] - qv);
       }
     }
     lds_barrier();      // every wave is done with H_c
   } else {
+    stage_v();
+    form_q();
+    issue_s();
+    lds_barrier();       // the staged k~, v~ and gates
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt) X[nt] = Q[nt];
   }
 
   // ---- GLA output: o^T = scale [e^{G_t} S_c^T x^ + V~^T Z'^T] ---------------
-  // The S_c loads go out first; the in-block products (they need only k~) run while
-  // they arrive.
-  StateLd<> sst;
-  state_issue_b<false>(sst, lb > 0 ? p.ws_sb + bso : nullptr, tid);
-  state_issue_s<false>(sst, (lb == 0 || off_g > SEG_STATE_DROP) ? p.ws_s0 + so : nullptr, tid);
-  if constexpr (!SOLVE) lds_barrier();     // the staged k~, v~ and gates
+  // The in-block products (they need only k~) run while S_c arrives.
   f32x4 O[8];
   {
     f16x8 xh[4], xl[4];
@@ -1318,12 +1418,14 @@ __global__ __launch_bounds__(NTHR, 2) void gka_solve_kernel(Params p) {
         for (int jt = 0; jt <= W; ++jt) Z[jt] = mfma16h(a[jt], xl[ks], Z[jt]);
       }
 #pragma unroll
-      for (int jt = 0; jt <= W; ++jt)
+      for (int jt = 0; jt <= W; ++jt) {
+        const f32x4 gj = *reinterpret_cast<const f32x4*>(&SC(SC_G, 16 * jt + 4 * q4));
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int j = 16 * jt + 4 * q4 + v;
-          Z[jt][v] = (j <= tb) ? Z[jt][v] * fast_exp(GT - SC(SC_G, j)) : 0.f;
+          const float e = fast_exp(GT - gj[v]);
+          Z[jt][v] = (16 * jt + 4 * q4 + v <= tb) ? Z[jt][v] * e : 0.f;
         }
+      }
       zb0 = h8(Z[0], Z[1]);
       if constexpr (W >= 2) zb1 = h8(Z[2], Z[3]);
     });
@@ -1664,7 +1766,7 @@ __global__ __launch_bounds__(C_NTHR, 2) void cheb_dk_kernel(Params p, Bwd w) {
   const int64_t so = ((int64_t)b.s_id * H + h) * DD;
   const int64_t bso = ((int64_t)gb * H + h) * DD;
   StateLd<C_NTHR> hst;
-  solve::state_issue_b<true>(hst, b.lb > 0 ? p.ws_hb + bso : nullptr, tid);
+  solve::state_issue_b<true>(hst, b.lb > 0 ? p.ws_hb + bso : nullptr, p.ws_hb, tid);
   const float off_gk = p.ws_boff[((int64_t)gb * H + h) * 2];
   // Dn: wave w's tile row w, column j (rows 16 w + l16, columns 16 j + 4 q4 ..)
   bf16x4 dn[8];
@@ -1688,7 +1790,7 @@ __global__ __launch_bounds__(C_NTHR, 2) void cheb_dk_kernel(Params p, Bwd w) {
   }
   const float fro = s_ok ? w.fro[ts] : 0.f;
   const float g_l = wave == 0 ? block_decay(p, b, h, lane) : 0.f;
-  solve::state_issue_s<true>(hst, (b.lb == 0 || off_gk > solve::SEG_STATE_DROP) ? p.ws_h0 + so : nullptr, tid);
+  solve::state_issue_s<true>(hst, (b.lb == 0 || off_gk > solve::SEG_STATE_DROP) ? p.ws_h0 + so : nullptr, p.ws_h0, tid);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     dk0[i] = (s_ok && w.dk_add) ? *reinterpret_cast<const f32x4*>(w.dk_add + ro + 16 * i)
@@ -2067,7 +2169,7 @@ __global__ __launch_bounds__(GB_NTHR, 2) void gla_bwd_kernel(Params p, GlaBwd w)
   const int64_t so = ((int64_t)b.s_id * H + h) * DD;
   const int64_t bso = ((int64_t)gb * H + h) * DD;
   StateLd<GB_NTHR> sst;
-  solve::state_issue_b<false>(sst, b.lb > 0 ? p.ws_sb + bso : nullptr, tid);
+  solve::state_issue_b<false>(sst, b.lb > 0 ? p.ws_sb + bso : nullptr, p.ws_hb, tid);
   const float off_g = p.ws_boff[((int64_t)gb * H + h) * 2 + 1];
   // dSn: wave w's tile row w, column j (rows K = 16 w + l16, columns V = 16 j + 4 q4 ..)
   bf16x4 dsn[8];
@@ -2092,7 +2194,7 @@ __global__ __launch_bounds__(GB_NTHR, 2) void gla_bwd_kernel(Params p, GlaBwd w)
   }
   const float al = s_ok ? gla_alpha(w, ti) : 0.f;
   const float g_l = (wave == 0 && lane < b.nval) ? ldsc(p.g, (int64_t)(b.tok0 + lane) * H + h, p.g_dt) : 0.f;
-  solve::state_issue_s<false>(sst, (b.lb == 0 || off_g > solve::SEG_STATE_DROP) ? p.ws_s0 + so : nullptr, tid);
+  solve::state_issue_s<false>(sst, (b.lb == 0 || off_g > solve::SEG_STATE_DROP) ? p.ws_s0 + so : nullptr, p.ws_h0, tid);
 
   // ---- staging: k, v (fp16 as given), do, u and dSn (scaled), S_c as the solve forms it
   if (wave == 0) SC(GS_G, lane) = scan64(g_l);
