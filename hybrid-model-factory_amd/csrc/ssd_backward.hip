@@ -27,15 +27,11 @@
 // oracle/ssd.py; mamba_ssm's backward (un-vendored) computes the same gradients
 // with its own kernels (training/.../layers/mamba/mamba2.py:555-580 calls it).
 //
-// Three launches over 64-token chunks (rows of a segment table, one chunk each):
-//   ssd_bwd_local_kernel  (chunk, C group's heads in turn; chunk, head at headdim
-//                          128): the chunk's zero-start end state
-//                          sum_s e^{A_L - A_s} dt'_s x_s B_s^T, its share
-//                          sum_t e^{A_t} g_t C_t^T of dS0, and e^{A_L}
-//   ssd_bwd_scan_kernel   (sequence, head, 1024 state elements): the forward chain
-//                          S0(c+1) = e^{A_L(c)} S0(c) + local(c) gives every chunk's
-//                          start state, the reverse chain dS1 of every chunk and dS0
-//                          of the sequence's start
+// Launches over 64-token chunks (rows of a segment table, one chunk each):
+//   ssd_bwd_states_kernel (block of rows, direction, head, 64 state rows): every chunk's
+//                          start state S0 and end-state gradient dS1, and dS0 of the
+//                          sequences' starts; before it, where rows are cut into several
+//                          blocks, once more for the blocks' totals
 //   ssd_bwd_group_kernel  (chunk, C group): everything else, for the group's heads
 //                          in turn, the next head's inputs loading into registers
 //                          during the current head's products; where B and C are
@@ -45,6 +41,7 @@
 // x shared by several heads (HX < H), or B shared wider than a C group, accumulate
 // with fp32 atomics; everything else is stored.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -71,11 +68,10 @@ struct Params {
   const int* seg;                            // [nrows][8] segment rows (one chunk each)
   const int* seqs;                           // [nseq][2]: first row, rows
   int nrows, nseq;
-  bf16* loc;                                 // ws [nrows][H][P][N]: dS0 shares
-  bf16* sloc;                                // ws [nrows][H][P][N]: zero-start end states
-  float* edec;                               // ws [nrows][H]: e^{A_L}
   bf16* S0;                                  // ws [nrows][H][P][N]: chunk start states
   bf16* dS1;                                 // ws [nrows][H][P][N]: end-state gradients
+  float* tot;                                // ws [2][blocks][H][P][N]: the states launch's
+  float* tdec;                               // ws [2][blocks][H]: block totals and decays
   // outputs (contiguous)
   void* dx;    int x_shared;                 // [T][HX][P]
   void* dB;    int b_shared;                 // [T][G][N]
@@ -150,241 +146,312 @@ __device__ __forceinline__ Tok token_scalars(const Params& p, int h, int tok0, i
   return token_scalars_raw(p, h, d, nval, lane);
 }
 
-// ---------------------------------------------------------------------------
-// local: sloc[r][h] = sum_s dt'_s e^{A_L - A_s} x_s B_s^T, loc[r][h] = sum_t e^{A_t}
-// g_t C_t^T (P x N each, stored in bf16: the scans accumulate them in fp32),
-// edec[r][h] = e^{A_L}
-// ---------------------------------------------------------------------------
-template <int P, int N>
-constexpr int local_lds_bytes() { return 2 * L * (P + 8) * 2 + 2 * L * (N + 8) * 2 + 2 * L * 4; }
+constexpr int row_ld(int w) { return w == 64 ? w + 8 : w + 16; }
 
-template <int P, int N>
-__global__ __launch_bounds__(NTHR) void ssd_bwd_local_kernel(Params p) {
-  constexpr int LDX = P + 8, LDB = N + 8;
-  constexpr int VX = L * P / 8 / NTHR, VB = L * N / 8 / NTHR;
-  extern __shared__ __align__(16) unsigned char lsm[];
-  bf16* sG = reinterpret_cast<bf16*>(lsm);                     // e^{A_t} g_t       [L][LDX]
-  bf16* sXW = sG + L * LDX;                                    // dt'_s e^{A_L-A_s} x_s
-  bf16* sC = sXW + L * LDX;                                    // [L][LDB]
-  bf16* sB = sC + L * LDB;
-  float* sEA = reinterpret_cast<float*>(sB + L * LDB);
-  float* sWT = sEA + L;
+// ---------------------------------------------------------------------------
+// states: every chunk's start state S0 and the gradient dS1 of its end state, one chain
+// over the chunks in either direction (dir 0: S0(c+1) = e^{A_L} S0(c) + sum_s dt'_s
+// e^{A_L - A_s} x_s B_s^T, forward; dir 1: dS1(c-1) = e^{A_L} dS1(c) + sum_t e^{A_t} g_t C_t^T,
+// backward), held in fp32 MFMA accumulators; each chunk's state is stored in bf16 before
+// the chunk is added.
+//
+// One workgroup per (block of Lr table rows, direction, head, 64 state rows), eight waves.
+// A row that begins its sequence (ends it, backward) resets the chain to h0 (dT), so a
+// block may hold several sequences.  Where a sequence crosses blocks, a launch before
+// this one (TOT) has left each block's contribution and decay, and the chain starts from
+// their sum over the sequence's blocks before it: two reads of x, dy, B and C in place of
+// one, so blocks are cut only to fill the chip (see launch).
+// What bounds it: memory, and the path to it.  Each chunk's terms as a launch of their
+// own, then a scan over them, moved every state through memory twice more than this (a
+// chunk's share written, read, its state written): 0.40 + 0.43 ms at 2 x 16384 tokens,
+// H = 64, P = 64, N = 128, G = 8, where these chains take 0.49 (1.07 GB written, 0.67 GB
+// read: 0.35 at the rate of a copy).  64 state rows per workgroup: with 32, two workgroups
+// per CU load and stage every B and C row twice as often, 0.59 ms there.  (0.31 without
+// the stores, 0.41 with cached inputs.)
+// The loads of SD chunks are in flight; the LDS tiles alternate, one barrier per chunk;
+// the scalar chain over a chunk's tokens runs in one wave of four, four chunks at a time.
+// LDS: B's (C's) features in the order pos(n) = 32-block | bit 2 of n | bits 4,3 | bits 1,0,
+// so that the two 16-row tiles of a 32-feature block leave 8 consecutive features of a
+// state row in each lane (one 16-byte store) and the transposing reads stay contiguous.
+// ---------------------------------------------------------------------------
+constexpr int SP = 64;                    // state rows per workgroup
+constexpr int STHR = 512;
+constexpr int SD = 4;                     // chunks in flight
+
+template <int N>
+struct SLay {
+  static constexpr int LDB = row_ld(N), LDX = SP + 16;      // rows 72 (36) and 40 dwords apart
+  static constexpr int SZ_B = L * LDB, SET = SZ_B + L * LDX;   // elements
+  static constexpr int SW = L + 4;                          // a chunk's weights and its decay
+};
+
+// One chunk's inputs in flight.
+template <int N>
+struct StateIn {
+  bf16x8 m[L * N / 8 / STHR], x, z;
+  int nval, fl, n, r;                     // tokens, row begins (1) / ends (2) a sequence, its n, row
+};
+
+template <int P, int N, bool TOT>
+__global__ __launch_bounds__(STHR, 2) void ssd_bwd_states_kernel(Params p, int Lr, int nblk) {
+  using Y = SLay<N>;
+  constexpr int VB = L * N / 8 / STHR, TPR = N / 8;          // 16-byte pieces of a B row
+  constexpr int NB = N / 32, PBW = N / 64;                   // 32-feature blocks; p tiles per wave
+  __shared__ __align__(16) bf16 lds[2 * Y::SET];
+  __shared__ __align__(16) float sW[8 * Y::SW];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q4 = lane >> 4, l16 = lane & 15;
-  const int H = p.H, GC = p.GC, HC = H / GC, HB = H / p.G, HXS = H / p.HX;
-  // headdim 64: one workgroup per (chunk, C group), C staged once (B too when its
-  // groups are C's), the group's heads in turn with the next one's rows loading
-  // into registers during the current one's products.  Headdim 128: one workgroup
-  // per (chunk, head) (the rows of a second head would not fit in registers).
-  constexpr bool AHEAD = P == 64;
-  const int per_row = AHEAD ? GC : H, nh = AHEAD ? HC : 1;
-  const int r = blockIdx.x / per_row;
-  const int h_first = AHEAD ? (blockIdx.x % per_row) * HC : blockIdx.x % per_row;
-  const int gc = h_first / HC;
-  const Row ro = load_row(p.seg, r);
-  const int tok0 = ro.bos, nval = ro.eos - ro.bos;
-  const bool b_once = AHEAD && p.G == GC;
-#pragma unroll
-  for (int i = 0; i < VB; ++i) {
-    const int e = (i * NTHR + tid) * 8, t = e / N, c = e % N;
-    bf16x8 cv = {}, bv = {};
-    if (t < nval) {
-      cv = *reinterpret_cast<const bf16x8*>(p.C + (int64_t)(tok0 + t) * p.c_ts + (int64_t)gc * p.c_gs + c);
-      if (b_once)
-        bv = *reinterpret_cast<const bf16x8*>(p.B + (int64_t)(tok0 + t) * p.b_ts +
-                                              (int64_t)(h_first / HB) * p.b_gs + c);
-    }
-    *reinterpret_cast<bf16x8*>(sC + t * LDB + c) = cv;
-    if (b_once) *reinterpret_cast<bf16x8*>(sB + t * LDB + c) = bv;
-  }
-  constexpr int VZ = P == 64 ? VX : 1;
-  struct In { bf16x8 x[VX], dy[VX], z[VZ], b[VB]; uint32_t dt; };
-  const auto fetch = [&](int h, In& q) {
-    const int hx = h / HXS, g = h / HB;
-#pragma unroll
-    for (int i = 0; i < VX; ++i) {
-      const int e = (i * NTHR + tid) * 8, t = e / P, c = e % P;
-      q.x[i] = q.dy[i] = bf16x8{};
-      if constexpr (P == 64) q.z[i] = bf16x8{};
-      if (t < nval) {
-        q.dy[i] = *reinterpret_cast<const bf16x8*>(p.dy + (int64_t)(tok0 + t) * p.dy_ts + (int64_t)h * p.dy_hs + c);
-        q.x[i] = *reinterpret_cast<const bf16x8*>(p.x + (int64_t)(tok0 + t) * p.x_ts + (int64_t)hx * p.x_hs + c);
-        if constexpr (P == 64) {
-          if (p.z) q.z[i] = *reinterpret_cast<const bf16x8*>(p.z + (int64_t)(tok0 + t) * p.z_ts + (int64_t)h * p.z_hs + c);
-        }
-      }
-    }
-    if (!b_once) {
-#pragma unroll
-      for (int i = 0; i < VB; ++i) {
-        const int e = (i * NTHR + tid) * 8, t = e / N, c = e % N;
-        q.b[i] = bf16x8{};
-        if (t < nval)
-          q.b[i] = *reinterpret_cast<const bf16x8*>(p.B + (int64_t)(tok0 + t) * p.b_ts + (int64_t)g * p.b_gs + c);
-      }
-    }
-    q.dt = (wave == 0 && lane < nval)
-               ? ld_bits(p.dt, (int64_t)(tok0 + lane) * p.dt_ts + (int64_t)h * p.dt_hs, p.dt_dt) : 0u;
-  };
-  In in;
-  if constexpr (AHEAD) fetch(h_first, in);
-  constexpr int PBW = P / 16 / 4;   // p blocks per wave
-  for (int ih = 0; ih < nh; ++ih) {
-    const int h = h_first + ih;
-    if (wave == 0) {
-      const Tok tk = AHEAD ? token_scalars_raw(p, h, bits_f32(in.dt, p.dt_dt), nval, lane)
-                           : token_scalars(p, h, tok0, nval, lane);
-      const float aend = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tk.acs), 63));
-      sEA[lane] = fast_exp(tk.acs);
-      sWT[lane] = tk.dtv * fast_exp(aend - tk.acs);
-      if (lane == L - 1) p.edec[(int64_t)r * H + h] = expf(aend);
-    }
-    __syncthreads();   // the scalars; the previous head's products have read the tiles
-    if constexpr (!AHEAD) {   // headdim 128: the rows straight from memory
-      const int hx = h / HXS, g = h / HB;
-#pragma unroll
-      for (int i = 0; i < VX; ++i) {
-        const int e = (i * NTHR + tid) * 8, t = e / P, c = e % P;
-        in.x[i] = in.dy[i] = bf16x8{};
-        if (t < nval) {
-          in.dy[i] = *reinterpret_cast<const bf16x8*>(p.dy + (int64_t)(tok0 + t) * p.dy_ts + (int64_t)h * p.dy_hs + c);
-          in.x[i] = *reinterpret_cast<const bf16x8*>(p.x + (int64_t)(tok0 + t) * p.x_ts + (int64_t)hx * p.x_hs + c);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < VB; ++i) {
-        const int e = (i * NTHR + tid) * 8, t = e / N, c = e % N;
-        bf16x8 bv = {};
-        if (t < nval)
-          bv = *reinterpret_cast<const bf16x8*>(p.B + (int64_t)(tok0 + t) * p.b_ts + (int64_t)g * p.b_gs + c);
-        *reinterpret_cast<bf16x8*>(sB + t * LDB + c) = bv;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < VX; ++i) {
-      const int e = (i * NTHR + tid) * 8, t = e / P, c = e % P;
-      const float ea = sEA[t], wt = sWT[t];
-      bf16x8 o, xw;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float v = (float)in.dy[i][j];
-        if constexpr (P == 64) {
-          if (p.z) v *= silu((float)in.z[i][j]);
-        }
-        o[j] = (bf16)(v * ea);
-        xw[j] = (bf16)((float)in.x[i][j] * wt);
-      }
-      *reinterpret_cast<bf16x8*>(sG + t * LDX + c) = o;
-      *reinterpret_cast<bf16x8*>(sXW + t * LDX + c) = xw;
-    }
-    if (AHEAD && !b_once) {
-#pragma unroll
-      for (int i = 0; i < VB; ++i) {
-        const int e = (i * NTHR + tid) * 8, t = e / N, c = e % N;
-        *reinterpret_cast<bf16x8*>(sB + t * LDB + c) = in.b[i];
-      }
-    }
-    __syncthreads();
-    if constexpr (AHEAD) {
-      if (ih + 1 < nh) fetch(h + 1, in);
-    }
-    // wave w: p rows [16 (w PBW + i), ...), all n tiles, for both products (one after
-    // the other: their tiles would not fit in registers together at headdim 128)
-#pragma unroll 1
-    for (int which = 0; which < 2; ++which) {
-      const bf16* sa = which ? sXW : sG;
-      const bf16* sb = which ? sB : sC;
-      f32x4 acc[PBW][N / 16];
-#pragma unroll
-      for (int i = 0; i < PBW; ++i)
-#pragma unroll
-        for (int j = 0; j < N / 16; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k0 = 0; k0 < L; k0 += 32) {
-        bf16x8 bf[N / 16];
-#pragma unroll
-        for (int j = 0; j < N / 16; ++j) bf[j] = frag_t(sb, LDB, k0, 16 * j, lane);
-#pragma unroll
-        for (int i = 0; i < PBW; ++i) {
-          const bf16x8 af = frag_t(sa, LDX, k0, 16 * (wave * PBW + i), lane);
-#pragma unroll
-          for (int j = 0; j < N / 16; ++j) acc[i][j] = mfma16(af, bf[j], acc[i][j]);
-        }
-      }
-      bf16* dst = (which ? p.sloc : p.loc) + ((int64_t)r * H + h) * P * N;
-#pragma unroll
-      for (int i = 0; i < PBW; ++i)
-#pragma unroll
-        for (int j = 0; j < N / 16; ++j)
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            dst[(16 * (wave * PBW + i) + 4 * q4 + v) * N + 16 * j + l16] = (bf16)acc[i][j][v];
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// scans over a sequence's chunks, 4 state elements per thread, PF chunks' loads in
-// flight ahead of the dependent chain:
-//   forward: S0(first) = h0 (or 0), S0(c+1) = e^{A_L(c)} S0(c) + sloc(c)
-//   reverse: dS1(last) = dT (or 0), dS1(c-1) = e^{A_L(c)} dS1(c) + loc(c); dh0 =
-//            the value before the first chunk
-// ---------------------------------------------------------------------------
-constexpr int PF = 4;
-__device__ __forceinline__ f32x4 ld4(const float* q) { return *reinterpret_cast<const f32x4*>(q); }
-__device__ __forceinline__ f32x4 ld4(const bf16* q) {
-  const bf16x4 v = *reinterpret_cast<const bf16x4*>(q);
-  return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-}
-__device__ __forceinline__ void st4b(bf16* q, f32x4 v) {
-  *reinterpret_cast<bf16x4*>(q) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
-}
-
-__global__ __launch_bounds__(256) void ssd_bwd_scan_kernel(Params p, int PN) {
   const int H = p.H;
-  const int n = blockIdx.x / H, h = blockIdx.x % H;
-  const int first = p.seqs[2 * n], cnt = p.seqs[2 * n + 1];
-  const int e = (blockIdx.y * 256 + threadIdx.x) * 4;
-  if (e >= PN) return;
-  const int64_t sb = ((int64_t)n * H + h) * PN + e;
-  auto off = [&](int k) { return ((int64_t)(first + k) * H + h) * PN + e; };
-  auto dec = [&](int k) { return p.edec[(int64_t)(first + k) * H + h]; };
-  // Chain position m of a direction: chunk k = m (forward) or cnt-1-m (reverse).
-  // Full groups of PF run without branches (the prefetch index is clamped in
-  // bounds), so each load is waited for only where it is used; the tail is guarded.
-  auto chain = [&](bool fwd, f32x4 X, const bf16* src, bf16* dst) -> f32x4 {
-    if (cnt == 0) return X;
-    auto kk = [&](int m) { return fwd ? m : cnt - 1 - m; };
-    f32x4 buf[PF];
-#pragma unroll
-    for (int j = 0; j < PF; ++j) buf[j] = ld4(src + off(kk(min(j, cnt - 1))));
-    int m = 0;
-    for (; m + PF <= cnt; m += PF) {
-#pragma unroll
-      for (int j = 0; j < PF; ++j) {
-        const int k = kk(m + j);
-        st4b(dst + off(k), X);
-        const float d = dec(k);
-        const f32x4 l = buf[j];
-        buf[j] = ld4(src + off(kk(min(m + j + PF, cnt - 1))));
-        X = X * d + l;
-      }
+  const int tot = gridDim.x, id = blockIdx.x;
+  int u = tot % 8 ? id : (id % 8) * (tot / 8) + id / 8;      // consecutive units on one XCD
+  const int p0 = (u % (P / SP)) * SP;
+  u /= P / SP;
+  const int h = u % H;
+  u /= H;
+  const int dir = u & 1, b = u >> 1;
+  int ra = b * Lr, rb = min(ra + Lr, p.nrows);
+  if constexpr (TOT) {
+    // needed by a block after (before) this one only if a sequence crosses into it; only
+    // the crossing sequence's rows count
+    if (dir == 0) {
+      if (rb >= p.nrows) return;
+      const Row nx = load_row(p.seg, rb);
+      if (nx.idx == 0) return;
+      ra = max(ra, nx.first);
+    } else {
+      if (ra == 0) return;
+      const Row ro = load_row(p.seg, ra);
+      if (ro.idx == 0) return;
+      rb = min(rb, ro.first + ro.nseg);
     }
+  }
+  const int cnt = rb - ra;
+  const int nb = wave % NB, pb0 = (wave / NB) * PBW;
+  // this lane's part of the state: rows p0 + 16 (pb0 + i) + l16, features n_l .. n_l + 7
+  const int n_l = 32 * nb + 8 * q4;
+  const auto pn = [&](int i) { return (p0 + 16 * (pb0 + i) + l16) * N + n_l; };
+  f32x4 X[PBW][2];
+  const auto load_state = [&](const float* s) {     // [P][N] fp32, or null
 #pragma unroll
-    for (int j = 0; j < PF; ++j) {
-      if (m + j < cnt) {
-        const int k = kk(m + j);
-        st4b(dst + off(k), X);
-        X = X * dec(k) + buf[j];
-      }
-    }
-    return X;
+    for (int i = 0; i < PBW; ++i)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+        X[i][a] = s ? *reinterpret_cast<const f32x4*>(s + pn(i) + 4 * a) : f32x4{0.f, 0.f, 0.f, 0.f};
   };
-  chain(true, p.h0 ? ld4(p.h0 + sb) : f32x4{0.f, 0.f, 0.f, 0.f}, p.sloc, p.S0);
-  {
-    const f32x4 G = chain(false, p.dT ? ld4(p.dT + sb) : f32x4{0.f, 0.f, 0.f, 0.f}, p.loc, p.dS1);
-    if (p.dh0) *reinterpret_cast<f32x4*>(p.dh0 + sb) = G;
+  const auto store_state = [&](float* s) {
+#pragma unroll
+    for (int i = 0; i < PBW; ++i)
+#pragma unroll
+      for (int a = 0; a < 2; ++a) *reinterpret_cast<f32x4*>(s + pn(i) + 4 * a) = X[i][a];
+  };
+  const float* init = dir ? p.dT : p.h0;
+  const auto init_of = [&](int n) { return init ? init + ((int64_t)n * H + h) * P * N : nullptr; };
+  const auto tot_at = [&](int j) { return p.tot + (((int64_t)dir * nblk + j) * H + h) * P * N; };
+  const auto dec_at = [&](int j) -> float& { return p.tdec[((int64_t)dir * nblk + j) * H + h]; };
+  load_state(nullptr);
+  if (!TOT && b == 0 && dir == 1 && p.dh0) {
+    // sequences without tokens: dh0 = dT
+    for (int n0 = 0; n0 < p.nseq; n0 += 64) {
+      uint64_t e = __ballot(n0 + lane < p.nseq && p.seqs[2 * min(n0 + lane, p.nseq - 1) + 1] == 0);
+      for (; e; e &= e - 1) {
+        const int n = n0 + __builtin_ctzll(e);
+        load_state(init_of(n));
+        store_state(p.dh0 + ((int64_t)n * H + h) * P * N);
+      }
+    }
+    load_state(nullptr);
+  }
+  if (cnt <= 0) return;
+  if (!TOT && nblk > 1) {
+    // the sequence's blocks before this one
+    const Row ro = load_row(p.seg, dir ? rb - 1 : ra);
+    const int end = ro.first + ro.nseg - 1;
+    const int j0 = dir ? end / Lr : ro.first / Lr;
+    for (int j = j0; j != b; j += dir ? -1 : 1) {
+      const float d = j == j0 ? 0.f : dec_at(j);
+      const float* t = tot_at(j);
+#pragma unroll
+      for (int i = 0; i < PBW; ++i)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+          X[i][a] = X[i][a] * d + *reinterpret_cast<const f32x4*>(t + pn(i) + 4 * a);
+    }
+  }
+
+  const bf16* mat = dir ? p.C + (int64_t)(h / (H / p.GC)) * p.c_gs : p.B + (int64_t)(h / (H / p.G)) * p.b_gs;
+  const int64_t m_ts = dir ? p.c_ts : p.b_ts;
+  const bf16* src = (dir ? p.dy + (int64_t)h * p.dy_hs : p.x + (int64_t)(h / (H / p.HX)) * p.x_hs) + p0;
+  const int64_t s_ts = dir ? p.dy_ts : p.x_ts;
+  const bool has_z = dir && p.z;
+  const bf16* zs = has_z ? p.z + (int64_t)h * p.z_hs + p0 : nullptr;
+  const bool f32dt = p.dt_dt == HMX_F32;
+  const uint16_t* dts = static_cast<const uint16_t*>(p.dt);
+  const float bias = p.dt_bias ? p.dt_bias[h] : 0.f, A_h = p.A[h];
+  const int tx = tid / (SP / 8), cx = (tid % (SP / 8)) * 8;               // this thread's piece of x
+  const int tm = tid / TPR, cm = (tid % TPR) * 8;            // and of B: rows tm + i STHR / TPR
+
+  // The scalars of a chunk (its tokens' weights, its decay), a serial chain over the 64
+  // lanes, are formed four chunks at a time, one per wave (waves w and w + 4 alike), two
+  // groups of four ahead of the chunk (loads of dt) and one group ahead (the chain); sW
+  // holds two groups.
+  const auto row_of = [&](int m) { return dir ? rb - 1 - m : ra + m; };
+  struct Span { int bos, eos; };
+  struct Dt { uint16_t lo, hi; int nv; };  // dt of token `lane` as stored (an fp32's halves)
+  const auto scal_row = [&](int grp) {     // of this wave's chunk of a group
+    const int* r = p.seg + (int64_t)row_of(min(4 * grp + (wave & 3), cnt - 1)) * 8;
+    return Span{r[1], r[2]};
+  };
+  const auto scal_fetch = [&](const Span& g) {
+    const int nv = g.eos - g.bos;
+    const int64_t di = (int64_t)(g.bos + min(lane, max(nv - 1, 0))) * p.dt_ts + (int64_t)h * p.dt_hs;
+    return Dt{dts[f32dt ? 2 * di : di], dts[f32dt ? 2 * di + 1 : di], nv};
+  };
+  const auto scal_form = [&](const Dt& g, int grp) {
+    const uint32_t lo = g.lo, hi = g.hi;
+    float dtv = (f32dt ? __builtin_bit_cast(float, lo | (hi << 16)) : bits_f32(lo, p.dt_dt)) + bias;
+    if (p.softplus) dtv = softplus20(dtv);
+    dtv = fminf(fmaxf(dtv, p.dt_min), p.dt_max);
+    if (lane >= g.nv) dtv = 0.f;
+    const float acs = scan64(dtv * A_h, lane);
+    const float aend = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acs), 63));
+    float* o = sW + (4 * (grp & 1) + (wave & 3)) * Y::SW;
+    o[lane] = dir ? fast_exp(acs) : dtv * fast_exp(aend - acs);
+    if (lane == 0) o[L] = expf(aend);
+  };
+
+  // rows of the table, 64 chain positions at a time across the lanes
+  int i_n = 0, i_bos = 0, i_nv = 0, i_fl = 0;
+  const int64_t xo = tx * s_ts + cx, mo = tm * m_ts + cm, mi = (STHR / TPR) * m_ts, zo = tx * p.z_ts + cx;
+  const auto fetch = [&](StateIn<N>& q, int m) {
+    // past the last chunk: that one again (a load that may be skipped cannot be counted,
+    // and the waits for the chunks in flight would be waits for all of them)
+    const bool fresh = (m & 63) == 0 && m < cnt;
+    m = min(m, cnt - 1);
+    if (fresh) {
+      const Row ro = load_row(p.seg, row_of(min(m + lane, cnt - 1)));
+      i_n = ro.n;
+      i_bos = ro.bos;
+      i_nv = ro.eos - ro.bos;
+      i_fl = (ro.idx == 0 ? 1 : 0) | (ro.idx == ro.nseg - 1 ? 2 : 0);
+    }
+    const int64_t tok0 = __builtin_amdgcn_readlane(i_bos, m & 63);
+    q.nval = __builtin_amdgcn_readlane(i_nv, m & 63);
+    q.fl = __builtin_amdgcn_readlane(i_fl, m & 63);
+    q.n = __builtin_amdgcn_readlane(i_n, m & 63);
+    q.r = row_of(m);
+    const bf16* sb = src + tok0 * s_ts;
+    const bf16* mb = mat + tok0 * m_ts;
+    int64_t ox = xo, oz = zo, om[VB];
+#pragma unroll
+    for (int i = 0; i < VB; ++i) om[i] = mo + i * mi;
+    if (q.nval < L) {
+      // rows past the chunk's tokens load its last one; their x is dropped where it is staged
+      const int last = max(q.nval - 1, 0);
+      ox = min(tx, last) * s_ts + cx;
+      oz = min(tx, last) * p.z_ts + cx;
+#pragma unroll
+      for (int i = 0; i < VB; ++i) om[i] = min(tm + i * (STHR / TPR), last) * m_ts + cm;
+    }
+    q.x = *reinterpret_cast<const bf16x8*>(sb + ox);
+#pragma unroll
+    for (int i = 0; i < VB; ++i) q.m[i] = *reinterpret_cast<const bf16x8*>(mb + om[i]);
+    if (has_z) q.z = *reinterpret_cast<const bf16x8*>(zs + tok0 * p.z_ts + oz);
+  };
+
+  float ldec = 1.f;                       // decay over the rows walked (TOT)
+  const auto step = [&](StateIn<N>& q, int m) {
+    bf16* sM = lds + (m & 1) * Y::SET;
+    bf16* sX = sM + Y::SZ_B;
+    const float* sw = sW + (m & 7) * Y::SW;
+    const float wt = sw[tx], dec = sw[L];
+    if (q.fl & (dir ? 2 : 1)) {
+      load_state(init_of(q.n));
+#pragma unroll
+      for (int i = 0; i < PBW; ++i)
+#pragma unroll
+        for (int a = 0; a < 2; ++a) asm volatile("" : "+v"(X[i][a]));   // waited for here only
+    }
+    if constexpr (!TOT) {
+      bf16* dst = (dir ? p.dS1 : p.S0) + ((int64_t)q.r * H + h) * P * N;
+#pragma unroll
+      for (int i = 0; i < PBW; ++i)
+        *reinterpret_cast<bf16x8*>(dst + pn(i)) =
+            bf16x8{(bf16)X[i][0][0], (bf16)X[i][0][1], (bf16)X[i][0][2], (bf16)X[i][0][3],
+                   (bf16)X[i][1][0], (bf16)X[i][1][1], (bf16)X[i][1][2], (bf16)X[i][1][3]};
+    } else {
+      ldec *= dec;
+    }
+    {
+      float v[8];
+      bf16x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = (float)q.x[j];
+      if (has_z) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] *= silu((float)q.z[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (bf16)(tx < q.nval ? v[j] * wt : 0.f);
+      *reinterpret_cast<bf16x8*>(sX + tx * Y::LDX + cx) = o;
+#pragma unroll
+      for (int i = 0; i < VB; ++i) {
+        bf16* d = sM + (tm + i * (STHR / TPR)) * Y::LDB + (cm & ~31) + ((cm & 24) >> 1);
+        const bf16x8 y = q.m[i];
+        *reinterpret_cast<bf16x4*>(d) = bf16x4{y[0], y[1], y[2], y[3]};
+        *reinterpret_cast<bf16x4*>(d + 16) = bf16x4{y[4], y[5], y[6], y[7]};
+      }
+    }
+    const int fl = q.fl, n = q.n;
+    fetch(q, m + SD);
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < PBW; ++i)
+#pragma unroll
+      for (int a = 0; a < 2; ++a) X[i][a] *= dec;
+#pragma unroll
+    for (int k0 = 0; k0 < L; k0 += 32) {
+      bf16x8 fa[2], fx[PBW];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) fa[a] = frag_t_perm(sM, Y::LDB, k0, 32 * nb + 16 * a, lane);
+#pragma unroll
+      for (int i = 0; i < PBW; ++i) fx[i] = frag_t_perm(sX, Y::LDX, k0, 16 * (pb0 + i), lane);
+#pragma unroll
+      for (int i = 0; i < PBW; ++i)
+#pragma unroll
+        for (int a = 0; a < 2; ++a) X[i][a] = mfma16(fa[a], fx[i], X[i][a]);
+    }
+    if (!TOT && dir && (fl & 1) && p.dh0) store_state(p.dh0 + ((int64_t)n * H + h) * P * N);
+  };
+  static_assert(SD == 4, "one group of scalars per pass of the loop");
+  const Span r0 = scal_row(0), r1 = scal_row(1);
+  Span rn = scal_row(2);
+  const Dt d0 = scal_fetch(r0);
+  Dt dn = scal_fetch(r1);
+  StateIn<N> q[SD];
+#pragma unroll
+  for (int j = 0; j < SD; ++j) {
+    fetch(q[j], j);
+    __builtin_amdgcn_sched_barrier(0);    // in this order: the loop's waits count on it
+  }
+  scal_form(d0, 0);
+  lds_barrier();
+  for (int m = 0;;) {
+    scal_form(dn, m / 4 + 1);
+    dn = scal_fetch(rn);
+    rn = scal_row(m / 4 + 3);
+    step(q[0], m);
+    if (++m == cnt) break;
+    step(q[1], m);
+    if (++m == cnt) break;
+    step(q[2], m);
+    if (++m == cnt) break;
+    step(q[3], m);
+    if (++m == cnt) break;
+  }
+  if constexpr (TOT) {
+    store_state(tot_at(b));
+    if (p0 == 0 && tid == 0) dec_at(b) = ldec;
   }
 }
 
@@ -420,8 +487,6 @@ __global__ __launch_bounds__(256) void ssd_bwd_scan_kernel(Params p, int PN) {
 // at 2 x 8192, H = 64, P = 64 with one head per group 2.17 -> 1.47 ms.
 // ---------------------------------------------------------------------------
 constexpr int GTHR = 512;
-
-constexpr int row_ld(int w) { return w == 64 ? w + 8 : w + 16; }
 
 template <int P, int N>
 struct GLay {
@@ -1362,20 +1427,25 @@ __global__ __launch_bounds__(NTHR, 1) void ssd_bwd_chunk_kernel(Params p) {
 
 template <int P, int N>
 void launch(const Params& p, hipStream_t s) {
-  constexpr int lsm = local_lds_bytes<P, N>();
   constexpr int smem = Lay<P, N>::BYTES;
-  (void)hipFuncSetAttribute((const void*)ssd_bwd_local_kernel<P, N>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lsm);
   (void)hipFuncSetAttribute((const void*)ssd_bwd_chunk_kernel<P, N>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  hipLaunchKernelGGL((ssd_bwd_local_kernel<P, N>), dim3(p.nrows * (P == 64 ? p.GC : p.H)),
-                     dim3(NTHR), lsm, s, p);
-  hipLaunchKernelGGL(ssd_bwd_scan_kernel, dim3(p.nseq * p.H, (P * N + 1023) / 1024), dim3(256), 0,
-                     s, p, P * N);
+  // blocks of table rows: one where the heads alone give a workgroup per CU, else as
+  // many as that takes, of no fewer than 8 rows
+  const int units = p.H * 2 * (P / SP);
+  const int want = std::min((256 + units - 1) / units, std::max(p.nrows / 8, 1));
+  const int Lr = std::max((p.nrows + want - 1) / want, 1);
+  const int nblk = std::max((p.nrows + Lr - 1) / Lr, 1);
+  if (nblk > 1)
+    hipLaunchKernelGGL((ssd_bwd_states_kernel<P, N, true>), dim3(units * nblk), dim3(STHR), 0, s, p, Lr, nblk);
+  hipLaunchKernelGGL((ssd_bwd_states_kernel<P, N, false>), dim3(units * nblk), dim3(STHR), 0, s, p, Lr, nblk);
+  if (p.nrows == 0) return;               // sequences without tokens only
   // the group kernel shares C B^T and W's products over the heads (B and C grouped
   // alike) and forms no y' (which only z needs); it is the faster one at every size
-  // measured (its comment), from one head per group on
-  if (p.G == p.GC && !p.z) {
+  // measured (its comment), from one head per group on.  It addresses a chunk's 64 rows
+  // with 32-bit byte offsets; the other kernel takes any stride.
+  const bool near = std::max(std::max(p.x_ts, p.dy_ts), std::max(p.b_ts, p.c_ts)) < (1 << 24);
+  if (p.G == p.GC && !p.z && near) {
     constexpr int gsm = GLay<P, N>::BYTES;
     (void)hipFuncSetAttribute((const void*)ssd_bwd_group_kernel<P, N>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, gsm);
@@ -1392,8 +1462,10 @@ using namespace hmx;
 using namespace hmx::ssdb;
 
 extern "C" size_t hmx_ssd_chunk_bwd_workspace_bytes(int32_t nrows, int32_t H, int32_t P, int32_t N) {
+  // S0, dS1 (bf16); the block totals (fp32, both directions, at most nrows / 8 blocks)
+  // and their decays
   const size_t st = (size_t)nrows * H * P * N;
-  return st * (2 + 2 + 2 + 2) + (size_t)nrows * H * 4 + 256;
+  return st * (2 + 2 + 1) + (size_t)nrows * H * 4 + 256;
 }
 
 extern "C" int hmx_ssd_chunk_bwd(
@@ -1445,11 +1517,10 @@ extern "C" int hmx_ssd_chunk_bwd(
   p.seg = seg_table; p.seqs = seq_table; p.nrows = nrows; p.nseq = nseq;
   const size_t st = (size_t)nrows * H * P * N;
   unsigned char* ws = static_cast<unsigned char*>(workspace);
-  p.loc = reinterpret_cast<bf16*>(ws);
-  p.sloc = reinterpret_cast<bf16*>(ws + st * 2);
-  p.S0 = reinterpret_cast<bf16*>(ws + st * 4);
-  p.dS1 = reinterpret_cast<bf16*>(ws + st * 6);
-  p.edec = reinterpret_cast<float*>(ws + st * 8);
+  p.S0 = reinterpret_cast<bf16*>(ws);
+  p.dS1 = reinterpret_cast<bf16*>(ws + st * 2);
+  p.tot = reinterpret_cast<float*>(ws + st * 4);
+  p.tdec = reinterpret_cast<float*>(ws + st * 5);
   p.dx = dx; p.x_shared = HX < H;
   p.dB = dB; p.b_shared = G < H;
   p.dC = dC; p.gbf16 = grad_dtype == HMX_BF16;
@@ -1458,11 +1529,6 @@ extern "C" int hmx_ssd_chunk_bwd(
   p.H = H; p.HX = HX; p.G = G; p.GC = GC; p.softplus = dt_softplus;
   p.dt_min = dt_min; p.dt_max = dt_max;
   hipStream_t s = (hipStream_t)stream;
-  if (nrows == 0) {   // empty sequences only: dh0 = dT
-    hipLaunchKernelGGL(ssd_bwd_scan_kernel, dim3(nseq * H, (P * N + 1023) / 1024), dim3(256), 0, s,
-                       p, P * N);
-    return check_launch(fn);
-  }
   if (P == 64 && N == 128) launch<64, 128>(p, s);
   else if (P == 64) launch<64, 64>(p, s);
   else if (N == 128) launch<128, 128>(p, s);

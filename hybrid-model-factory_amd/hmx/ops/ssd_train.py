@@ -4,9 +4,10 @@ The training layer calls mamba_ssm's ``mamba_chunk_scan_combined`` under autogra
 (training/src/hmf/model/hybrid_zoo/layers/mamba/mamba2.py:555-580).  The forward
 here is the HIP scan of ops/ssd.py.  The backward (csrc/ssd_backward.hip) forms
 the state at the start of every 64-token chunk again from the inputs (nothing
-beyond them is kept between forward and backward): a local pass per chunk, one
-scan launch running the forward state chain and the reverse chain of the state
-gradients, then the per-chunk gradient kernel.
+beyond them is kept between forward and backward): one launch runs the forward state
+chain and the reverse chain of the state gradients over the chunks (a launch before it
+sums blocks of chunks where few heads would leave the chip idle), then the per-chunk
+gradient kernel.
 """
 from __future__ import annotations
 

@@ -177,6 +177,24 @@ def test_backward_groups_without_z(dev, P, N, H, G, l):
         _check(g[k], g_ref[k], f"groups P={P} N={N} d{k}", scale=sA if k == "A" else None)
 
 
+@pytest.mark.parametrize("P,N,H,lens", [(64, 128, 2, (1400, 3, 64, 65, 900, 1)), (128, 64, 1, (30, 1100, 1)),
+                                        (64, 64, 3, (64,) * 17)])
+def test_backward_state_chains_cross_blocks(dev, P, N, H, lens):
+    """Few heads, many chunks: the state chains run in blocks of chunks that sequences
+    cross, end in and begin in (a sequence over more than two blocks, several within one,
+    one-token and whole last chunks), with initial and final states."""
+    inp, wy, wf = _inputs(1, sum(lens), H, 1, P, N, 990 + len(lens), False, False)
+    idx = torch.cat([torch.full((n,), i, dtype=torch.int32) for i, n in enumerate(lens)])[None]
+    kw = dict(dt_softplus=True, return_final_states=True)
+    g = _grads(inp, wy, wf, dict(kw, seq_idx=idx.to(dev)), dev, None)
+    torch.cuda.synchronize()
+    kw["seq_idx"] = idx
+    g_ref = _grads(inp, wy, wf, kw, None, torch.float64)
+    sA = _dA_scale(inp, wy, wf, kw)
+    for k in g_ref:
+        _check(g[k], g_ref[k], f"blocks P={P} N={N} d{k}", scale=sA if k == "A" else None)
+
+
 def test_backward_headdim_128_with_z_raises(dev):
     inp, _, _ = _inputs(1, 64, 2, 1, 128, 64, 1, True, False)
     x = inp["x"].to(dev).requires_grad_(True)
