@@ -304,7 +304,8 @@ __global__ __launch_bounds__(STHR, 2) void ssd_bwd_states_kernel(Params p, int L
   };
   const auto scal_fetch = [&](const Span& g) {
     const int nv = g.eos - g.bos;
-    const int64_t di = (int64_t)(g.bos + min(lane, max(nv - 1, 0))) * p.dt_ts + (int64_t)h * p.dt_hs;
+    const int64_t t = nv > 0 ? g.bos + min(lane, nv - 1) : 0;      // (a row without tokens: any)
+    const int64_t di = t * p.dt_ts + (int64_t)h * p.dt_hs;
     return Dt{dts[f32dt ? 2 * di : di], dts[f32dt ? 2 * di + 1 : di], nv};
   };
   const auto scal_form = [&](const Dt& g, int grp) {
@@ -331,8 +332,8 @@ __global__ __launch_bounds__(STHR, 2) void ssd_bwd_states_kernel(Params p, int L
     if (fresh) {
       const Row ro = load_row(p.seg, row_of(min(m + lane, cnt - 1)));
       i_n = ro.n;
-      i_bos = ro.bos;
       i_nv = ro.eos - ro.bos;
+      i_bos = i_nv > 0 ? ro.bos : 0;
       i_fl = (ro.idx == 0 ? 1 : 0) | (ro.idx == ro.nseg - 1 ? 2 : 0);
     }
     const int64_t tok0 = __builtin_amdgcn_readlane(i_bos, m & 63);
