@@ -195,6 +195,29 @@ def test_backward_state_chains_cross_blocks(dev, P, N, H, lens):
         _check(g[k], g_ref[k], f"blocks P={P} N={N} d{k}", scale=sA if k == "A" else None)
 
 
+def test_backward_far_apart_gradient_rows(dev):
+    """dy with token rows 2^24 elements apart (a chunk's rows past the 32-bit byte offsets
+    of the group kernel): the general kernel takes it; the same gradients as from
+    contiguous rows, to the rounding of two kernels that each meet _check's bound."""
+    l, H, P = 3, 2, 64
+    inp, wy, _ = _inputs(1, l, H, 1, P, 128, 995, False, False)
+    inp.pop("z")
+    leaves = {k: v.to(dev).requires_grad_(True) for k, v in inp.items()}
+    args = dict(leaves)
+    y = hmx.mamba_chunk_scan_combined(args.pop("x"), args.pop("dt"), args.pop("A"), args.pop("B"),
+                                      args.pop("C"), 256, dt_softplus=True, **args)
+    dy = wy.to(dev, torch.bfloat16)
+    step = 1 << 24
+    far = torch.zeros((l - 1) * step + H * P, dtype=torch.bfloat16, device=dev)
+    far = far.as_strided((1, l, H, P), (l * step, step, P, 1))
+    far.copy_(dy)
+    g = torch.autograd.grad(y, list(leaves.values()), dy, retain_graph=True)
+    g_far = torch.autograd.grad(y, list(leaves.values()), far)
+    torch.cuda.synchronize()
+    for k, a, b in zip(leaves, g_far, g):
+        _check(a, b, f"far d{k}")
+
+
 def test_backward_headdim_128_with_z_raises(dev):
     inp, _, _ = _inputs(1, 64, 2, 1, 128, 64, 1, True, False)
     x = inp["x"].to(dev).requires_grad_(True)
