@@ -527,14 +527,22 @@ __device__ __forceinline__ void st8(bf16* row, int f0, const bf16x8& y) {
 }
 
 // Raw buffer resource over rows 0 .. nrows-1 (w elements of `es` bytes, ts elements
-// apart): rows past the end read zeros and write nothing.  The host keeps 64 rows of
-// any stride inside 32-bit offsets.
+// apart): past its end nothing is read (zeros) or written.  The host keeps 64 rows of
+// any stride inside 31-bit offsets.  Where ts < w (0: an operand constant over the
+// tokens) the rows after nrows-1 overlap the ones before, so a load names them missing
+// by row_off, not by their place.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, int nrows, int64_t ts,
                                                            int w, int es) {
   const uint32_t bytes = nrows > 0 ? (uint32_t)(((int64_t)(nrows - 1) * ts + w) * es) : 0u;
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
+constexpr uint32_t ROW_OFF = 1u << 31;    // past any resource
+// byte offset of feature c of row t of a bf16 operand, past the resource's end for rows
+// t >= nval (a select, not a branch: the loads stay countable)
+__device__ __forceinline__ uint32_t row_off(int t, int64_t ts, int c, int nval) {
+  return t < nval ? (uint32_t)((t * ts + c) * 2) : ROW_OFF;
 }
 __device__ __forceinline__ bf16x8 ld_row(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
@@ -581,8 +589,8 @@ __global__ __launch_bounds__(GTHR, 2) void ssd_bwd_group_kernel(Params p) {
 #pragma unroll
     for (int i = 0; i < VB; ++i) {
       const int t = i * RS + tid / (N / 8), c = (tid % (N / 8)) * 8;
-      bv[i] = ld_row(rb, (uint32_t)(((int64_t)t * p.b_ts + c) * 2));
-      cv[i] = ld_row(rc, (uint32_t)(((int64_t)t * p.c_ts + c) * 2));
+      bv[i] = ld_row(rb, row_off(t, p.b_ts, c, nval));
+      cv[i] = ld_row(rc, row_off(t, p.c_ts, c, nval));
     }
   };
   const auto fetch = [&](int tid, int h, In& q) {
@@ -592,8 +600,8 @@ __global__ __launch_bounds__(GTHR, 2) void ssd_bwd_group_kernel(Params p) {
 #pragma unroll
     for (int i = 0; i < VX; ++i) {
       const int t = i * RX + tid / (P / 8), c = (tid % (P / 8)) * 8;
-      q.x[i] = ld_row(rx, (uint32_t)(((int64_t)t * p.x_ts + c) * 2));
-      q.dy[i] = ld_row(ry, (uint32_t)(((int64_t)t * p.dy_ts + c) * 2));
+      q.x[i] = ld_row(rx, row_off(t, p.x_ts, c, nval));
+      q.dy[i] = ld_row(ry, row_off(t, p.dy_ts, c, nval));
     }
     const bf16* s0 = p.S0 + ((int64_t)r * H + h) * P * N;
     const bf16* ds = p.dS1 + ((int64_t)r * H + h) * P * N;
@@ -1444,8 +1452,9 @@ void launch(const Params& p, hipStream_t s) {
   // the group kernel shares C B^T and W's products over the heads (B and C grouped
   // alike) and forms no y' (which only z needs); it is the faster one at every size
   // measured (its comment), from one head per group on.  It addresses a chunk's 64 rows
-  // with 32-bit byte offsets; the other kernel takes any stride.
-  const bool near = std::max(std::max(p.x_ts, p.dy_ts), std::max(p.b_ts, p.c_ts)) < (1 << 24);
+  // with 31-bit byte offsets; the other kernel takes any stride.
+  const auto ts = {p.x_ts, p.dy_ts, p.b_ts, p.c_ts};
+  const bool near = std::min(ts) >= 0 && std::max(ts) < (1 << 24) && (int64_t)p.HX * P < (1 << 23);
   if (p.G == p.GC && !p.z && near) {
     constexpr int gsm = GLay<P, N>::BYTES;
     (void)hipFuncSetAttribute((const void*)ssd_bwd_group_kernel<P, N>,

@@ -218,6 +218,37 @@ def test_backward_far_apart_gradient_rows(dev):
         _check(a, b, f"far d{k}")
 
 
+@pytest.mark.parametrize("P,over,l", [(64, "C", 130), (64, "x", 65), (64, "xBC", 66), (128, "C", 65),
+                                      (128, "x", 130)])
+def test_backward_operands_constant_over_tokens(dev, P, over, l):
+    """Operands expanded over the tokens (token stride 0) under a loss that pools the
+    tokens (dy expanded too) and a ragged last chunk: the rows past its tokens overlap
+    real ones, and count nothing.  Every gradient against the oracle's."""
+    inp, wy, _ = _inputs(1, l, 4, 2, P, 128, 1010 + l, False, True)
+    inp.update({k: inp[k][:, :1].expand(-1, l, -1, -1) for k in over})
+    wy = wy[:, :1].bfloat16().expand(-1, l, -1, -1)
+    kw = dict(dt_softplus=True)
+
+    def grads(fn, conv):
+        t = {k: conv(v).requires_grad_(True) for k, v in inp.items() if v is not None}
+        a = dict(t)
+        y = fn(a.pop("x"), a.pop("dt"), a.pop("A"), a.pop("B"), a.pop("C"), 256, **a, **kw)
+        return dict(zip(t, torch.autograd.grad(y, list(t.values()), conv(wy))))
+
+    def on_dev(v):      # .to() keeps no stride of 0: the token's row moved, then expanded
+        if v.dim() == 4 and v.stride(1) == 0:
+            return v[:, :1].to(dev).expand(-1, l, -1, -1)
+        return v.to(dev)
+
+    assert all(on_dev(inp[k]).stride(1) == 0 for k in over) and on_dev(wy).stride(1) == 0
+    g = grads(hmx.mamba_chunk_scan_combined, on_dev)
+    torch.cuda.synchronize()
+    g_ref = grads(ref.mamba_chunk_scan_combined, lambda v: v.double())
+    sA = _dA_scale(inp, wy, None, kw)
+    for k in g_ref:
+        _check(g[k], g_ref[k], f"over={over} P={P} d{k}", scale=sA if k == "A" else None)
+
+
 def test_backward_headdim_128_with_z_raises(dev):
     inp, _, _ = _inputs(1, 64, 2, 1, 128, 64, 1, True, False)
     x = inp["x"].to(dev).requires_grad_(True)
