@@ -1942,8 +1942,8 @@ struct GradPre {
   float g, b;
 };
 
-// the row of ld_row without a branch: a missing row reads the block's first one and
-// becomes zeros
+// the row of ld_row without a branch: a missing row reads the block's first one (nval > 0)
+// and becomes zeros
 __device__ __forceinline__ bf16x8 ld_row_nb(const bf16* src, int64_t ts, int tok0, int nval, int tid) {
   const int row = tid >> 4, f0 = (tid & 15) * 8;
   const bool ok = row < nval;
@@ -1977,10 +1977,11 @@ __device__ __forceinline__ void put_row_i(f16* dst, const bf16x8& x, bool l2, fl
 }
 // a raw buffer resource over a block's nval rows of a [tokens][H][D] bf16 output: stores
 // past them are dropped, so the rows need no branch around a store (a wait after one
-// would drain every store before it)
+// would drain every store before it; none for a table row without tokens)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t out_rows(const bf16* o, int64_t tok, int h, int H, int nval) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(o) + (tok * H + h) * D, 0,
-                                           (uint32_t)(((int64_t)(nval - 1) * H * D + D) * 2), 0x00020000);
+                                           nval > 0 ? (uint32_t)(((int64_t)(nval - 1) * H * D + D) * 2) : 0u,
+                                           0x00020000);
 }
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void st_row4(__amdgpu_buffer_rsrc_t r, uint32_t off, const f32x4& x) {
@@ -2041,8 +2042,9 @@ __global__ __launch_bounds__(BNTHR, 2) void gdn_bwd_grad_kernel(Bwd p) {
   if (it >= total) return;
   int cb = it / H, h = it - cb * H;
   int tok0 = p.ctab[cb * 4], nval = p.ctab[cb * 4 + 1];
-  GradPre pre;
-  grad_load(p, pre, (int64_t)cb * H + h, h, tok0, nval, tid, wave, lane);
+  // a table row without tokens loads nothing and, with nval <= 0, stores nothing
+  GradPre pre{};
+  if (nval > 0) grad_load(p, pre, (int64_t)cb * H + h, h, tok0, nval, tid, wave, lane);
   for (;;) {
     const int nxt = it + gridDim.x;
     int ncb = 0, nh = 0, ntok0 = 0, nnval = 0;
@@ -2077,7 +2079,7 @@ __global__ __launch_bounds__(BNTHR, 2) void gdn_bwd_grad_kernel(Bwd p) {
       *reinterpret_cast<uint32_t*>(sT + i * LL + icol(j)) = pre.t;
       *reinterpret_cast<uint32_t*>(sPm + i * LL + icol(j)) = pre.pm;
     }
-    if (nxt < total) grad_load(p, pre, (int64_t)ncb * H + nh, nh, ntok0, nnval, tid, wave, lane);
+    if (nnval > 0) grad_load(p, pre, (int64_t)ncb * H + nh, nh, ntok0, nnval, tid, wave, lane);
     lds_barrier();
 
     // ---- P1: (K^ S0)^T and K^ dS (this wave's value columns), a tile of Q^K^T or

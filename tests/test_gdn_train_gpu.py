@@ -9,6 +9,7 @@ sigmoid(.) (times 2 with allow_neg_eigval).  The loss is sum(o . do) (+ <ht, dht
 when the final state is used).  Every gradient (q, k, v, g, beta and the initial
 state) is compared norm-wise: relative error below 1e-2.  The kernels round each
 MFMA operand once to fp16 (2^-11 relative) and write dq, dk, dv in bf16 (2^-8)."""
+import numpy as np
 import pytest
 import torch
 
@@ -177,3 +178,25 @@ def test_backward_layer_gates_against_oracle(dev):
     print("errors", {n: f"{e:.2e}" for n, e in errs.items()})
     for name, e in errs.items():
         assert e < GRAD_REL, f"{name}: rel {e:.3e}"
+
+
+@pytest.mark.parametrize("T,H", [(70, 2), (1280, 8)])
+def test_backward_block_row_without_tokens(dev, monkeypatch, T, H):
+    """A block table row without tokens reads and writes nothing, as a workgroup's first
+    block (few blocks) and as a later one (more blocks and heads than CUs): the gradients
+    are the same bits as without the row."""
+    from hmx.ops import gdn_train as gtr
+    q, k, v, g, beta, do = _inputs(1, T, H, 41, dev)
+    args = (q, k, v, g, beta, D ** -0.5, None, do, None, [(0, T)], True)
+    want = gtr.chunk_backward(*args)
+    plan = gtr._block_plan
+
+    def with_empty_row(bounds):
+        rows, cu = plan(bounds)
+        return np.concatenate([rows, np.zeros((1, 4), np.int32)]), cu
+
+    monkeypatch.setattr(gtr, "_block_plan", with_empty_row)
+    got = gtr.chunk_backward(*args)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dq", "dk", "dv", "dg", "dbeta"), got, want):
+        assert torch.equal(a, b), name
