@@ -215,8 +215,12 @@ def ptr(t: torch.Tensor | None):
 
 def stream_of(t: torch.Tensor):
     """torch's current stream on the tensor's device, as the raw handle: building a
-    torch.cuda.Stream object for it takes 2.1 us, this 0.1."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    torch.cuda.Stream object for it takes 2.1 us, this 0.1.  A tensor off the GPU raises
+    (the raw call would take its index -1 for the current device)."""
+    index = t.get_device()
+    if index < 0:
+        raise ValueError(f"expected a tensor on a GPU, got one on {t.device}")
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 PLAN_GDN, PLAN_GKA, PLAN_SSD = 0, 1, 2

@@ -66,6 +66,13 @@ def test_wrappers_raise_reference_errors_on_cpu():
                                                  inplace_final_state=False)
 
 
+def test_stream_of_a_host_tensor_raises():
+    """No launch takes a host tensor's device index (-1) for the current device: an op
+    whose other checks do not look at the device raises before its kernel runs."""
+    with pytest.raises(ValueError, match="on a GPU"):
+        _lib.stream_of(torch.zeros(1))
+
+
 @pytest.mark.parametrize("cs", [[1, 4], [0, 5, 3], [0, 4, 9], []])
 def test_bad_cu_seqlens_rejected(cs):
     """Sequence bounds are checked on the host before any kernel reads them:
