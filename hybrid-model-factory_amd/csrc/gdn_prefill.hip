@@ -1984,9 +1984,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t out_rows(const bf16* o, int64_
                                            0x00020000);
 }
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// (WIDE: the output is 8-byte aligned; else element by element)
+template <bool WIDE>
 __device__ __forceinline__ void st_row4(__amdgpu_buffer_rsrc_t r, uint32_t off, const f32x4& x) {
-  const bf16x4 y = {(bf16)x[0], (bf16)x[1], (bf16)x[2], (bf16)x[3]};
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, y), r, off, 0, 0);
+  if constexpr (WIDE) {
+    const bf16x4 y = {(bf16)x[0], (bf16)x[1], (bf16)x[2], (bf16)x[3]};
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, y), r, off, 0, 0);
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const bf16 y = (bf16)x[v];
+      __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, y), r, off + 2 * v, 0, 0);
+    }
+  }
 }
 __device__ __forceinline__ f32x4 ld4_h(const f16* a) {
   const f16x4 x = *reinterpret_cast<const f16x4*>(a);
@@ -2005,6 +2015,7 @@ __device__ __forceinline__ float sum4(const f32x4& x) { return (x[0] + x[1]) + (
 // 8 x 4096 tokens, H = 32: 1.34 -> 1.26 ms (3.4 GB read, 0.9 GB written, 0.85 ms at the
 // rate of a copy).  Latency bounds it: six barriers and the chains between them at two
 // waves per SIMD; with S0 and dS read from cache it takes 1.22 ms, without its stores 1.25.
+template <bool WIDE>
 __global__ __launch_bounds__(BNTHR, 2) void gdn_bwd_grad_kernel(Bwd p) {
   __shared__ __align__(16) unsigned char smem[G_SMEM];
   f16* sK = reinterpret_cast<f16*>(smem + G_OFF_K);
@@ -2136,7 +2147,7 @@ __global__ __launch_bounds__(BNTHR, 2) void gdn_bwd_grad_kernel(Bwd p) {
         const f32x4 Z = mfma16h(bw, frag_t_i(sT, LL, 0, 16 * mt, lane), zero);
         *reinterpret_cast<f16x4*>(sW + r * LR + ic) = h4(W[mt]);
         *reinterpret_cast<f16x4*>(sZ + r * LR + ic) = h4(Z);
-        st_row4(ov, (uint32_t)((r * H * D + c0 + 4 * q4) * 2), Z * sc.B[r]);
+        st_row4<WIDE>(ov, (uint32_t)((r * H * D + c0 + 4 * q4) * 2), Z * sc.B[r]);
         const float zs = q4_sum(sum4(Z * Ut[mt]));
         if (q4 == 0) sPB[wave * C + r] = zs;
       }
@@ -2254,8 +2265,8 @@ __global__ __launch_bounds__(BNTHR, 2) void gdn_bwd_grad_kernel(Bwd p) {
           dk = (dk - kh[mt] * sk) * sRk[r];
         }
         const uint32_t o = (uint32_t)((r * H * D + c0 + 4 * q4) * 2);
-        st_row4(oq, o, dq);
-        st_row4(ok, o, dk);
+        st_row4<WIDE>(oq, o, dq);
+        st_row4<WIDE>(ok, o, dk);
       }
     }
     if (wave == 7) {
@@ -2393,7 +2404,11 @@ extern "C" int hmx_gdn_train_bwd(const void* q, int64_t q_token_stride, const vo
   hipLaunchKernelGGL(gdn_bwd_combine_kernel, dim3(N, H), dim3(BNTHR), 0, s, p);
   hipLaunchKernelGGL(gdn_bwd_chain_kernel, dim3(nchain_segments, H), dim3(BNTHR), 0, s, p,
                      (int)CH_WALK);
-  if (nblock_total > 0)
-    hipLaunchKernelGGL(gdn_bwd_grad_kernel, dim3(grad_grid), dim3(BNTHR), 0, s, p);
+  if (nblock_total > 0) {
+    // dq, dk and dv may lie at any element (the rows are then multiples of 256 bytes apart)
+    const bool wide = ((uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) % 8 == 0;
+    if (wide) hipLaunchKernelGGL(gdn_bwd_grad_kernel<true>, dim3(grad_grid), dim3(BNTHR), 0, s, p);
+    else hipLaunchKernelGGL(gdn_bwd_grad_kernel<false>, dim3(grad_grid), dim3(BNTHR), 0, s, p);
+  }
   return check_launch("hmx_gdn_train_bwd");
 }

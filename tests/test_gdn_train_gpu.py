@@ -200,3 +200,31 @@ def test_backward_block_row_without_tokens(dev, monkeypatch, T, H):
     torch.cuda.synchronize()
     for name, a, b in zip(("dq", "dk", "dv", "dg", "dbeta"), got, want):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("T", [1, 70])
+def test_backward_outputs_at_any_element(dev, monkeypatch, T):
+    """The C entry takes dq, dk and dv at any element: two bytes past their buffers'
+    starts the gradients are the same bits, and the elements around them stay."""
+    from hmx import _lib
+    from hmx.ops import gdn_train as gtr
+    H = 3
+    q, k, v, g, beta, do = _inputs(1, T, H, 43, dev)
+    args = (q, k, v, g, beta, D ** -0.5, None, do, None, [(0, T)], True)
+    want = gtr.chunk_backward(*args)
+    n = T * H * D
+    bufs = [torch.full((n + 2,), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(3)]
+    call = _lib.call
+
+    def shifted(name, *a):
+        a = list(a)
+        if name == "hmx_gdn_train_bwd":
+            a[24:27] = [b.data_ptr() + 2 for b in bufs]
+        return call(name, *a)
+
+    monkeypatch.setattr(_lib, "call", shifted)
+    gtr.chunk_backward(*args)
+    torch.cuda.synchronize()
+    for name, b, w in zip(("dq", "dk", "dv"), bufs, want):
+        assert int((b[1:n + 1] != w.flatten()).sum()) == 0, name
+        assert b[0] == 7.0 and b[n + 1] == 7.0, name
