@@ -1452,10 +1452,11 @@ void launch(const Params& p, hipStream_t s) {
   // the group kernel shares C B^T and W's products over the heads (B and C grouped
   // alike) and forms no y' (which only z needs); it is the faster one at every size
   // measured (its comment), from one head per group on.  It addresses a chunk's 64 rows
-  // with 31-bit byte offsets; the other kernel takes any stride.
+  // with 31-bit byte offsets and stores dx in pieces of up to 16 bytes; the other kernel
+  // takes any stride, and dx at any element.
   const auto ts = {p.x_ts, p.dy_ts, p.b_ts, p.c_ts};
   const bool near = std::min(ts) >= 0 && std::max(ts) < (1 << 24) && (int64_t)p.HX * P < (1 << 23);
-  if (p.G == p.GC && !p.z && near) {
+  if (p.G == p.GC && !p.z && near && (uintptr_t)p.dx % 16 == 0) {
     constexpr int gsm = GLay<P, N>::BYTES;
     (void)hipFuncSetAttribute((const void*)ssd_bwd_group_kernel<P, N>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, gsm);

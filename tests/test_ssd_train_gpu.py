@@ -249,6 +249,36 @@ def test_backward_operands_constant_over_tokens(dev, P, over, l):
         _check(g[k], g_ref[k], f"over={over} P={P} d{k}", scale=sA if k == "A" else None)
 
 
+@pytest.mark.parametrize("P", [64, 128])
+def test_backward_dx_at_any_element(dev, monkeypatch, P):
+    """The C entry takes dx at any element: two bytes past its buffer's start it is that of
+    an aligned buffer (to the rounding of two kernels), and the elements around it stay."""
+    from hmx import _lib
+    from hmx.ops.ssd_train import ssd_chunk_scan_bwd
+    T, H = 70, 2
+    inp, wy, _ = _inputs(1, T, H, 1, P, 128, 1030, False, False)
+    t = {k: v[0].to(dev) if k in ("x", "dt", "B", "C") else v.to(dev)
+         for k, v in inp.items() if v is not None}
+    args = (t["x"], t["dt"], t["A"], t["B"], t["C"], t["D"], None, t["dt_bias"], True,
+            (0.0, float("inf")), [(0, T)], None, wy[0].to(dev))
+    want = ssd_chunk_scan_bwd(*args)[0]
+    n = T * H * P
+    buf = torch.full((n + 2,), 7.0, dtype=torch.bfloat16, device=dev)
+    call = _lib.call
+
+    def shifted(name, *a):
+        a = list(a)
+        if name == "hmx_ssd_chunk_bwd":
+            a[38] = buf.data_ptr() + 2
+        return call(name, *a)
+
+    monkeypatch.setattr(_lib, "call", shifted)
+    ssd_chunk_scan_bwd(*args)
+    torch.cuda.synchronize()
+    _check(buf[1:n + 1].view_as(want), want, f"dx P={P}")
+    assert buf[0] == 7.0 and buf[n + 1] == 7.0
+
+
 def test_backward_headdim_128_with_z_raises(dev):
     inp, _, _ = _inputs(1, 64, 2, 1, 128, 64, 1, True, False)
     x = inp["x"].to(dev).requires_grad_(True)
