@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import itertools
 import os
 from pathlib import Path
 
@@ -230,21 +231,40 @@ def plan_segments(op: int, bounds: list[tuple[int, int]], tokens: int, H: int, c
                   segment_chunks: int | None = None) -> tuple[np.ndarray, int]:
     """The segment table of a chunked prefill (hmx_plan_segments_bounds, host code)
     as an int32 [rows, 8] array, and the chunks of all sequences.  The table depends on
-    the sizes alone: the last few distinct ones are kept (read-only), since the two
-    library calls and their arrays take about 8 us of a short call's host time."""
-    return _plan(op, tuple((int(a), int(b)) for a, b in bounds), int(tokens), int(H),
-                 int(cu_count), int(segment_chunks or 0))
+    the sizes alone, and the last few distinct ones are kept (read-only): lengths planned
+    before take 1 us (4 for 256 sequences) and new ones 10 (48), where asking the library
+    for the table's size first and keeping none takes 12 (84) for any."""
+    args = (tokens, H, cu_count, segment_chunks or 0)
+    try:
+        return _plan(op, tuple(bounds), *args)
+    except TypeError:      # bounds as lists or an array
+        return _plan(op, tuple(map(tuple, bounds)), *args)
 
 
-@functools.lru_cache(maxsize=256)
+@functools.lru_cache(maxsize=64)
 def _plan(op: int, bounds: tuple, tokens: int, H: int, cu_count: int, segment_chunks: int):
-    be = np.ascontiguousarray(np.asarray(bounds, dtype=np.int64).reshape(-1, 2))
+    n = len(bounds)
+    tokens, H, cu_count = int(tokens), int(H), int(cu_count)
+    be = np.fromiter(itertools.chain.from_iterable(bounds), np.int64, 2 * n)
     nrows, nblk = ctypes.c_int32(0), ctypes.c_int32(0)
-    args = (op, be.ctypes.data_as(_P), len(be), tokens, H, cu_count, segment_chunks)
-    call("hmx_plan_segments_bounds", *args, None, 0, ctypes.byref(nrows), ctypes.byref(nblk))
-    table = np.empty((nrows.value, 8), dtype=np.int32)
-    call("hmx_plan_segments_bounds", *args, table.ctypes.data_as(_P), nrows.value,
-         ctypes.byref(nrows), ctypes.byref(nblk))
+    args = (op, be.ctypes.data, n, tokens, H, cu_count, int(segment_chunks))
+
+    def build(rows):
+        table = np.empty((rows, 8), dtype=np.int32)
+        call("hmx_plan_segments_bounds", *args, table.ctypes.data, rows, ctypes.byref(nrows),
+             ctypes.byref(nblk))
+        return table
+
+    # one call into a table that holds what the planner makes of it without
+    # segment_chunks (a row a sequence, or up to four workgroups a CU); a larger
+    # table's size comes back in nrows
+    room = n + max(0, 4 * cu_count // max(H, 1))
+    try:
+        table = build(room)[:nrows.value]
+    except ValueError:
+        if nrows.value <= room:
+            raise
+        table = build(nrows.value)
     table.flags.writeable = False
     return table, nblk.value
 

@@ -154,3 +154,24 @@ def test_plan_rejects_short_table_and_bad_op():
     assert rc == _lib.HMX_EINVAL
     with pytest.raises(ValueError):
         _lib.plan_segments(7, [(0, 10)], 10, 32, 256)
+
+
+def test_new_lengths_are_planned_in_one_library_call(monkeypatch):
+    """A batch of lengths not seen before costs one call of the planner and a repeated one
+    none; a table larger than the one call was given takes a second."""
+    names = []
+    call = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (names.append(name), call(name, *a))[1])
+    for nseq in (1, 3, 256):
+        bounds = [(101 * i, 101 * i + 101) for i in range(nseq)]
+        for again in range(2):
+            names.clear()
+            table, nblk = _lib.plan_segments(_lib.PLAN_GDN, bounds, 101 * nseq, 24, 256)
+            assert len(names) == 1 - again, (nseq, names)
+            assert (table.tolist(), nblk) == _py_plan(_lib.PLAN_GDN, bounds, 24, 256, None)
+    for form in (list(map(list, bounds)), np.asarray(bounds)):
+        assert _lib.plan_segments(_lib.PLAN_GDN, form, 101 * nseq, 24, 256)[0].tolist() == table.tolist()
+    names.clear()
+    table, nblk = _lib.plan_segments(_lib.PLAN_GDN, [(0, 30011)], 30011, 24, 256, 1)
+    assert len(names) == 2
+    assert (table.tolist(), nblk) == _py_plan(_lib.PLAN_GDN, [(0, 30011)], 24, 256, 1)
