@@ -230,8 +230,15 @@ PLAN_GDN, PLAN_GKA, PLAN_SSD = 0, 1, 2
 def plan_segments(op: int, bounds: list[tuple[int, int]], tokens: int, H: int, cu_count: int,
                   segment_chunks: int | None = None) -> tuple[np.ndarray, int]:
     """The segment table of a chunked prefill (hmx_plan_segments_bounds, host code)
-    as an int32 [rows, 8] array, and the chunks of all sequences.  The table depends on
-    the sizes alone, and the last few distinct ones are kept (read-only): lengths planned
+    as an int32 [rows, 8] array, and the chunks of all sequences."""
+    table, nblk = segment_plan(op, bounds, tokens, H, cu_count, segment_chunks)
+    return table.copy(), nblk
+
+
+def segment_plan(op: int, bounds: list[tuple[int, int]], tokens: int, H: int, cu_count: int,
+                 segment_chunks: int | None = None) -> tuple[np.ndarray, int]:
+    """plan_segments with a read-only table.  It depends on the sizes alone, and the last
+    few distinct ones are kept, shared by all callers and threads: lengths planned
     before take 1 us (4 for 256 sequences) and new ones 10 (48), where asking the library
     for the table's size first and keeping none takes 12 (84) for any."""
     args = (tokens, H, cu_count, segment_chunks or 0)
@@ -265,8 +272,13 @@ def _plan(op: int, bounds: tuple, tokens: int, H: int, cu_count: int, segment_ch
         if nrows.value <= room:
             raise
         table = build(nrows.value)
-    table.flags.writeable = False
-    return table, nblk.value
+    return read_only(table), nblk.value
+
+
+def read_only(a: np.ndarray) -> np.ndarray:
+    """``a``, marked read-only: a plan kept for several callers."""
+    a.flags.writeable = False
+    return a
 
 
 def require_gpu(*tensors: torch.Tensor | None) -> None:

@@ -295,9 +295,9 @@ def _segment_table(op: int, bounds: list[tuple[int, int]], tokens: int, H: int,
                    device: torch.device, segment_chunks: int | None = None):
     """The segment table (int32 [rows, 8]: n, bos, eos, c_start, c_end, seg_idx,
     first_seg, nseg) and the total chunk count for prefill ``op`` on ``device``,
-    from the library's host planner.  With ``segment_chunks`` every sequence is cut
+    from the library's host planner (read-only).  With ``segment_chunks`` every sequence is cut
     into equal segments of at most that many chunks (tests)."""
-    return _lib.plan_segments(op, bounds, tokens, H, _cu_count(device), segment_chunks)
+    return _lib.segment_plan(op, bounds, tokens, H, _cu_count(device), segment_chunks)
 
 
 def chunk_gated_delta_rule_gqa(

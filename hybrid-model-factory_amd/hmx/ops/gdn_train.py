@@ -43,9 +43,9 @@ def block_table(bounds: list[tuple[int, int]]):
 
 @functools.lru_cache(maxsize=64)
 def _block_plan(bounds: tuple):
-    """block_table, kept for the last few distinct sizes (it depends on them alone and
-    takes 0.5 ms at 1024 blocks)."""
-    return block_table(bounds)
+    """block_table (read-only), kept for the last few distinct sizes (it depends on them
+    alone and takes 0.5 ms at 1024 blocks)."""
+    return tuple(map(_lib.read_only, block_table(bounds)))
 
 
 @functools.lru_cache(maxsize=64)
@@ -54,7 +54,7 @@ def _chain_plan(bounds: tuple, H: int, cu_count: int, seg_blocks):
     cu = _block_plan(bounds)[1]
     rows = chain_segments(cu, H, cu_count, seg_blocks)
     check_chain_segments(rows, cu)
-    return rows
+    return _lib.read_only(rows)
 
 
 def chain_segments(cu_blocks: np.ndarray, H: int, cu_count: int, seg_blocks: int | None = None):

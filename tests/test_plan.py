@@ -175,3 +175,20 @@ def test_new_lengths_are_planned_in_one_library_call(monkeypatch):
     table, nblk = _lib.plan_segments(_lib.PLAN_GDN, [(0, 30011)], 30011, 24, 256, 1)
     assert len(names) == 2
     assert (table.tolist(), nblk) == _py_plan(_lib.PLAN_GDN, [(0, 30011)], 24, 256, 1)
+
+
+def test_kept_plans_are_not_shared_for_writing():
+    """plan_segments hands out a table of the caller's own; the tables kept between calls
+    (segments, blocks, chain runs, chunks) cannot be written."""
+    from hmx.ops import gdn_train, ssd_train
+    bounds = ((0, 700), (700, 5000))
+    args = (_lib.PLAN_GDN, list(bounds), 5000, 32, 256)
+    table, _ = _lib.plan_segments(*args)
+    want = table.tolist()
+    table[:] = -1
+    assert _lib.plan_segments(*args)[0].tolist() == want
+    kept = [_lib.segment_plan(*args)[0], *gdn_train._block_plan(bounds),
+            gdn_train._chain_plan(bounds, 32, 256, None), *ssd_train._chunk_arrays(bounds)]
+    for a in kept:
+        with pytest.raises(ValueError, match="read-only"):
+            a[:] = -1
