@@ -20,6 +20,14 @@ int check_launch(const char* what) {
   return HMX_OK;
 }
 
+int cu_count() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return 256;
+  return cus;
+}
+
 }  // namespace hmx
 
 extern "C" int hmx_abi_version(void) { return HMX_ABI_VERSION; }

@@ -15,6 +15,7 @@ namespace hmx {
 // ----------------------------------------------------------------------------
 int set_error(int code, const char* fmt, ...);
 int check_launch(const char* what);
+int cu_count();   // compute units of the current device (a partition's, where it is one)
 
 #define HMX_REQUIRE(cond, code, ...)                 \
   do {                                               \

@@ -2388,12 +2388,8 @@ extern "C" int hmx_gdn_train_bwd(const void* q, int64_t q_token_stride, const vo
   p.dg = dg; p.dbeta = dbeta; p.dh0 = dh0;
   p.H = H; p.nblk = nblock_total; p.scale = scale; p.l2norm = use_qk_l2norm;
   hipStream_t s = (hipStream_t)stream;
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    cus = 256;
   const int64_t work = (int64_t)nblock_total * H;
-  const int grad_grid = (int)std::min<int64_t>(work, (int64_t)cus);
+  const int grad_grid = (int)std::min<int64_t>(work, (int64_t)cu_count());
   if (nblock_total > 0)
     hipLaunchKernelGGL(gdn_bwd_prep_kernel, dim3(nblock_total, H), dim3(BNTHR), 0, s, p);
   // where each chain run starts; for heads with an exact run, every run's R and

@@ -41,11 +41,11 @@
 // x shared by several heads (HX < H), or B shared wider than a C group, accumulate
 // with fp32 atomics; everything else is stored.
 
-#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
 #include "mfma.hpp"
+#include "ssd_backward_plan.hpp"
 
 namespace hmx {
 namespace ssdb {
@@ -1439,24 +1439,14 @@ void launch(const Params& p, hipStream_t s) {
   constexpr int smem = Lay<P, N>::BYTES;
   (void)hipFuncSetAttribute((const void*)ssd_bwd_chunk_kernel<P, N>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  // blocks of table rows: one where the heads alone give a workgroup per CU, else as
-  // many as that takes, of no fewer than 8 rows
   const int units = p.H * 2 * (P / SP);
-  const int want = std::min((256 + units - 1) / units, std::max(p.nrows / 8, 1));
-  const int Lr = std::max((p.nrows + want - 1) / want, 1);
-  const int nblk = std::max((p.nrows + Lr - 1) / Lr, 1);
+  const auto [Lr, nblk] = state_blocks(p.nrows, units, cu_count());
   if (nblk > 1)
     hipLaunchKernelGGL((ssd_bwd_states_kernel<P, N, true>), dim3(units * nblk), dim3(STHR), 0, s, p, Lr, nblk);
   hipLaunchKernelGGL((ssd_bwd_states_kernel<P, N, false>), dim3(units * nblk), dim3(STHR), 0, s, p, Lr, nblk);
   if (p.nrows == 0) return;               // sequences without tokens only
-  // the group kernel shares C B^T and W's products over the heads (B and C grouped
-  // alike) and forms no y' (which only z needs); it is the faster one at every size
-  // measured (its comment), from one head per group on.  It addresses a chunk's 64 rows
-  // with 31-bit byte offsets and stores dx in pieces of up to 16 bytes; the other kernel
-  // takes any stride, and dx at any element.
-  const auto ts = {p.x_ts, p.dy_ts, p.b_ts, p.c_ts};
-  const bool near = std::min(ts) >= 0 && std::max(ts) < (1 << 24) && (int64_t)p.HX * P < (1 << 23);
-  if (p.G == p.GC && !p.z && near && (uintptr_t)p.dx % 16 == 0) {
+  if (takes_group_kernel(p.G, p.GC, p.z != nullptr, p.x_ts, p.dy_ts, p.b_ts, p.c_ts, (int64_t)p.HX * P,
+                         (uintptr_t)p.dx)) {
     constexpr int gsm = GLay<P, N>::BYTES;
     (void)hipFuncSetAttribute((const void*)ssd_bwd_group_kernel<P, N>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, gsm);
