@@ -143,18 +143,21 @@ __device__ __forceinline__ SegInfo load_seg(const int* seg, int s) {
   return SegInfo{r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7]};
 }
 
-// The segment of block gb: the last s with segblk[s] <= gb (segblk is non-decreasing),
-// counted 64 segments at a time across the wave's lanes -- one round trip to memory
-// where a binary search takes one per halving.
+// The segment of block gb: the last s with segblk[s] <= gb (segblk is non-decreasing and
+// starts at 0), by a 64-way search across the wave's lanes: one round trip to memory up to
+// 64 segments and two up to 4096, where a binary search takes one per halving.
 __device__ __forceinline__ int segment_of(const Params& p, int gb, int lane) {
-  int n = 0;
-  for (int s0 = 0; s0 < p.nseg_total; s0 += 64) {
-    const int s = s0 + lane;
-    const int c = __builtin_popcountll(__ballot(s < p.nseg_total && p.segblk[min(s, p.nseg_total - 1)] <= gb));
-    n += c;
-    if (c < 64) break;
+  const auto count = [&](int lo, int step, int n) {   // of lo, lo + step, .. < lo + n
+    const int s = lane * step;
+    return __builtin_popcountll(__ballot(s < n && p.segblk[lo + min(s, n - 1)] <= gb));
+  };
+  int lo = 0, n = p.nseg_total;
+  while (n > 64) {
+    const int step = (n + 63) / 64, c = count(lo, step, n) - 1;
+    lo += c * step;
+    n = min(step, n - c * step);
   }
-  return __builtin_amdgcn_readfirstlane(n - 1);
+  return __builtin_amdgcn_readfirstlane(lo + count(lo, 1, n) - 1);
 }
 
 // Sum of squares of an 8-feature slice over the 16 lanes of its DPP row.

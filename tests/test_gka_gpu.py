@@ -281,3 +281,29 @@ def test_gka_training_decode_steps(dev):
                                               0.1, 0.02, "chebyshev", 0, None, None)
     torch.cuda.synchronize()
     assert hk1 is None and o.shape == (1, 1, 2, 128)
+
+
+@pytest.mark.parametrize("nseq", [64, 65, 4097, 4200])
+def test_gka_prefill_many_segments(dev, nseq):
+    """Blocks find their segment among more than one and more than two rounds of the 64-way
+    search, empty sequences among them: the same bits as in calls of a few sequences."""
+    lens = [(i * 7) % 4 for i in range(nseq)]
+    cs = [0]
+    for n in lens:
+        cs.append(cs[-1] + n)
+    q, k, v, alpha, g, gk, beta, _ = _mk(cs[-1], 1, 1, 77)
+    ops = [x.to(dev) for x in (q, k, v, alpha, g, gk, beta)]
+
+    def run(a, e):
+        cu = torch.tensor([c - cs[a] for c in cs[a:e + 1]], dtype=torch.int32)
+        return hmx.gka_chebyshev_gla_prefill(*(x[:, cs[a]:cs[e]] for x in ops), 0.09, num_iter=2,
+                                             cu_seqlens=cu)
+
+    o, hkk, hkv = run(0, nseq)
+    for a in range(0, nseq, 60):
+        e = min(a + 60, nseq)
+        if cs[a] == cs[e]:
+            continue
+        oa, ka, va = run(a, e)
+        assert torch.equal(o[:, cs[a]:cs[e]], oa), (a, e)
+        assert torch.equal(hkk[a:e], ka) and torch.equal(hkv[a:e], va), (a, e)
