@@ -196,10 +196,11 @@ def test_backward_state_chains_cross_blocks(dev, P, N, H, lens):
 
 
 def test_backward_far_apart_gradient_rows(dev):
-    """dy with token rows 2^24 elements apart (a chunk's rows past the 32-bit byte offsets
-    of the group kernel): the general kernel takes it; the same gradients as from
-    contiguous rows, to the rounding of two kernels that each meet _check's bound."""
-    l, H, P = 3, 2, 64
+    """dy with token rows 2^26 elements apart, so that row 32 of a chunk is 2^32 bytes past
+    its first (32-bit offsets would read row 0 there, and nothing for the rows between):
+    the general kernel takes it; the same gradients as from contiguous rows, to the rounding
+    of two kernels that each meet _check's bound."""
+    l, H, P = 34, 2, 64
     inp, wy, _ = _inputs(1, l, H, 1, P, 128, 995, False, False)
     inp.pop("z")
     leaves = {k: v.to(dev).requires_grad_(True) for k, v in inp.items()}
@@ -207,8 +208,8 @@ def test_backward_far_apart_gradient_rows(dev):
     y = hmx.mamba_chunk_scan_combined(args.pop("x"), args.pop("dt"), args.pop("A"), args.pop("B"),
                                       args.pop("C"), 256, dt_softplus=True, **args)
     dy = wy.to(dev, torch.bfloat16)
-    step = 1 << 24
-    far = torch.zeros((l - 1) * step + H * P, dtype=torch.bfloat16, device=dev)
+    step = 1 << 26
+    far = torch.empty((l - 1) * step + H * P, dtype=torch.bfloat16, device=dev)
     far = far.as_strided((1, l, H, P), (l * step, step, P, 1))
     far.copy_(dy)
     g = torch.autograd.grad(y, list(leaves.values()), dy, retain_graph=True)
@@ -216,6 +217,36 @@ def test_backward_far_apart_gradient_rows(dev):
     torch.cuda.synchronize()
     for k, a, b in zip(leaves, g_far, g):
         _check(a, b, f"far d{k}")
+
+
+@pytest.mark.parametrize("P,H,HX,G,l", [(64, 6, 2, 3, 70), (64, 4, 1, 1, 130), (128, 4, 2, 2, 65),
+                                        (128, 3, 1, 3, 64)])
+def test_backward_x_shared_by_heads(dev, P, H, HX, G, l):
+    """x heads shared by several heads, with B and C grouped alike and no z (the group
+    kernel's fp32 stores of dB and dC, and its atomics into dx), within a group and over
+    several, with whole and ragged last chunks."""
+    from hmx.ops.ssd_train import ssd_chunk_scan_bwd
+    inp, wy, _ = _inputs(1, l, H, G, P, 128, 1050 + l, False, False)
+    inp["x"] = inp["x"][:, :, :HX].contiguous()
+    t = {k: v[0].to(dev) if k in ("x", "dt", "B", "C") else v.to(dev)
+         for k, v in inp.items() if v is not None}
+    got = ssd_chunk_scan_bwd(t["x"], t["dt"], t["A"], t["B"], t["C"], t["D"], None, t["dt_bias"],
+                             True, (0.0, float("inf")), [(0, l)], None, wy[0].to(dev))
+    torch.cuda.synchronize()
+    g = dict(zip(("x", "dt", "A", "B", "C", "D", "dt_bias"), got))
+    assert all(g[k].dtype == torch.float32 for k in ("x", "B", "C"))
+    g["D"] = g["D"].sum(-1)
+    inp["initial_states"] = None
+    ref_in = {k: v.double().requires_grad_(True) for k, v in inp.items() if v is not None}
+    a = dict(ref_in)
+    xx = a.pop("x").repeat_interleave(H // HX, dim=2)
+    y = ref.mamba_chunk_scan_combined(xx, a.pop("dt"), a.pop("A"), a.pop("B"), a.pop("C"), 256,
+                                      dt_softplus=True, **a)
+    (y * wy.double()).sum().backward()
+    sA = _dA_scale(dict(inp, x=inp["x"].repeat_interleave(H // HX, dim=2)), wy, None,
+                   dict(dt_softplus=True))
+    for k, v in ref_in.items():
+        _check(g[k], v.grad, f"x heads {HX}/{H} P={P} d{k}", scale=sA if k == "A" else None)
 
 
 @pytest.mark.parametrize("P,over,l", [(64, "C", 130), (64, "x", 65), (64, "xBC", 66), (128, "C", 65),
