@@ -140,12 +140,6 @@ __device__ __forceinline__ Tok token_scalars_raw(const Params& p, int h, float d
   const float acs = scan64(dtv * p.A[h], lane);
   return Tok{dtv, acs, fac};
 }
-__device__ __forceinline__ Tok token_scalars(const Params& p, int h, int tok0, int nval, int lane) {
-  float d = 0.f;
-  if (lane < nval) d = load_any(p.dt, (int64_t)(tok0 + lane) * p.dt_ts + (int64_t)h * p.dt_hs, p.dt_dt);
-  return token_scalars_raw(p, h, d, nval, lane);
-}
-
 constexpr int row_ld(int w) { return w == 64 ? w + 8 : w + 16; }
 
 // ---------------------------------------------------------------------------
@@ -482,10 +476,12 @@ __global__ __launch_bounds__(STHR, 2) void ssd_bwd_states_kernel(Params p, int L
 // What bounds it: latency at two waves per SIMD, then memory (1.8 GB read and 0.45 GB
 // written at 2 x 16384 tokens, H = 64, P = 64, N = 128, G = 8: 0.44 ms at the rate of a
 // copy; S0 and dS1, 16 KB each per head and chunk, are 1.07 GB of it).  Measured there:
-// 0.76 ms where ssd_bwd_chunk_kernel (four waves per CU, nine products, scalar LDS
-// reads) takes 1.96; forward + backward 3.14 -> 1.95 ms.  At 8 x 4096 tokens, H = 32,
-// P = N = 128 with 1, 4 or 8 heads per group 3.13 -> 2.27, 2.76 -> 2.00, 2.70 -> 1.97 ms;
-// at 2 x 8192, H = 64, P = 64 with one head per group 2.17 -> 1.47 ms.
+// 0.75 ms where ssd_bwd_chunk_kernel (four waves per CU, nine products, scalar LDS
+// reads) takes 1.96.  In forward + backward, both with the chunk states still formed by
+// two launches: 3.14 against 1.95 ms; at 8 x 4096 tokens, H = 32, P = N = 128 with 1, 4
+// or 8 heads per group 3.13 against 2.27, 2.76 against 2.00, 2.70 against 1.97 ms; at
+// 2 x 8192, H = 64, P = 64 with one head per group 2.17 against 1.47 ms.  (With the state
+// chains 1.56 ms there and 1.82 at 8 x 4096 with one head per group.)
 // ---------------------------------------------------------------------------
 constexpr int GTHR = 512;
 
