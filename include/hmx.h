@@ -302,7 +302,8 @@ int hmx_gdn_train_fwd(const void* q, int64_t q_token_stride, const void* k, cons
  * stride dout_token_stride) and, optionally, dht (the gradient of the final states,
  * fp32 [N][H][128][128]).  block_states: hmx_gdn_train_fwd's; block_table int32
  * [nblock_total][4] = (first token, tokens (1-32), sequence, block index within
- * the sequence); cu_blocks [N+1].  chain_segments int32 [nchain_segments][3] =
+ * the sequence; a row past the sequences' own with 0 tokens is passed over);
+ * cu_blocks [N+1].  chain_segments int32 [nchain_segments][3] =
  * (sequence, first block, end block) cuts every sequence's blocks into runs that
  * one workgroup each walks backward.  Required order (not checked here; the Python
  * wrapper checks it on the host): rows grouped by ascending sequence 0..N-1, every
@@ -315,7 +316,7 @@ int hmx_gdn_train_fwd(const void* q, int64_t q_token_stride, const void* k, cons
  * finds no such warm-up takes every run's exact start from a combine over the runs
  * (each run's chain from zero and its transposed transition product).  Writes dq,
  * dk, dv [tokens][H][128] bf16 (rows
- * of the blocks' tokens only), dg and dbeta [tokens][H] fp32, and dh0 (the
+ * of the blocks' tokens only; fastest 8-byte aligned, at any element), dg and dbeta [tokens][H] fp32, and dh0 (the
  * gradient of the initial states, fp32 [N][H][128][128]) when not null.
  * workspace: hmx_gdn_train_bwd_workspace_bytes(nblock_total, nchain_segments, N, H) bytes.
  * Replaces: the backward of fla's chunk_gated_delta_rule (un-vendored; the training
@@ -579,6 +580,9 @@ size_t hmx_ssd_chunk_workspace_bytes(int32_t nseg_total, int32_t nseq, int32_t H
  *  C [tokens, GC, N], z and dy [tokens, H, P], dt [tokens, H] f32/bf16/f16, fp32 A,
  *  D [H, P], dt_bias).  h0: fp32 [nseq, H, P, N] start states or NULL (zero);
  *  d_final: fp32 [nseq, H, P, N] gradient of the end states, or NULL.
+ *  Any token strides (0 for an operand constant over the tokens) that are multiples
+ *  of 8; an x, B, C or dy whose rows lie 2^24 elements or more apart, or a dx off 16
+ *  bytes, takes the slower kernel.
  *  Outputs, contiguous: dx [tokens, HX, P], dB [tokens, G, N], dC [tokens, GC, N]
  *  in grad_dtype (HMX_F32, or HMX_BF16 when none accumulates: HX = H and G = H or
  *  G = GC); dx accumulates when HX < H and dB when G < H and G != GC (then fp32,
